@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "common.h"
+#include "harm_dev.h"
 #include "net_dev.h"
 
 namespace ann {
@@ -339,13 +340,15 @@ static int upload_model(ann_ctx* ctx, const ann_model_desc* d) {
     for (int t = 0; t < S * NP; ++t) {
         AngBlock& ab = M.ang[t];
         for (int k = 0; k < kGridK; ++k)
-            for (int m = 0; m <= kMomZ; ++m) {
-                double c = 0.0;
-                if (M.moment_z > 0 && k < ab.nk && m <= ab.zint[k]) {
-                    c = std::pow(2.0, m - ab.zint[k]) * std::pow((double)ab.lamh[k], m);
+            for (int l = 0; l <= kMomZ; ++l) {
+                // (1/2 + lambda c / 2)^zeta = sum_m C(zeta,m) 2^(m-zeta) (lambda/2)^m c^m in Legendre polynomials
+                double a = 0.0;
+                for (int m = l; M.moment_z > 0 && k < ab.nk && m <= ab.zint[k]; m += 2) {
+                    double c = std::pow(2.0, m - ab.zint[k]) * std::pow((double)ab.lamh[k], m);
                     for (int q = 0; q < m; ++q) c = c * (ab.zint[k] - q) / (q + 1);
+                    a += c * legendre_of_power(m, l);
                 }
-                ab.mcoef[k][m] = (float)c;
+                ab.lcoef[k][l] = (float)a;
             }
     }
     int maxin = 1;
@@ -925,9 +928,8 @@ static hipError_t ensure_work(ann_ctx* ctx) {
         if ((e = dalloc(ctx->d_u, 3 * (size_t)N)) != hipSuccess) return e;
         if ((e = dalloc(ctx->d_F, 3 * (size_t)N)) != hipSuccess) return e;
         if ((e = dalloc(ctx->d_atomvir, 9 * (size_t)N)) != hipSuccess) return e;
-        if (ctx->hm.moment_z > 0) {   // moments of the moment form: [N][S][4][monomials]
-            const int z = ctx->hm.moment_z, nm = (z + 1) * (z + 2) * (z + 3) / 6;
-            if ((e = dalloc(ctx->d_T, (size_t)N * ctx->S * kMaxUnionEta * nm)) != hipSuccess) return e;
+        if (ctx->hm.moment_z > 0) {   // moments of the moment form: [N][S][4][harmonics]
+            if ((e = dalloc(ctx->d_T, (size_t)N * ctx->S * kMaxUnionEta * nharm(ctx->hm.moment_z))) != hipSuccess) return e;
         }
         ctx->T_gen = ~0ull;
         ctx->work_atoms = N;

@@ -56,7 +56,7 @@ struct AngBlock {
     float zeta[kGridK];
     int zint[kGridK];              // integer zeta (>=0) or -1
     int outm[kGridG * kGridK];     // function index of (g, k)
-    float mcoef[kGridK][kMomZ + 1];  // moment form: C(zeta,m) 2^(m-zeta) (lambda/2)^m of combination k
+    float lcoef[kGridK][kMomZ + 1];  // moment form: Legendre coefficients of (1/2 + lambda c / 2)^zeta, combination k
 };
 
 struct NetDesc {

@@ -18,6 +18,7 @@
 // (radial) or over first triplet legs with the second leg looped (angular);
 // FP64 lane sums and a fixed butterfly, so the result is deterministic.
 #include "basis_dev.h"
+#include "harm_dev.h"
 #include "pairvec_dev.h"
 
 namespace ann {
@@ -102,29 +103,22 @@ __device__ inline double angular64(int name, double ieta2, double zeta, double l
     return pow(fabs(0.5 + lamh * c), zeta) * fr * f0 * f1;
 }
 
-// monomials x^a y^b z^c of total degree <= kMomZ in degree order (as the FP32
-// moment kernels number them) and their multinomial weights m!/(a! b! c!)
-constexpr int kMonoAll = (kMomZ + 1) * (kMomZ + 2) * (kMomZ + 3) / 6;
-struct MonoFixed {
-    int a[kMonoAll], b[kMonoAll], c[kMonoAll], m[kMonoAll];
-    double w[kMonoAll];
-    constexpr MonoFixed() : a(), b(), c(), m(), w() {
-        int q = 0;
-        for (int mm = 0; mm <= kMomZ; ++mm)
-            for (int aa = mm; aa >= 0; --aa)
-                for (int bb = mm - aa; bb >= 0; --bb) {
-                    const int cc = mm - aa - bb;
-                    int fm = 1, fa = 1, fb = 1, fc = 1;
-                    for (int t = 2; t <= mm; ++t) fm *= t;
-                    for (int t = 2; t <= aa; ++t) fa *= t;
-                    for (int t = 2; t <= bb; ++t) fb *= t;
-                    for (int t = 2; t <= cc; ++t) fc *= t;
-                    a[q] = aa; b[q] = bb; c[q] = cc; m[q] = mm;
-                    w[q] = (double)(fm / (fa * fb * fc));
-                    ++q;
-                }
+// Legendre coefficients of (1/2 + c / 2)^zeta; those of (1/2 - c / 2)^zeta carry (-1)^l
+struct LegFixed {
+    double a[kMomZ + 1][kMomZ + 1];
+    constexpr LegFixed() : a() {
+        for (int z = 0; z <= kMomZ; ++z) {
+            double binom = 1.0;
+            for (int m = 0; m <= z; ++m) {
+                double c = binom;
+                for (int t = 0; t < z; ++t) c *= 0.5;
+                for (int l = m & 1; l <= m; l += 2) a[z][l] += c * legendre_of_power(m, l);
+                binom = binom * (z - m) / (m + 1);
+            }
+        }
     }
 };
+__constant__ LegFixed c_leg = LegFixed();
 
 __device__ inline double wave_sum64(double v) {
 #pragma unroll
@@ -174,6 +168,9 @@ __device__ inline double cut64f(int name, double rc, double r) {
     return cut64(name, rc, r);
 }
 
+// neighbours per chunk of function rows
+constexpr int kPreRows = 32;
+
 // One wavefront per atom.  Z: largest zeta of the moment form (0: the model
 // has no moment form; angular inputs are then summed over triplets).  With
 // A.Tout set (moment form only) the moments of every atom are also written in
@@ -190,20 +187,19 @@ __global__ __launch_bounds__(64) void k_precise(PreciseArgs A, int maxn) {
     if (q0 == q1 && !wantT) return;
     const int S = M.S, NP = M.NP;
     constexpr int ZP = Z + 1;
-    constexpr int NM = Z > 0 ? (Z + 1) * (Z + 2) * (Z + 3) / 6 : 1;
-    constexpr int PWS = Z > 0 ? (3 * Z) | 1 : 1;          // powers k = 1..Z of the three components
-    constexpr int NMH = Z > 1 ? NM - 4 : 1;               // monomials of degree >= 2
-    constexpr int GH = Z > 1 ? kWave / NMH : 1;           // neighbour groups of the degree >= 2 sums
-    // LDS: (r, fc) and, moment form, widths and powers; triplet form, unit vectors
+    constexpr int NM = nharm(Z);
+    constexpr int PWS = NM | 1;                           // function values per neighbour, odd stride
+    constexpr int NG = Z > 0 ? kWave / NM : 1;            // neighbour groups of the moment sums
+    // LDS: (r, fc) and, moment form, unit vectors, widths and one chunk of function rows; triplet form, unit vectors
     double2* rf = reinterpret_cast<double2*>(smem64);
     double4* ef = reinterpret_cast<double4*>(rf + maxn);                   // [maxn] (Z > 0)
     double4* uv = ef;                                                        // [maxn] unit vectors (Z == 0)
-    double* pw = reinterpret_cast<double*>(ef + maxn);                      // [maxn][PWS] (Z > 0)
-    double* T = pw + (Z > 0 ? (size_t)maxn * PWS : 0);                      // [S][4][NM]
+    double* hv = reinterpret_cast<double*>(ef + maxn);                      // [maxn][3] unit vectors (Z > 0)
+    double* pw = hv + (Z > 0 ? 3 * (size_t)maxn : 0);                       // [kPreRows][PWS]
+    double* T = pw + (Z > 0 ? (size_t)kPreRows * PWS : 0);                  // [S][4][NM]
     double* Dg = T + (Z > 0 ? S * 4 * NM : 0);                              // [S][4]
     double* Am = Dg + (Z > 0 ? S * 4 : 0);                                  // [NP][4][ZP]
-    double* part = Am + (Z > 0 ? NP * 4 * ZP : 0);                          // [GH][NMH][4]
-    int* seg = reinterpret_cast<int*>(part + (Z > 1 ? GH * NMH * 4 : 0));   // [kMaxSpecies + 1]
+    int* seg = reinterpret_cast<int*>(Am + (Z > 0 ? NP * 4 * ZP : 0));      // [kMaxSpecies + 1]
     const int o = A.off[i], n = A.off[i + 1] - o;
     const double* R = A.cells + 9 * A.sof[i];
     const uint64_t lt = (1ull << lane) - 1ull;
@@ -278,16 +274,8 @@ __global__ __launch_bounds__(64) void k_precise(PreciseArgs A, int maxn) {
 #pragma unroll
                 for (int u = 0; u < 4; ++u) e[u] = u < U ? exp(-r2 * M.uieta2_64[a][u]) * f : 0.0;
                 ef[p] = make_double4(e[0], e[1], e[2], e[3]);
-                double* row = pw + (size_t)p * PWS;
 #pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    double qv = h[c];
-#pragma unroll
-                    for (int k = 0; k < Z; ++k) {
-                        row[c * Z + k] = qv;
-                        qv *= h[c];
-                    }
-                }
+                for (int c = 0; c < 3; ++c) hv[3 * p + c] = h[c];
             } else {
                 uv[p] = make_double4(h[0], h[1], h[2], 0.0);
             }
@@ -330,91 +318,78 @@ __global__ __launch_bounds__(64) void k_precise(PreciseArgs A, int maxn) {
     }
     if (q == q1 && !wantT) return;
     if constexpr (Z > 0) {
-        static_assert(Z <= kMomZ, "the monomial table covers the moment form's degrees");
-        constexpr MonoFixed mo{};
+        static_assert(Z <= kMomZ, "the Legendre table covers the moment form's degrees");
         for (int b = 0; b < S; ++b) {
             const int s0 = seg[b], s1 = seg[b + 1];
-            // degree <= 1 moments (1, x, y, z) and the diagonal sums: lanes over
-            // neighbours, one transposing reduction of 4 x 5 values (padded to 32)
-            {
-                double v[32];
+            // moments: function rows of a chunk of neighbours (lanes over
+            // neighbours), then lane = (function, neighbour group)
+            const int al = lane % NM, g = lane / NM;
+            double t4[4] = {0.0, 0.0, 0.0, 0.0}, d4[4] = {0.0, 0.0, 0.0, 0.0};
+            for (int c0 = s0; c0 < s1; c0 += kPreRows) {
+                const int c1 = min(c0 + kPreRows, s1);
+                __syncthreads();
+                for (int J = c0 + lane; J < c1; J += kWave) {
+                    double C[ZP], Sn[ZP], qv[qidx(Z, Z) + 1], y[NM];
+                    harm_factors<Z, double>(hv[3 * J], hv[3 * J + 1], hv[3 * J + 2], C, Sn, qv);
+                    harm_values<Z, double>(C, Sn, qv, y);
+                    double* row = pw + (size_t)(J - c0) * PWS;
 #pragma unroll
-                for (int x = 0; x < 32; ++x) v[x] = 0.0;
-                for (int J = s0 + lane; J < s1; J += kWave) {
-                    const double4 e4 = ef[J];
-                    const double* row = pw + (size_t)J * PWS;
-                    const double hx = row[0], hy = row[Z], hz = row[2 * Z];
-                    const double ev[4] = {e4.x, e4.y, e4.z, e4.w};
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        v[5 * u] += ev[u];
-                        v[5 * u + 1] += ev[u] * hx;
-                        v[5 * u + 2] += ev[u] * hy;
-                        v[5 * u + 3] += ev[u] * hz;
-                        v[5 * u + 4] += ev[u] * ev[u];
-                    }
+                    for (int f = 0; f < NM; ++f) row[f] = y[f];
                 }
-                int idx;
-                const double sv = wave_sum_multi64<32>(v, idx);
-                if ((lane & 1) == 0 && idx < 20) {
-                    const int u = idx / 5, c = idx % 5;
-                    if (c < 4) T[(b * 4 + u) * NM + c] = sv;
-                    else Dg[b * 4 + u] = sv;
-                }
-            }
-            // degree >= 2: lane = (monomial, neighbour group), powers from the rows
-            if (Z > 1) {
-                const int al = 4 + lane % NMH, g = lane / NMH;
-                if (g < GH) {
-                    const int ea = mo.a[al], eb = mo.b[al], ec = mo.c[al];
-                    double t4[4] = {0.0, 0.0, 0.0, 0.0};
-                    auto pv = [&](const double* row, int c, int e) { return e == 0 ? 1.0 : row[c * Z + e - 1]; };
-                    for (int J = s0 + g; J < s1; J += GH) {
-                        const double* row = pw + (size_t)J * PWS;
-                        const double mono = pv(row, 0, ea) * pv(row, 1, eb) * pv(row, 2, ec);
+                __syncthreads();
+                if (g < NG)
+                    for (int J = c0 + g; J < c1; J += NG) {
+                        const double yv = pw[(size_t)(J - c0) * PWS + al];
                         const double4 e4 = ef[J];
-                        t4[0] += e4.x * mono; t4[1] += e4.y * mono; t4[2] += e4.z * mono; t4[3] += e4.w * mono;
+                        t4[0] += e4.x * yv; t4[1] += e4.y * yv; t4[2] += e4.z * yv; t4[3] += e4.w * yv;
                     }
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) part[(g * NMH + al - 4) * 4 + u] = t4[u];
-                }
-                __syncthreads();
-                for (int it = lane; it < NMH * 4; it += kWave) {
-                    double sum = 0.0;
-                    for (int gg = 0; gg < GH; ++gg) sum += part[gg * NMH * 4 + it];
-                    T[(b * 4 + it % 4) * NM + 4 + it / 4] = sum;
-                }
-                __syncthreads();
             }
+            for (int J = s0 + lane; J < s1; J += kWave) {
+                const double4 e4 = ef[J];
+                d4[0] += e4.x * e4.x; d4[1] += e4.y * e4.y; d4[2] += e4.z * e4.z; d4[3] += e4.w * e4.w;
+            }
+            double sum4[4] = {t4[0], t4[1], t4[2], t4[3]};
+#pragma unroll
+            for (int gg = 1; gg < NG; ++gg)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) sum4[u] += __shfl(t4[u], lane + gg * NM);
+            if (lane < NM)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) T[(b * 4 + u) * NM + al] = sum4[u];
+            int idx;
+            const double dv = wave_sum_multi64<4>(d4, idx);
+            if ((lane & (kWave / 4 - 1)) == 0) Dg[b * 4 + idx] = dv;
         }
         __syncthreads();
         if (wantT) {
             const int TS = S * 4 * NM;
             for (int x = lane; x < TS; x += kWave) A.Tout[(size_t)i * TS + x] = (float)T[x];
         }
-        // A_m(p, u) = sum_{|alpha| = m} w_alpha T_b T_c (b != c); (... - D_b) / 2 for b == c
+        // A_l(p, u) = sum_m T_b T_c (b != c); (... - D_b) / 2 for b == c
         for (int it = lane; it < NP * 4 * ZP; it += kWave) {
             const int p = it / (4 * ZP), u = (it / ZP) % 4, m = it % ZP;
             int c = 0;
             while ((c + 1) * (c + 2) / 2 <= p) ++c;
             const int b = p - c * (c + 1) / 2;
-            const int qa = m * (m + 1) * (m + 2) / 6, qb = (m + 1) * (m + 2) * (m + 3) / 6;
             double sum = 0.0;
-            for (int x = qa; x < qb; ++x) sum += mo.w[x] * T[(b * 4 + u) * NM + x] * T[(c * 4 + u) * NM + x];
+            for (int x = m * m; x < (m + 1) * (m + 1); ++x) sum += T[(b * 4 + u) * NM + x] * T[(c * 4 + u) * NM + x];
             if (b == c) sum = 0.5 * (sum - Dg[b * 4 + u]);
             Am[it] = sum;
         }
         __syncthreads();
-        // G = sum_m C(zeta, m) 2^-zeta lambda^m A_m: one lane per item
+        // G = sum_l a_l A_l, a_l the Legendre coefficients of (1/2 + lambda c / 2)^zeta: one lane per item
         for (int t = q + lane; t < q1; t += kWave) {
             const PreItem it = A.items[t];
-            double g = 0.0, binom = 1.0, lp = 1.0;
-            for (int m = 0; m <= it.zint; ++m) {
-                g += binom * lp * Am[(it.blk * 4 + it.u) * ZP + m];
-                binom = binom * (it.zint - m) / (m + 1);
-                lp *= (double)it.lam;
+            double g = 0.0;
+            if (it.lam == 0) {
+                g = ldexp(Am[(it.blk * 4 + it.u) * ZP], -it.zint);
+            } else {
+                for (int l = 0; l <= it.zint; ++l) {
+                    const double a = c_leg.a[it.zint][l] * Am[(it.blk * 4 + it.u) * ZP + l];
+                    g += it.lam < 0 && (l & 1) ? -a : a;
+                }
             }
-            put(it.k, g * ldexp(1.0, -it.zint));
+            put(it.k, g);
         }
     } else {
         // angular items outside the moment form: lanes over the first leg, the
@@ -447,13 +422,10 @@ __global__ __launch_bounds__(64) void k_precise(PreciseArgs A, int maxn) {
 }
 
 static size_t precise_smem(int maxn, int Z, int S, int NP) {
-    const int NM = Z > 0 ? (Z + 1) * (Z + 2) * (Z + 3) / 6 : 1;
     size_t b = (size_t)maxn * sizeof(double2) + (size_t)maxn * sizeof(double4);
-    if (Z > 0) {
-        const int PWS = (3 * Z) | 1, NMH = Z > 1 ? NM - 4 : 1, GH = Z > 1 ? kWave / NMH : 1;
-        b += sizeof(double) * ((size_t)maxn * PWS + (size_t)S * 4 * NM + S * 4 + (size_t)NP * 4 * (Z + 1) +
-                               (Z > 1 ? (size_t)GH * NMH * 4 : 0));
-    }
+    if (Z > 0)
+        b += sizeof(double) * (3 * (size_t)maxn + (size_t)kPreRows * (nharm(Z) | 1) + (size_t)S * 4 * nharm(Z) + S * 4 +
+                               (size_t)NP * 4 * (Z + 1));
     return b + sizeof(int) * (kMaxSpecies + 1);
 }
 

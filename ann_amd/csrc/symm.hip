@@ -34,6 +34,7 @@
 #include <vector>
 
 #include "basis_dev.h"
+#include "harm_dev.h"
 #include "net_dev.h"
 
 namespace ann {
@@ -866,67 +867,46 @@ __global__ __launch_bounds__(64) void k_fast(SymmArgs A) {
 //
 // For GAUSS angular blocks with integer zeta <= 5 the triplet sum factorises
 // exactly.  With e_u(r) = exp(-r^2/eta_u^2) fc(r) and c = r^_j . r^_k,
-//   (1/2 + lambda c / 2)^zeta = sum_m C(zeta,m) 2^(m-zeta) (lambda/2)^m c^m,
-//   c^m = sum_{|alpha|=m} (m!/alpha!) r^_j^alpha r^_k^alpha,
+//   (1/2 + lambda c / 2)^zeta = sum_l a_l P_l(c),
+//   P_l(c) = sum_m Y_lm(r^_j) Y_lm(r^_k)                 (harm_dev.h)
 // so a block (species b, species c, width u) needs only the per-species
-// moments T_b[u][alpha] = sum_{j in b} e_u(r_j) r^_j^alpha and
+// moments T_b[u][lm] = sum_{j in b} e_u(r_j) Y_lm(r^_j) and
 // D_b[u] = sum_{j in b} e_u(r_j)^2:
-//   A_m = sum_{|alpha|=m} w_alpha T_b T_c                (b != c)
-//   A_m = (sum_{|alpha|=m} w_alpha T_b T_b - D_b) / 2    (b == c: pairs j < k)
-//   G(u, lambda, zeta) = sum_m C(zeta,m) 2^(m-zeta) (lambda/2)^m A_m.
-// Work per atom is O(n M) with M = (Z+1)(Z+2)(Z+3)/6 monomials instead of
-// O(n^2) triplets.  The adjoint differentiates the same chain: dE/dT_b from
-// the block contractions, then per neighbour the polynomial
-// Q(r^) = sum_alpha dE/dT_b[u][alpha] r^^alpha and its gradient.  The
-// tangent (force-loss second backward) is the forward-mode derivative.
-// FP32 throughout: the alternating binomial sum amplifies rounding by at most
-// C(5,2) = 10 for zeta <= 5; larger zeta keeps the triplet kernels.
+//   A_l = sum_m T_b T_c                                  (b != c)
+//   A_l = (sum_m T_b T_b - D_b) / 2                      (b == c: pairs j < k)
+//   G(u, lambda, zeta) = sum_l a_l A_l.
+// Work per atom is O(n M) with M = (Z+1)^2 functions instead of O(n^2)
+// triplets.  The adjoint differentiates the same chain: dE/dT_b from the block
+// contractions, then per neighbour the function sum_lm dE/dT_b[u][lm] Y_lm(r^)
+// and its gradient.  The tangent (force-loss second backward) is the
+// forward-mode derivative.
+// The kernels issue vector instructions most of the time, so the number of
+// functions is what counts: the harmonics are the (Z+1)^2 independent functions
+// among the (Z+1)(Z+2)(Z+3)/6 monomials of the unit vector's components (25
+// against 35 at zeta 4, 36 against 56 at zeta 5), and as an orthogonal basis
+// they have no alternating sum to amplify FP32 rounding.  Monomials against
+// harmonics, MI355X: E+F of 32 preconditioned water boxes (FP64 moments) 265 ->
+// 216 us, 512 uneven water cells 4.18 -> 3.94 ms, five MD steps of 1 M atoms
+// 103.0 -> 97.2 ms, 64 water boxes and Li/P/S training unchanged.
 
-__host__ __device__ constexpr int nmono(int Z) { return (Z + 1) * (Z + 2) * (Z + 3) / 6; }
-// neighbours per chunk of power rows (G: 32 and adjoint: 64, which frees LDS
-// for more resident wavefronts; tangent: every neighbour at once, measured
-// faster with its two-level rows), and the floats of the region that holds them (it
-// also holds the cutoff pairs, two floats per neighbour, before the powers are
-// needed; with stored moments only those)
+// neighbours per chunk of function rows (G: 32 and adjoint: 64, which frees LDS
+// for more resident wavefronts; tangent: every neighbour at once while a row is
+// short, up to degree 2, else 32), and the floats of the region that holds them (it also holds the cutoff pairs, two floats per neighbour, before
+// the rows are needed; with stored moments only those)
 constexpr int kPwRows = 64;
 // adjoint: dE/dT entries per lane held in registers while they replace the moments
 constexpr int kUbRegs = 8;
-__host__ __device__ inline int pw_chunk(int mode, int maxn) {
-    return mode == 2 ? maxn : (mode == 0 || mode == 3 ? kPwRows / 2 : kPwRows);
+__host__ __device__ inline int pw_chunk(int mode, int maxn, int pws) {
+    return mode == 2 && pws <= 32 ? maxn : (mode == 1 ? kPwRows : kPwRows / 2);
 }
 __host__ __device__ inline int pw_floats(int mode, int maxn, int pws, bool haveT) {
-    const int rows = pw_chunk(mode, maxn);
+    const int rows = pw_chunk(mode, maxn, pws);
     if (mode == 3) {                                // fused: also the adjoint vectors and network vectors
         const int m = rows * pws > 3 * maxn ? rows * pws : 3 * maxn;
         return m > 3 * kVecMaxWidth ? m : 3 * kVecMaxWidth;
     }
     return haveT ? 2 * maxn : (rows * pws > 2 * maxn ? rows * pws : 2 * maxn);
 }
-__host__ __device__ constexpr int mono_start(int m) { return m * (m + 1) * (m + 2) / 6; }
-__host__ __device__ constexpr int ifact(int n) { return n <= 1 ? 1 : n * ifact(n - 1); }
-// position of x^a y^b z^c in the monomial order below
-__host__ __device__ constexpr int mono_index(int a, int b, int c) {
-    return mono_start(a + b + c) + (b + c) * (b + c + 1) / 2 + c;
-}
-
-// monomials of total degree <= kMomZ ordered by degree, then exponent of x and
-// y descending; every smaller degree bound is a prefix
-struct MonoTable {
-    int a[nmono(kMomZ)], b[nmono(kMomZ)], c[nmono(kMomZ)], m[nmono(kMomZ)];
-    float w[nmono(kMomZ)];
-    constexpr MonoTable() : a(), b(), c(), m(), w() {
-        int q = 0;
-        for (int mm = 0; mm <= kMomZ; ++mm)
-            for (int aa = mm; aa >= 0; --aa)
-                for (int bb = mm - aa; bb >= 0; --bb) {
-                    const int cc = mm - aa - bb;
-                    a[q] = aa; b[q] = bb; c[q] = cc; m[q] = mm;
-                    w[q] = (float)(ifact(mm) / (ifact(aa) * ifact(bb) * ifact(cc)));
-                    ++q;
-                }
-    }
-};
-__constant__ MonoTable c_mono = MonoTable();
 
 __device__ __forceinline__ int pair_of(int b, int c) { return b <= c ? c * (c + 1) / 2 + b : b * (b + 1) / 2 + c; }
 
@@ -1042,11 +1022,12 @@ __device__ __forceinline__ void fused_net(const SymmArgs& A, const NetDesc& D, i
 // the waves of a workgroup are independent.
 template <int MODE, int Z>
 __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, float4* smem4) {
-    constexpr int NM = nmono(Z);
+    constexpr int NM = nharm(Z);
     constexpr int ZP = Z + 1;
-    constexpr int PWS = (3 * ZP * (MODE == 2 ? 2 : 1)) | 1;   // powers per neighbour, odd stride
+    constexpr int PWS = (NM * (MODE == 2 ? 2 : 1)) | 1;      // function values per neighbour, odd stride
     constexpr int U4 = kMaxUnionEta;
-    constexpr int NG = kWave / NM;                           // lane groups over the neighbours
+    constexpr int NW = NM <= 4 ? 4 : (NM <= 16 ? 16 : (NM <= 32 ? 32 : kWave));   // lanes of one group
+    constexpr int NG = kWave / NW;                           // lane groups over the neighbours
     constexpr bool FUSED = MODE == 3;                        // G, network and adjoint of the atom
     constexpr bool ADJ = MODE == 1 || FUSED;                 // per-slot adjoint vectors written
     constexpr int GM = FUSED ? 0 : MODE;                     // mode of the basis phase
@@ -1082,9 +1063,7 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
     // adjoint: dE/dT overwrites the moments when it fits a few registers per lane
     const bool ub_in_T = S * NM * U4 <= kUbRegs * kWave;
     float* Ub = ub_in_T ? T : Am + NP * U4 * ZP;               // [S][NM][U4] (mode 1)
-    float* part = Am + NP * U4 * ZP + (ADJ && !ub_in_T ? S * NM * U4 : 0);   // [NG][NM][U4] x (1 or 2)
-    float* wq = part + (NG > 1 ? NG * NM * U4 * (MODE == 2 ? 2 : 1) : 0);   // [NM] monomial weights
-    float* nb = FUSED ? pw : wq + NM;                           // fused: [3][kVecMaxWidth] network vectors (power rows' region)
+    float* nb = pw;                                             // fused: [3][kVecMaxWidth] network vectors (function rows' region)
     // cutoffs live in the power rows until the radial part is done (fused: the
     // adjoint's radial part runs after the moments, so they have their own rows)
     sm.fg = reinterpret_cast<float2*>(FUSED ? fgr : pw);
@@ -1106,7 +1085,6 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
         }
     }
     n = fast_load(A, Mo, i, a, o, n, sm, MODE != 0, ADJ, MODE == 2 ? tv : nullptr);
-    if (lane < NM) wq[lane] = c_mono.w[lane];
     if (MODE == 1) {
 #pragma unroll
         for (int h = 0; h < kPreD; ++h) {
@@ -1129,123 +1107,88 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
         }
         for (int q = kPreT * kWave + lane; q < TS; q += kWave) T[q] = A.Tin[(size_t)i * TS + q];
     }
-    // powers of the unit vector (and, for the tangent, their derivatives along
-    // the projected direction (t - r^ (r^.t)) / r) of neighbours c0 .. c1-1,
+    // function values of the unit vector (and, for the tangent, their derivatives
+    // along the projected direction (t - r^ (r^.t)) / r) of neighbours c0 .. c1-1,
     // at most pw_chunk, into the chunk rows (the moment loop below walks each
     // species segment in such chunks, so for G and the adjoint the rows take a
     // fixed slice of LDS instead of one row per neighbour)
-    auto power_rows = [&](int c0, int c1) {
+    auto function_rows = [&](int c0, int c1) {
         for (int J = c0 + lane; J < c1; J += kWave) {
             const float4 gq = sm.g[J];
             float* row = pw + (size_t)(J - c0) * PWS;
-            const float v3[3] = {gq.x, gq.y, gq.z};
-            float d3[3] = {0.f, 0.f, 0.f};
+            float C[ZP], Sn[ZP], q[qidx(Z, Z) + 1], y[NM];
+            harm_factors<Z, float>(gq.x, gq.y, gq.z, C, Sn, q);
+            harm_values<Z, float>(C, Sn, q, y);
+#pragma unroll
+            for (int f = 0; f < NM; ++f) row[f] = y[f];
             if (MODE == 2) {
                 const float4 t4 = tv[J];
-                d3[0] = (t4.x - gq.x * t4.w) * gq.w;
-                d3[1] = (t4.y - gq.y * t4.w) * gq.w;
-                d3[2] = (t4.z - gq.z * t4.w) * gq.w;
-            }
+                harm_along<Z, float>(C, Sn, q, (t4.x - gq.x * t4.w) * gq.w, (t4.y - gq.y * t4.w) * gq.w,
+                                     (t4.z - gq.z * t4.w) * gq.w, y);
 #pragma unroll
-            for (int x = 0; x < 3; ++x) {
-                float p = 1.0f;
-#pragma unroll
-                for (int k = 0; k < ZP; ++k) {
-                    if (MODE == 2) row[3 * ZP + x * ZP + k] = k == 0 ? 0.0f : (float)k * p * d3[x];
-                    row[x * ZP + k] = k == 0 ? 1.0f : (p *= v3[x]);
-                }
+                for (int f = 0; f < NM; ++f) row[NM + f] = y[f];
             }
         }
     };
     wave_sync();
-    // moments T_b[u][alpha]: lane = (alpha, group); groups stride the neighbours.
-    // G with zeta 4 (35 monomials, one group would leave 29 lanes idle):
-    // monomials 1, x, y, z are summed with the diagonal sums below and the other
-    // 31 run as two groups of 32 lanes, joined by one cross-half exchange.
-    constexpr bool SPLIT = GM == 0 && NM == 35;
-    constexpr int NGL = SPLIT ? 2 : NG;                        // neighbour groups of the loop
+    // moments T_b[u][f]: lane = (function, group); groups stride the neighbours
     if (!haveT) {
-        const int al = SPLIT ? min(4 + lane % 32, NM - 1) : lane % NM;
-        const int grp = SPLIT ? lane / 32 : lane / NM;
-        const bool act = SPLIT ? lane % 32 < 31 : grp < NG;
-        const int ea = c_mono.a[al], eb = c_mono.b[al], ec = c_mono.c[al];
+        const int al = lane % NW, grp = lane / NW;
+        const bool act = al < NM;
         for (int b = 0; b < S; ++b) {
             const int s0 = sm.seg[b], s1 = sm.seg[b + 1];
             float acc[U4], dacc[U4];
 #pragma unroll
             for (int u = 0; u < U4; ++u) { acc[u] = 0.0f; dacc[u] = 0.0f; }
-            // one neighbour of the segment: T[u][alpha] += e_u(r) r^^alpha
+            // one neighbour of the segment: T[u][f] += e_u(r) Y_f(r^)
             auto step = [&](const float* row, int J) {
-                const float px = row[ea], py = row[ZP + eb], pz = row[2 * ZP + ec];
-                const float mono = px * py * pz;
+                const float yv = row[al];
                 const float4 e4 = sm.ef[J];
-                acc[0] += e4.x * mono; acc[1] += e4.y * mono; acc[2] += e4.z * mono; acc[3] += e4.w * mono;
+                acc[0] += e4.x * yv; acc[1] += e4.y * yv; acc[2] += e4.z * yv; acc[3] += e4.w * yv;
                 if (MODE == 2) {
-                    const float dmono = row[3 * ZP + ea] * py * pz + px * row[4 * ZP + eb] * pz +
-                                        px * py * row[5 * ZP + ec];
+                    const float dy = row[NM + al];
                     const float4 f4 = sm.efd[J];
-                    const float wm = tv[J].w * mono;
-                    dacc[0] += f4.x * wm + e4.x * dmono;
-                    dacc[1] += f4.y * wm + e4.y * dmono;
-                    dacc[2] += f4.z * wm + e4.z * dmono;
-                    dacc[3] += f4.w * wm + e4.w * dmono;
+                    const float wm = tv[J].w * yv;
+                    dacc[0] += f4.x * wm + e4.x * dy;
+                    dacc[1] += f4.y * wm + e4.y * dy;
+                    dacc[2] += f4.z * wm + e4.z * dy;
+                    dacc[3] += f4.w * wm + e4.w * dy;
                 }
             };
-            const int chunk = pw_chunk(MODE, maxn);
+            const int chunk = pw_chunk(MODE, maxn, PWS);
             for (int c0 = s0; c0 < s1; c0 += chunk) {
                 const int c1 = min(c0 + chunk, s1);
                 wave_sync();                                    // the previous chunk's rows are read
-                power_rows(c0, c1);
+                function_rows(c0, c1);
                 wave_sync();
                 if (act) {
                     int J = c0 + grp;
-                    // four neighbours per trip: their power rows sit at fixed offsets
+                    // four neighbours per trip: their rows sit at fixed offsets
                     // from one address, so the loads use immediate offsets and overlap
-                    for (; J + 3 * NGL < c1; J += 4 * NGL) {
+                    for (; J + 3 * NG < c1; J += 4 * NG) {
                         const float* row = pw + (size_t)(J - c0) * PWS;
                         step(row, J);
-                        step(row + NGL * PWS, J + NGL);
-                        step(row + 2 * NGL * PWS, J + 2 * NGL);
-                        step(row + 3 * NGL * PWS, J + 3 * NGL);
+                        step(row + NG * PWS, J + NG);
+                        step(row + 2 * NG * PWS, J + 2 * NG);
+                        step(row + 3 * NG * PWS, J + 3 * NG);
                     }
-                    for (; J < c1; J += NGL) step(pw + (size_t)(J - c0) * PWS, J);
+                    for (; J < c1; J += NG) step(pw + (size_t)(J - c0) * PWS, J);
                 }
             }
-            if (SPLIT) {
+            // butterflies over the groups, whose width is a power of two
 #pragma unroll
-                for (int u = 0; u < U4; ++u) acc[u] += __shfl_xor(acc[u], 32);
-                if (act && grp == 0) {
+            for (int bit = NW; bit < kWave; bit <<= 1)
 #pragma unroll
-                    for (int u = 0; u < U4; ++u) T[(b * U4 + u) * NM + al] = acc[u];
+                for (int u = 0; u < U4; ++u) {
+                    acc[u] += __shfl_xor(acc[u], bit);
+                    if (MODE == 2) dacc[u] += __shfl_xor(dacc[u], bit);
                 }
-            } else if (NG == 1) {
-                if (act) {
+            if (lane < NM) {
 #pragma unroll
-                    for (int u = 0; u < U4; ++u) {
-                        T[(b * U4 + u) * NM + al] = acc[u];
-                        if (MODE == 2) dT[(b * U4 + u) * NM + al] = dacc[u];
-                    }
+                for (int u = 0; u < U4; ++u) {
+                    T[(b * U4 + u) * NM + al] = acc[u];
+                    if (MODE == 2) dT[(b * U4 + u) * NM + al] = dacc[u];
                 }
-            } else {
-                if (act) {
-#pragma unroll
-                    for (int u = 0; u < U4; ++u) {
-                        part[(grp * NM + al) * U4 + u] = acc[u];
-                        if (MODE == 2) part[NG * NM * U4 + (grp * NM + al) * U4 + u] = dacc[u];
-                    }
-                }
-                wave_sync();
-                for (int q = lane; q < NM * U4; q += kWave) {
-                    float s = 0.0f, ds = 0.0f;
-                    for (int gq = 0; gq < NG; ++gq) {
-                        s += part[gq * NM * U4 + q];
-                        if (MODE == 2) ds += part[NG * NM * U4 + gq * NM * U4 + q];
-                    }
-                    const int al2 = q / U4, u = q % U4;
-                    T[(b * U4 + u) * NM + al2] = s;
-                    if (MODE == 2) dT[(b * U4 + u) * NM + al2] = ds;
-                }
-                wave_sync();
             }
         }
         // diagonal sums D_b[u] (mode 2 also their tangent): lanes over the
@@ -1255,23 +1198,9 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
                 float d4[U4], t4[U4];
 #pragma unroll
                 for (int u = 0; u < U4; ++u) { d4[u] = 0.0f; t4[u] = 0.0f; }
-                float lo[SPLIT ? 4 * U4 : 1];                  // [u][1, x, y, z] (split G)
-#pragma unroll
-                for (int q = 0; q < (SPLIT ? 4 * U4 : 1); ++q) lo[q] = 0.0f;
                 for (int J = sm.seg[b] + lane; J < sm.seg[b + 1]; J += kWave) {
                     const float4 e4 = sm.ef[J];
                     d4[0] += e4.x * e4.x; d4[1] += e4.y * e4.y; d4[2] += e4.z * e4.z; d4[3] += e4.w * e4.w;
-                    if (SPLIT) {
-                        const float4 gq = sm.g[J];
-                        const float ev[U4] = {e4.x, e4.y, e4.z, e4.w};
-#pragma unroll
-                        for (int u = 0; u < U4; ++u) {
-                            lo[4 * u] += ev[u];
-                            lo[4 * u + 1] += ev[u] * gq.x;
-                            lo[4 * u + 2] += ev[u] * gq.y;
-                            lo[4 * u + 3] += ev[u] * gq.z;
-                        }
-                    }
                     if (MODE == 2) {
                         const float4 f4 = sm.efd[J];
                         const float w2 = 2.0f * tv[J].w;
@@ -1282,12 +1211,6 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
                 int idx;
                 const float sd = wave_sum_multi<U4>(d4, idx);
                 if ((lane & (kWave / U4 - 1)) == 0) D[b * U4 + idx] = sd;
-                if (SPLIT) {
-                    // monomial order starts 1, x, y, z (degree 0, then x, y, z)
-                    int qi;
-                    const float sl = wave_sum_multi<(SPLIT ? 4 * U4 : 1)>(lo, qi);
-                    if ((lane & (kWave / (4 * U4) - 1)) == 0) T[(b * U4 + qi / 4) * NM + qi % 4] = sl;
-                }
                 if (MODE == 2) {
                     const float st = wave_sum_multi<U4>(t4, idx);
                     if ((lane & (kWave / U4 - 1)) == 0) dD[b * U4 + idx] = st;
@@ -1317,7 +1240,7 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
 #pragma unroll
             for (int k = 0; k < kGridK; ++k) {
                 om[k] = B.outm[u * nk + k];
-                mc[k] = B.mcoef[k][m];
+                mc[k] = B.lcoef[k][m];
             }
             float s = 0.0f;
             if (use) {
@@ -1340,17 +1263,17 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
             const float* Tc = T + (c * U4 + u) * NM;
             const float* dTb = dT + (b * U4 + u) * NM;
             const float* dTc = dT + (c * U4 + u) * NM;
-            // degree m has (m + 1)(m + 2) / 2 monomials; every lane runs the
-            // length of the highest degree with the surplus terms weighted 0, so
-            // all loads are issued before the first product instead of one
-            // dependent round per monomial
-            constexpr int QD = (Z + 1) * (Z + 2) / 2;
-            const int q0 = mono_start(m), q1 = mono_start(m + 1);
+            // degree m has 2m + 1 functions; every lane runs the length of the
+            // highest degree with the surplus terms weighted 0, so all loads are
+            // issued before the first product instead of one dependent round per
+            // function
+            constexpr int QD = 2 * Z + 1;
+            const int q0 = m * m, q1 = q0 + 2 * m + 1;
 #pragma unroll
             for (int j = 0; j < QD; ++j) {
                 const int q = min(q0 + j, NM - 1);
-                const float w = q0 + j < q1 ? wq[q] : 0.0f;
-                s += GM == 0 ? w * Tb[q] * Tc[q] : w * (dTb[q] * Tc[q] + Tb[q] * dTc[q]);
+                const float w = q0 + j < q1 ? 1.0f : 0.0f;
+                s += GM == 0 ? (w * Tb[q]) * Tc[q] : w * (dTb[q] * Tc[q] + Tb[q] * dTc[q]);
             }
             if (b == c) s = 0.5f * (s - (GM == 0 ? D[b * U4 + u] : dD[b * U4 + u]));
         }
@@ -1368,7 +1291,7 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
             const int om = B.outm[g * nk + k];   // < kGridG * kGridK; used only when use
             float mc[ZP];
 #pragma unroll
-            for (int m = 0; m < ZP; ++m) mc[m] = B.mcoef[k][m];
+            for (int m = 0; m < ZP; ++m) mc[m] = B.lcoef[k][m];
             if (use) {
                 float v = 0.0f;
 #pragma unroll
@@ -1397,12 +1320,12 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
     // adjoint: dE/dT_b[alpha][u] and dE/dD_b[u]
     auto dEdT = [&](int it) {
         const int b = it / (NM * U4), al = (it / U4) % NM, u = it % U4;
-        int m = 0;   // degree of monomial al
+        int m = 0;   // degree of function al
 #pragma unroll
-        for (int mm = 1; mm <= Z; ++mm) m += al >= mono_start(mm) ? 1 : 0;
+        for (int mm = 1; mm <= Z; ++mm) m += al >= mm * mm ? 1 : 0;
         float s = 0.0f;
         for (int c = 0; c < S; ++c) s += Am[(pair_of(b, c) * U4 + u) * ZP + m] * T[(c * U4 + u) * NM + al];
-        return wq[al] * s;
+        return s;
     };
     if (ub_in_T) {
         // every lane's entries in registers, then written over the moments
@@ -1428,37 +1351,14 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
         dD[lane] = -0.5f * s;
     }
     wave_sync();
-    // per neighbour: Q(r^) = sum_alpha W_alpha r^^alpha and grad of sum V_alpha r^^alpha
-    constexpr MonoTable mt{};
+    // per neighbour: the radial and angular derivatives of sum_u e_u sum_f dE/dT[f][u] Y_f
     for (int J = lane; J < n; J += kWave) {
         int b = 0;
         while (b + 1 < S && J >= sm.seg[b + 1]) ++b;
         const float4 gq = sm.g[J];
         const float4 e4 = sm.ef[J], f4 = sm.efd[J];
-        // every monomial of r^ once (one product each from a lower one); the
-        // gradient of x^a y^b z^c is (a, b, c) times monomials of one degree less
-        float mono[NM];
-        mono[0] = 1.0f;
-#pragma unroll
-        for (int q = 1; q < NM; ++q) {
-            const int ea = mt.a[q], eb = mt.b[q], ec = mt.c[q];
-            mono[q] = ea > 0 ? mono[mono_index(ea > 0 ? ea - 1 : 0, eb, ec)] * gq.x
-                             : (eb > 0 ? mono[mono_index(ea, eb > 0 ? eb - 1 : 0, ec)] * gq.y
-                                       : mono[mono_index(ea, eb, ec > 0 ? ec - 1 : 0)] * gq.z);
-        }
-        float Qd = 0.0f, g0 = 0.0f, g1 = 0.0f, g2 = 0.0f;
-        const float4* Ubb = reinterpret_cast<const float4*>(Ub + b * NM * U4);
-#pragma unroll
-        for (int q = 0; q < NM; ++q) {
-            const int ea = mt.a[q], eb = mt.b[q], ec = mt.c[q];
-            const float4 w4 = Ubb[q];
-            const float V = e4.x * w4.x + e4.y * w4.y + e4.z * w4.z + e4.w * w4.w;
-            const float W = f4.x * w4.x + f4.y * w4.y + f4.z * w4.z + f4.w * w4.w;
-            Qd += W * mono[q];
-            if (ea > 0) g0 += (V * (float)ea) * mono[mono_index(ea > 0 ? ea - 1 : 0, eb, ec)];
-            if (eb > 0) g1 += (V * (float)eb) * mono[mono_index(ea, eb > 0 ? eb - 1 : 0, ec)];
-            if (ec > 0) g2 += (V * (float)ec) * mono[mono_index(ea, eb, ec > 0 ? ec - 1 : 0)];
-        }
+        float Qd, g0, g1, g2;
+        harm_adjoint<Z>(gq.x, gq.y, gq.z, e4, f4, reinterpret_cast<const float4*>(Ub + b * NM * U4), Qd, g0, g1, g2);
         const float dd = 2.0f * (dD[b * U4] * e4.x * f4.x + dD[b * U4 + 1] * e4.y * f4.y +
                                  dD[b * U4 + 2] * e4.z * f4.z + dD[b * U4 + 3] * e4.w * f4.w);
         const float rg = gq.x * g0 + gq.y * g1 + gq.z * g2;
@@ -1531,18 +1431,15 @@ __global__ void k_queue_reset(int* __restrict__ queue) {
 
 // LDS bytes of one wavefront of moment_atom<mode> (the layout at its top)
 static size_t moment_smem(const SymmArgs& A, int mode, int Z, int S, int NP) {
-    const int NM = nmono(Z), ZP = Z + 1, U4 = kMaxUnionEta;
+    const int NM = nharm(Z), ZP = Z + 1, U4 = kMaxUnionEta;
     const bool adj = mode == 1 || mode == 3;
-    const int PWS = (mode == 1 && A.Tin) ? 2 : (3 * ZP * (mode == 2 ? 2 : 1)) | 1;
-    const int NG = kWave / NM;
+    const int PWS = (mode == 1 && A.Tin) ? 2 : (NM * (mode == 2 ? 2 : 1)) | 1;
     size_t b = 16 * (size_t)A.maxn * (2 + (mode == 0 ? 0 : 1) + (mode == 2 ? 1 : 0));
     b += 4 * (adj ? 2 : 1) * (size_t)A.maxn + 4 * 16;                              // r, canon (adjoint), seg
     size_t f = (size_t)A.ldg + (mode == 1 ? 3 * (size_t)A.maxn : 0) + (mode == 3 ? 2 * (size_t)A.maxn : 0) +
                (size_t)pw_floats(mode, A.maxn, PWS, mode == 1 && A.Tin);
     f += (size_t)S * U4 * NM * (mode == 2 ? 2 : 1) + 2 * (size_t)S * U4 + (size_t)NP * U4 * ZP;
     f += (adj && S * NM * U4 > kUbRegs * kWave ? (size_t)S * NM * U4 : 0);         // dE/dT beside the moments
-    f += (NG > 1 ? (size_t)NG * NM * U4 * (mode == 2 ? 2 : 1) : 0);
-    f += NM;
     return b + 4 * f;
 }
 
