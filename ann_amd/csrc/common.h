@@ -92,6 +92,7 @@ struct DevModel {
     NetDesc net[kMaxSpecies];
     int all_grid;                               // every angular block is grid-shaped
     int fast_ng, fast_nk;                       // the common grid shape (0 if blocks differ)
+    int rad_gauss, nrad;                        // every radial block is GAUSSIAN; functions of the widest
     int moment_z;                               // largest zeta if the moment form applies, else 0
     int pre_off[kMaxSpecies + 1];               // FP64-evaluated inputs of species a: items [pre_off[a], pre_off[a+1])
     double uieta2_64[kMaxSpecies][kMaxUnionEta];  // union widths 1/eta^2 in FP64 (FP64-evaluated inputs)
@@ -110,6 +111,7 @@ struct PreItem {
 struct DevArrays {
     float* rad_rs = nullptr;
     float* rad_eta = nullptr;
+    float* rad_etal = nullptr;   // rad_eta times sqrt(log2 e)
     float* ang_eta = nullptr;
     float* ang_zeta = nullptr;
     float* ang_lam = nullptr;

@@ -60,6 +60,10 @@ struct SymmArgs {
     float* v;
     float* Tout;              // moment form, G: store each atom's moments T here (or null)
     const float* Tin;         // moment form, adjoint: moments of the same geometry (or null: recompute)
+    const float* rad_etal;    // rad_eta times sqrt(log2 e)
+    int rad_gauss;            // every radial block is GAUSSIAN
+    int nrad, nrs;            // widest radial block; its row stride in the adjoint's tables (odd)
+    int adjK;                 // atoms per wavefront of the stored-moment adjoint
     // fused E+F (mode 3): the network's parameter tables and inputs, the atom energies
     const float* wchunk;      // forward weight rows, biases, output neuron (net_dev.h layout)
     const float* wtrans;      // transposed weight rows (backward)
@@ -892,20 +896,21 @@ __global__ __launch_bounds__(64) void k_fast(SymmArgs A) {
 // neighbours per chunk of function rows (G: 32 and adjoint: 64, which frees LDS
 // for more resident wavefronts; tangent: every neighbour at once while a row is
 // short, up to degree 2, else 32), and the floats of the region that holds them (it also holds the cutoff pairs, two floats per neighbour, before
-// the rows are needed; with stored moments only those)
+// the rows are needed).  Mode 1 here is the adjoint that recomputes the moments:
+// it serves calls whose geometry no G call has seen
 constexpr int kPwRows = 64;
 // adjoint: dE/dT entries per lane held in registers while they replace the moments
 constexpr int kUbRegs = 8;
 __host__ __device__ inline int pw_chunk(int mode, int maxn, int pws) {
     return mode == 2 && pws <= 32 ? maxn : (mode == 1 ? kPwRows : kPwRows / 2);
 }
-__host__ __device__ inline int pw_floats(int mode, int maxn, int pws, bool haveT) {
+__host__ __device__ inline int pw_floats(int mode, int maxn, int pws) {
     const int rows = pw_chunk(mode, maxn, pws);
     if (mode == 3) {                                // fused: also the adjoint vectors and network vectors
         const int m = rows * pws > 3 * maxn ? rows * pws : 3 * maxn;
         return m > 3 * kVecMaxWidth ? m : 3 * kVecMaxWidth;
     }
-    return haveT ? 2 * maxn : (rows * pws > 2 * maxn ? rows * pws : 2 * maxn);
+    return rows * pws > 2 * maxn ? rows * pws : 2 * maxn;
 }
 
 __device__ __forceinline__ int pair_of(int b, int c) { return b <= c ? c * (c + 1) / 2 + b : b * (b + 1) / 2 + c; }
@@ -1050,12 +1055,10 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
     // [maxn][3] adjoint vectors (mode 1; fused: they share the power rows'
     // region, whose rows are dead once the moments are summed)
     float* sP = rowbuf + ldg + (FUSED ? 2 * maxn : 0);
-    // adjoint with stored moments: no power rows (the cutoff pairs still use their space)
-    const bool haveT = MODE == 1 && A.Tin != nullptr;
     const int TS = S * U4 * NM;                                 // moments per atom
     float* fgr = rowbuf + ldg;                                  // fused: [maxn] cutoff pairs of their own
     float* pw = FUSED ? sP : sP + (MODE == 1 ? 3 * maxn : 0);  // [pw_chunk][PWS] (one chunk of neighbours)
-    float* T = pw + pw_floats(MODE, maxn, PWS, haveT);         // [S][U4][NM]
+    float* T = pw + pw_floats(MODE, maxn, PWS);                // [S][U4][NM]
     float* dT = T + S * U4 * NM;                                // [S][U4][NM] (mode 2)
     float* D = dT + (MODE == 2 ? S * U4 * NM : 0);              // [S][U4]
     float* dD = D + S * U4;                                     // [S][U4] (mode 2: dD, mode 1: dE/dD)
@@ -1068,30 +1071,9 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
     // adjoint's radial part runs after the moments, so they have their own rows)
     sm.fg = reinterpret_cast<float2*>(FUSED ? fgr : pw);
 
-    // adjoint: the dE/dG row and the stored moments are loaded before the neighbours so
-    // that their latency overlaps the neighbour load (registers, written to LDS below)
-    constexpr int kPreT = 8, kPreD = 2;                         // moments / dE/dG prefetched per lane
-    float pre_d[kPreD], pre_t[kPreT];
-    if (MODE == 1) {
-#pragma unroll
-        for (int h = 0; h < kPreD; ++h) {
-            const int m = lane + h * kWave;
-            pre_d[h] = m < ldg ? A.dEdG[(size_t)i * ldg + m] : 0.0f;
-        }
-#pragma unroll
-        for (int h = 0; h < kPreT; ++h) {
-            const int q = lane + h * kWave;
-            pre_t[h] = (haveT && q < TS) ? A.Tin[(size_t)i * TS + q] : 0.0f;
-        }
-    }
     n = fast_load(A, Mo, i, a, o, n, sm, MODE != 0, ADJ, MODE == 2 ? tv : nullptr);
     if (MODE == 1) {
-#pragma unroll
-        for (int h = 0; h < kPreD; ++h) {
-            const int m = lane + h * kWave;
-            if (m < ldg) rowbuf[m] = pre_d[h];
-        }
-        for (int m = kPreD * kWave + lane; m < ldg; m += kWave) rowbuf[m] = A.dEdG[(size_t)i * ldg + m];
+        for (int m = lane; m < ldg; m += kWave) rowbuf[m] = A.dEdG[(size_t)i * ldg + m];
         for (int t = lane; t < 3 * n; t += kWave) sP[t] = 0.0f;
     } else {
         for (int m = lane; m < ldg; m += kWave) rowbuf[m] = 0.0f;
@@ -1099,14 +1081,6 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
     wave_sync();
     fast_radial<GM>(A, Mo, a, sm, tv, rowbuf, sP, rowbuf);
     wave_sync();
-    if (haveT) {
-#pragma unroll
-        for (int h = 0; h < kPreT; ++h) {
-            const int q = lane + h * kWave;
-            if (q < TS) T[q] = pre_t[h];
-        }
-        for (int q = kPreT * kWave + lane; q < TS; q += kWave) T[q] = A.Tin[(size_t)i * TS + q];
-    }
     // function values of the unit vector (and, for the tangent, their derivatives
     // along the projected direction (t - r^ (r^.t)) / r) of neighbours c0 .. c1-1,
     // at most pw_chunk, into the chunk rows (the moment loop below walks each
@@ -1132,7 +1106,7 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
     };
     wave_sync();
     // moments T_b[u][f]: lane = (function, group); groups stride the neighbours
-    if (!haveT) {
+    {
         const int al = lane % NW, grp = lane / NW;
         const bool act = al < NM;
         for (int b = 0; b < S; ++b) {
@@ -1376,6 +1350,206 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
     }
 }
 
+// Adjoint with stored moments.  One wavefront serves K consecutive atoms; its
+// lanes run over the atoms' list entries in list order, which are contiguous,
+// so every entry's vector stays in registers from the load to the store: no
+// regrouping by species and no LDS row per neighbour.  What differs between
+// entries (centre and neighbour species) is an LDS table per (atom, species):
+// the radial functions with their dE/dG and the moment adjoints dE/dT.
+//   1. dE/dG rows and moments of the K atoms into LDS;
+//   2. per block, width and degree, A = sum over functions of dE/dG times the
+//      Legendre coefficient; dE/dT[b][f] = sum_c A(b, c) T[c][f];
+//   3. lanes over entries: cutoff, radial sum, harm_adjoint, store.
+// The entries of two atoms fill the 64 lanes better than one atom's (water: 85
+// entries take two passes, 170 take three); K comes from the batch
+// (adj_atoms).  LDS does not depend on the widest row, so the registers
+// alone set the number of resident wavefronts, also for lists with a skin.
+// Bound by vector issue: about 1,300 wave instructions per atom (water, two atoms
+// per wavefront) against 2,800 of the form with one LDS row per neighbour.
+// Measured against it: 1,048,576 atoms, list with a skin, 8.57 -> 3.15 ms;
+// 273,561 atoms 1285 -> 576 us; 12,288 atoms 54 -> 36 us; Li/P/S, 21,872 atoms,
+// 67 -> 37 us.
+constexpr int kAdjAtoms = 2;
+
+// float4 entries of the wavefront's LDS slice (layout at the top of adjoint_wave)
+__host__ __device__ inline int adj_units(int K, int Z, int S, int NP, int nrs, int ldg) {
+    const int NM = nharm(Z), U4 = kMaxUnionEta;
+    return K * S * (NM | 1) + K * S * nrs + K * S + K * S * NM + K * (ldg / 4) + (K * NP * U4 * (Z + 1) + 3) / 4;
+}
+
+template <int Z>
+__device__ __forceinline__ void adjoint_wave(const SymmArgs& A, const int i0, const int K, float4* smem4) {
+    constexpr int NM = nharm(Z), NS = NM | 1, ZP = Z + 1, U4 = kMaxUnionEta;
+    const int lane = threadIdx.x % kWave;
+    const DevModel& Mo = *A.dm;
+    const int S = Mo.S, NP = Mo.NP, ldg = A.ldg, nrs = A.nrs;
+    float4* W = smem4;                                          // [K][S][NS] dE/dT, widths in the components
+    float4* R = W + K * S * NS;                                 // [K][S][nrs] radial: eta, rs, dE/dG, dE/dG eta
+    float4* dD = R + K * S * nrs;                               // [K][S] dE/dD
+    float* T = reinterpret_cast<float*>(dD + K * S);            // [K][S][U4][NM]
+    float* row = T + K * S * U4 * NM;                           // [K][ldg]
+    float* Am = row + K * ldg;                                  // [K][NP][U4][ZP]
+    int o[kAdjAtoms + 1], sp[kAdjAtoms];
+#pragma unroll
+    for (int q = 0; q <= kAdjAtoms; ++q) o[q] = A.off[i0 + min(q, K)];
+#pragma unroll
+    for (int q = 0; q < kAdjAtoms; ++q) sp[q] = A.species[i0 + min(q, K - 1)];
+    const int s_end = o[kAdjAtoms];
+    // the first entries' loads are in flight while the tables are built
+    int s = o[0] + lane;
+    float4 gn = make_float4(0.f, 0.f, 0.f, 0.f);
+    int bn = 0;
+    if (s < s_end) {
+        gn = A.geo[s];
+        bn = A.nsp[s];
+    }
+    {
+        const float4* gT = reinterpret_cast<const float4*>(A.Tin + (size_t)i0 * S * U4 * NM);
+        float4* lT = reinterpret_cast<float4*>(T);
+        for (int x = lane; x < K * S * NM; x += kWave) lT[x] = gT[x];
+        // the caller's rows: no alignment beyond a float's
+        for (int x = lane; x < K * ldg; x += kWave) row[x] = A.dEdG[(size_t)i0 * ldg + x];
+    }
+    wave_sync();
+    auto spec = [&](int q) {                                    // species of atom q, without a register array index
+        int a = sp[0];
+#pragma unroll
+        for (int k = 1; k < kAdjAtoms; ++k)
+            if (q == k) a = sp[k];
+        return a;
+    };
+    // radial tables (functions past a block's own carry dE/dG = 0)
+    for (int x = lane; x < K * S * nrs; x += kWave) {
+        const int m = x % nrs, b = (x / nrs) % S, q = x / (nrs * S);
+        const RadBlock rb = Mo.rad[spec(q) * S + b];
+        float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (m < rb.n) {
+            const float e = A.rad_gauss ? A.rad_etal[rb.par + m] : A.rad_eta[rb.par + m], g = row[q * ldg + rb.goff + m];
+            t = make_float4(e, A.rad_rs[rb.par + m], g, g * e);
+        }
+        R[x] = t;
+    }
+    // angular seeds: lanes over (atom, pair, width, degree); every descriptor load
+    // of a lane is issued before the first use
+    for (int x = lane; x < K * NP * U4 * ZP; x += kWave) {
+        const int l = x % ZP, u = (x / ZP) % U4, p = (x / (ZP * U4)) % NP, q = x / (ZP * U4 * NP);
+        const AngBlock& B = Mo.ang[spec(q) * NP + p];
+        const int nk = min(max(B.nk, 0), kGridK), goff = B.goff;
+        const bool use = B.n > 0 && u < B.ng;
+        int om[kGridK];
+        float lc[kGridK];
+#pragma unroll
+        for (int k = 0; k < kGridK; ++k) {
+            om[k] = B.outm[u * nk + k];                         // past nk: read, not used
+            lc[k] = B.lcoef[k][l];
+        }
+        float v = 0.0f;
+        if (use) {
+#pragma unroll
+            for (int k = 0; k < kGridK; ++k)
+                if (k < nk) v += row[q * ldg + goff + om[k]] * lc[k];
+        }
+        Am[x] = v;
+    }
+    wave_sync();
+    // dE/dT and dE/dD: lanes over (atom, species, function, width)
+    for (int x = lane; x < K * S * NM * U4; x += kWave) {
+        const int u = x % U4, f = (x / U4) % NM, b = (x / (U4 * NM)) % S, q = x / (U4 * NM * S);
+        int l = 0;                                              // degree of function f
+#pragma unroll
+        for (int d = 1; d <= Z; ++d) l += f >= d * d ? 1 : 0;
+        const float* Aq = Am + q * NP * U4 * ZP + u * ZP + l;
+        const float* Tq = T + q * S * U4 * NM + u * NM + f;
+        float v = 0.0f;
+        for (int c = 0; c < S; ++c) v += Aq[pair_of(b, c) * U4 * ZP] * Tq[c * U4 * NM];
+        reinterpret_cast<float*>(W)[((q * S + b) * NS + f) * U4 + u] = v;
+    }
+    for (int x = lane; x < K * S * U4; x += kWave) {
+        const int u = x % U4, b = (x / U4) % S, q = x / (U4 * S);
+        const float* Aq = Am + q * NP * U4 * ZP + (pair_of(b, b) * U4 + u) * ZP;
+        float v = 0.0f;
+#pragma unroll
+        for (int l = 0; l < ZP; ++l) v += Aq[l];
+        reinterpret_cast<float*>(dD)[x] = -0.5f * v;
+    }
+    wave_sync();
+    const float rc = Mo.rc;
+    for (; s < s_end; s += kWave) {
+        const float4 gq = gn;
+        const int b = bn;
+        if (s + kWave < s_end) {
+            gn = A.geo[s + kWave];
+            bn = A.nsp[s + kWave];
+        }
+        int q = 0, a = sp[0];
+#pragma unroll
+        for (int k = 1; k < kAdjAtoms; ++k)
+            if (s >= o[k]) { q = k; a = sp[k]; }
+        float px = 0.0f, py = 0.0f, pz = 0.0f;
+        if (gq.w <= rc) {                                       // entries beyond the cutoff (skin lists) get zero
+            const float r = gq.w, ir = __builtin_amdgcn_rcpf(r);   // 1 ulp
+            const float hx = gq.x * ir, hy = gq.y * ir, hz = gq.z * ir;
+            float fc, gc;
+            cutoff_fg(Mo.cutoff, Mo.rc, Mo.rci, Mo.pirc, r, fc, gc);
+            const int qb = q * S + b;
+            const float4* Rq = R + qb * nrs;
+            float amp;
+            if (A.rad_gauss) {
+                // d/dr [e fc] = e (gc - 2 eta^2 (r - rs) fc); eta carries sqrt(log2 e)
+                float se = 0.0f, sx = 0.0f;
+#pragma unroll 4
+                for (int m = 0; m < A.nrad; ++m) {
+                    const float4 t = Rq[m];
+                    const float x = t.x * (r - t.y), e = __builtin_amdgcn_exp2f(-(x * x));
+                    se += t.z * e;
+                    sx += t.w * (x * e);
+                }
+                amp = se * gc - 1.3862943611198906f * fc * sx;  // 2 / log2 e
+            } else {
+                const RadBlock rb = Mo.rad[a * S + b];
+                amp = 0.0f;
+                for (int m = 0; m < rb.n; ++m) {
+                    const float4 t = Rq[m];
+                    float v, d;
+                    radial_fd(rb.name, t.x, t.y, r, fc, gc, v, d);
+                    amp += t.z * d;
+                }
+            }
+            float e[U4], d[U4];
+#pragma unroll
+            for (int u = 0; u < U4; ++u) {
+                const float k = Mo.uieta2[a][u];                // 0 past the centre's widths: their dE/dT is 0
+                const float x = __expf(-k * r * r);
+                e[u] = x * fc;
+                d[u] = x * (-2.0f * r * k * fc + gc);
+            }
+            const float4 e4 = make_float4(e[0], e[1], e[2], e[3]), d4 = make_float4(d[0], d[1], d[2], d[3]);
+            float rad, g0, g1, g2;
+            harm_adjoint<Z>(hx, hy, hz, e4, d4, W + qb * NS, rad, g0, g1, g2);
+            const float4 D = dD[qb];
+            rad += amp + 2.0f * (D.x * e4.x * d4.x + D.y * e4.y * d4.y + D.z * e4.z * d4.z + D.w * e4.w * d4.w);
+            const float rg = hx * g0 + hy * g1 + hz * g2;
+            px = rad * hx + (g0 - hx * rg) * ir;
+            py = rad * hy + (g1 - hy * rg) * ir;
+            pz = rad * hz + (g2 - hz * rg) * ir;
+        }
+        A.P[3 * (size_t)s] = px;
+        A.P[3 * (size_t)s + 1] = py;
+        A.P[3 * (size_t)s + 2] = pz;
+    }
+}
+
+// Grid dispatch of the stored-moment adjoint: every wavefront of a block takes
+// A.adjK consecutive atoms on its own LDS slice.
+template <int Z>
+__global__ __launch_bounds__(256) void k_adjoint(SymmArgs A) {
+    extern __shared__ float4 smem_all[];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int i0 = (xcd_block(blockIdx.x, gridDim.x) * (blockDim.x / kWave) + wave) * A.adjK;
+    if (i0 >= A.N) return;
+    adjoint_wave<Z>(A, i0, min(A.adjK, A.N - i0), smem_all + (size_t)wave * (A.smem_wave / 16));
+}
+
 // Grid dispatch: a block holds blockDim.x / 64 atoms (the "atoms per
 // workgroup" tuning).
 template <int MODE, int Z>
@@ -1397,6 +1571,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
     if (i >= A.N) return;
     moment_atom<0, Z>(A, i, smem_all + (size_t)wave * (A.smem_wave / 16));
 }
+
+constexpr int kModeAdjT = 4;                                    // the stored-moment adjoint (adjoint_wave)
 
 // Persistent dispatch (a separate kernel, so that the grid kernel keeps its
 // own register allocation): a grid sized to the resident capacity, every
@@ -1420,7 +1596,15 @@ __global__ __launch_bounds__(256) void k_moment_queue(SymmArgs A) {
         int nk = 0;
         if (lane == 0) nk = atomicAdd(ctr, 1);
         const int2 it = A.items[beg + k];
-        for (int a = it.x; a < it.x + it.y; ++a) moment_atom<MODE, Z>(A, a, smem4);
+        if constexpr (MODE == kModeAdjT) {
+            const int ib = __builtin_amdgcn_readfirstlane(it.x), ie = ib + __builtin_amdgcn_readfirstlane(it.y);
+            for (int a = ib; a < ie; a += A.adjK) {
+                adjoint_wave<Z>(A, a, min(A.adjK, ie - a), smem4);
+                wave_sync();                                    // the next atoms reuse the LDS slice
+            }
+        } else {
+            for (int a = it.x; a < it.x + it.y; ++a) moment_atom<MODE, Z>(A, a, smem4);
+        }
         k = __shfl(nk, 0);
     }
 }
@@ -1433,11 +1617,11 @@ __global__ void k_queue_reset(int* __restrict__ queue) {
 static size_t moment_smem(const SymmArgs& A, int mode, int Z, int S, int NP) {
     const int NM = nharm(Z), ZP = Z + 1, U4 = kMaxUnionEta;
     const bool adj = mode == 1 || mode == 3;
-    const int PWS = (mode == 1 && A.Tin) ? 2 : (NM * (mode == 2 ? 2 : 1)) | 1;
+    const int PWS = (NM * (mode == 2 ? 2 : 1)) | 1;
     size_t b = 16 * (size_t)A.maxn * (2 + (mode == 0 ? 0 : 1) + (mode == 2 ? 1 : 0));
     b += 4 * (adj ? 2 : 1) * (size_t)A.maxn + 4 * 16;                              // r, canon (adjoint), seg
     size_t f = (size_t)A.ldg + (mode == 1 ? 3 * (size_t)A.maxn : 0) + (mode == 3 ? 2 * (size_t)A.maxn : 0) +
-               (size_t)pw_floats(mode, A.maxn, PWS, mode == 1 && A.Tin);
+               (size_t)pw_floats(mode, A.maxn, PWS);
     f += (size_t)S * U4 * NM * (mode == 2 ? 2 : 1) + 2 * (size_t)S * U4 + (size_t)NP * U4 * ZP;
     f += (adj && S * NM * U4 > kUbRegs * kWave ? (size_t)S * NM * U4 : 0);         // dE/dT beside the moments
     return b + 4 * f;
@@ -1522,7 +1706,26 @@ static SymmArgs make_args(ann_ctx* ctx) {
     A.geo = ctx->nl.geo;
     A.nsp = ctx->nl.nsp;
     A.nidx = ctx->nl.idx;
+    A.rad_etal = ctx->da.rad_etal;
+    A.rad_gauss = ctx->hm.rad_gauss;
+    A.nrad = ctx->hm.nrad;
+    A.nrs = A.nrad | 1;
+    A.adjK = 1;
     return A;
+}
+
+// Atoms per wavefront of the stored-moment adjoint.  A row of n entries takes
+// ceil(n / 64) passes, two rows together often one less; but two atoms' tables
+// are built one after the other, and half the wavefronts must still fill the
+// chip.  Measured (us, one / two / three atoms): 1,048,576 atoms 3559 / 3150 /
+// 3601, 273,561 atoms 673 / 576 / 649, 12,288 atoms 39.4 / 36.0 / 40.6, 5.5 k
+// 16.4 / 17.2 / 18.2, 2,048 atoms 17.0 / 25.1 / 30.6; argon, 4,096 atoms of 18
+// entries, 14.1 / 12.3 / 13.3 (both rows in one pass).  Three make more lanes
+// of an instruction read different LDS rows.
+static int adj_atoms(const ann_ctx* ctx) {
+    const int64_t N = ctx->natoms;
+    const bool one_pass = 2 * ctx->nl.npairs <= (int64_t)kWave * 7 / 8 * N;
+    return N >= 8192 || (N >= 4096 && one_pass) ? 2 : 1;
 }
 
 static size_t plain_smem(const SymmArgs& A, int mode) {
@@ -1541,6 +1744,25 @@ static size_t fast_smem(const SymmArgs& A, int mode) {
     return b;
 }
 
+using MomentKernel = void (*)(SymmArgs);
+template <int MODE, int Z>
+static MomentKernel pick_kernel(bool queued) {
+    if (queued) return k_moment_queue<MODE, Z>;
+    if constexpr (MODE == 0) return k_moment_g<Z>;
+    else if constexpr (MODE == kModeAdjT) return k_adjoint<Z>;
+    else return k_moment<MODE, Z>;
+}
+template <int MODE>
+static MomentKernel moment_kernel(int z, bool queued) {
+    switch (z) {
+        case 1: return pick_kernel<MODE, 1>(queued);
+        case 2: return pick_kernel<MODE, 2>(queued);
+        case 3: return pick_kernel<MODE, 3>(queued);
+        case 4: return pick_kernel<MODE, 4>(queued);
+        default: return pick_kernel<MODE, 5>(queued);
+    }
+}
+
 template <int MODE>
 static hipError_t run(ann_ctx* ctx, int form, SymmArgs A) {
     if (A.N == 0) return hipSuccess;
@@ -1557,26 +1779,25 @@ static hipError_t run(ann_ctx* ctx, int form, SymmArgs A) {
         const bool tfits = ctx->d_T && ctx->work_atoms >= A.N;
         if (MODE == 0 && tfits) A.Tout = ctx->d_T;
         if (MODE == 1 && tfits && ctx->T_gen == ctx->gen) A.Tin = ctx->d_T;
-        const size_t sw = (moment_smem(A, MODE, M.moment_z, M.S, M.NP) + 15) / 16 * 16;
+        const bool adjT = MODE == 1 && A.Tin;
+        size_t sw = (moment_smem(A, MODE, M.moment_z, M.S, M.NP) + 15) / 16 * 16;
+        if (adjT) {
+            A.adjK = adj_atoms(ctx);
+            while (A.adjK > 1 && adj_units(A.adjK, M.moment_z, M.S, M.NP, A.nrs, A.ldg) > 1024) --A.adjK;   // 16 KiB
+            sw = 16 * (size_t)adj_units(A.adjK, M.moment_z, M.S, M.NP, A.nrs, A.ldg);
+        }
         int apb = ctx->tune_apb[MODE];
         while (apb > 1 && sw * apb > 65536) apb /= 2;          // dynamic LDS of one workgroup
         A.smem_wave = (int)sw;
-        unsigned grid = (unsigned)((A.N + apb - 1) / apb), block = 64u * apb;
+        const int per = apb * (adjT ? A.adjK : 1);             // atoms of one workgroup
+        unsigned grid = (unsigned)((A.N + per - 1) / per), block = 64u * apb;
         const size_t sm = sw * apb;
         const bool queued = ctx->tune_queue == 1;
         if (queued) {
             const hipError_t ei = ensure_items(ctx);
             if (ei != hipSuccess) return ei;
         }
-        void (*kern)(SymmArgs) =
-            queued ? (M.moment_z == 1 ? k_moment_queue<MODE, 1> : M.moment_z == 2 ? k_moment_queue<MODE, 2>
-                      : M.moment_z == 3 ? k_moment_queue<MODE, 3> : M.moment_z == 4 ? k_moment_queue<MODE, 4>
-                      : k_moment_queue<MODE, 5>)
-                   : MODE == 0 ? (M.moment_z == 1 ? k_moment_g<1> : M.moment_z == 2 ? k_moment_g<2>
-                                  : M.moment_z == 3 ? k_moment_g<3> : M.moment_z == 4 ? k_moment_g<4> : k_moment_g<5>)
-                   : (M.moment_z == 1 ? k_moment<MODE, 1> : M.moment_z == 2 ? k_moment<MODE, 2>
-                      : M.moment_z == 3 ? k_moment<MODE, 3> : M.moment_z == 4 ? k_moment<MODE, 4>
-                      : k_moment<MODE, 5>);
+        MomentKernel kern = adjT ? moment_kernel<kModeAdjT>(M.moment_z, queued) : moment_kernel<MODE>(M.moment_z, queued);
         if (queued) {
             // persistent: enough workgroups for the most wavefronts a CU can hold
             // (32); those that find no room start later, find the queues empty
