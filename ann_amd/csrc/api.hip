@@ -520,6 +520,10 @@ extern "C" int ann_create(const ann_model_desc* desc, ann_ctx** out) {
     if (hipGetDevice(&dev) != hipSuccess) return fail(ANN_ERR_HIP, "no HIP device");
     ann_ctx* ctx = new ann_ctx;
     ctx->device = dev;
+    if (hipDeviceGetAttribute(&ctx->num_cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) {
+        delete ctx;
+        return fail(ANN_ERR_HIP, "device attributes");
+    }
     // the allocation-free entry point's scratch address on this device
     const hipError_t es = noalloc_init(dev);
     if (es != hipSuccess) {
@@ -933,7 +937,7 @@ static hipError_t ensure_work(ann_ctx* ctx) {
         if ((e = dalloc(ctx->d_u, 3 * (size_t)N)) != hipSuccess) return e;
         if ((e = dalloc(ctx->d_F, 3 * (size_t)N)) != hipSuccess) return e;
         if ((e = dalloc(ctx->d_atomvir, 9 * (size_t)N)) != hipSuccess) return e;
-        if (ctx->hm.moment_z > 0) {   // moments of the moment form: [N][S][4][harmonics]
+        if (ctx->hm.moment_z > 0) {   // moments of the moment form: [N][S][harmonics][4]
             if ((e = dalloc(ctx->d_T, (size_t)N * ctx->S * kMaxUnionEta * nharm(ctx->hm.moment_z))) != hipSuccess) return e;
         }
         ctx->T_gen = ~0ull;

@@ -363,7 +363,9 @@ __global__ __launch_bounds__(64) void k_precise(PreciseArgs A, int maxn) {
         __syncthreads();
         if (wantT) {
             const int TS = S * 4 * NM;
-            for (int x = lane; x < TS; x += kWave) A.Tout[(size_t)i * TS + x] = (float)T[x];
+            // the FP32 kernels' layout: widths innermost
+            for (int x = lane; x < TS; x += kWave)
+                A.Tout[(size_t)i * TS + x] = (float)T[(x / (4 * NM) * 4 + x % 4) * NM + (x / 4) % NM];
         }
         // A_l(p, u) = sum_m T_b T_c (b != c); (... - D_b) / 2 for b == c
         for (int it = lane; it < NP * 4 * ZP; it += kWave) {

@@ -63,7 +63,8 @@ struct SymmArgs {
     const float* rad_etal;    // rad_eta times sqrt(log2 e)
     int rad_gauss;            // every radial block is GAUSSIAN
     int nrad, nrs;            // widest radial block; its row stride in the adjoint's tables (odd)
-    int adjK;                 // atoms per wavefront of the stored-moment adjoint
+    int grows;                // function rows in LDS of the G kernel
+    int atomsK;               // atoms per wavefront of G and of the stored-moment adjoint
     // fused E+F (mode 3): the network's parameter tables and inputs, the atom energies
     const float* wchunk;      // forward weight rows, biases, output neuron (net_dev.h layout)
     const float* wtrans;      // transposed weight rows (backward)
@@ -893,11 +894,11 @@ __global__ __launch_bounds__(64) void k_fast(SymmArgs A) {
 // 216 us, 512 uneven water cells 4.18 -> 3.94 ms, five MD steps of 1 M atoms
 // 103.0 -> 97.2 ms, 64 water boxes and Li/P/S training unchanged.
 
-// neighbours per chunk of function rows (G: 32 and adjoint: 64, which frees LDS
-// for more resident wavefronts; tangent: every neighbour at once while a row is
-// short, up to degree 2, else 32), and the floats of the region that holds them (it also holds the cutoff pairs, two floats per neighbour, before
-// the rows are needed).  Mode 1 here is the adjoint that recomputes the moments:
-// it serves calls whose geometry no G call has seen
+// moment_atom's chunk of function rows (adjoint: 64, fused: 32; tangent: every
+// neighbour at once while a row is short, up to degree 2, else 32), and the
+// floats of the region that holds them (it also holds the cutoff pairs, two
+// floats per neighbour, before the rows are needed).  Mode 1 here is the adjoint
+// that recomputes the moments: it serves calls whose geometry no G call has seen.
 constexpr int kPwRows = 64;
 // adjoint: dE/dT entries per lane held in registers while they replace the moments
 constexpr int kUbRegs = 8;
@@ -1193,9 +1194,6 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
         }
     }
     wave_sync();
-    if (MODE == 0 && A.Tout) {
-        for (int q = lane; q < TS; q += kWave) A.Tout[(size_t)i * TS + q] = T[q];
-    }
     // block contractions (modes 0, 2, 3) or their adjoint seeds (mode 1; mode 3
     // after its network)
     auto adjoint_seeds = [&]() {
@@ -1386,7 +1384,7 @@ __device__ __forceinline__ void adjoint_wave(const SymmArgs& A, const int i0, co
     float4* W = smem4;                                          // [K][S][NS] dE/dT, widths in the components
     float4* R = W + K * S * NS;                                 // [K][S][nrs] radial: eta, rs, dE/dG, dE/dG eta
     float4* dD = R + K * S * nrs;                               // [K][S] dE/dD
-    float* T = reinterpret_cast<float*>(dD + K * S);            // [K][S][U4][NM]
+    float* T = reinterpret_cast<float*>(dD + K * S);            // [K][S][NM][U4]
     float* row = T + K * S * U4 * NM;                           // [K][ldg]
     float* Am = row + K * ldg;                                  // [K][NP][U4][ZP]
     int o[kAdjAtoms + 1], sp[kAdjAtoms];
@@ -1459,7 +1457,7 @@ __device__ __forceinline__ void adjoint_wave(const SymmArgs& A, const int i0, co
 #pragma unroll
         for (int d = 1; d <= Z; ++d) l += f >= d * d ? 1 : 0;
         const float* Aq = Am + q * NP * U4 * ZP + u * ZP + l;
-        const float* Tq = T + q * S * U4 * NM + u * NM + f;
+        const float* Tq = T + (q * S * NM + f) * U4 + u;
         float v = 0.0f;
         for (int c = 0; c < S; ++c) v += Aq[pair_of(b, c) * U4 * ZP] * Tq[c * U4 * NM];
         reinterpret_cast<float*>(W)[((q * S + b) * NS + f) * U4 + u] = v;
@@ -1540,14 +1538,287 @@ __device__ __forceinline__ void adjoint_wave(const SymmArgs& A, const int i0, co
 }
 
 // Grid dispatch of the stored-moment adjoint: every wavefront of a block takes
-// A.adjK consecutive atoms on its own LDS slice.
+// A.atomsK consecutive atoms on its own LDS slice.
 template <int Z>
 __global__ __launch_bounds__(256) void k_adjoint(SymmArgs A) {
     extern __shared__ float4 smem_all[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int i0 = (xcd_block(blockIdx.x, gridDim.x) * (blockDim.x / kWave) + wave) * A.adjK;
+    const int i0 = (xcd_block(blockIdx.x, gridDim.x) * (blockDim.x / kWave) + wave) * A.atomsK;
     if (i0 >= A.N) return;
-    adjoint_wave<Z>(A, i0, min(A.adjK, A.N - i0), smem_all + (size_t)wave * (A.smem_wave / 16));
+    adjoint_wave<Z>(A, i0, min(A.atomsK, A.N - i0), smem_all + (size_t)wave * (A.smem_wave / 16));
+}
+
+// G in the moment form.  One wavefront serves one atom and walks its list
+// entries 64 at a time: each lane forms its entry's cutoff, width factors and
+// harmonics in registers, and the entries of the pass get LDS places ordered by
+// neighbour species, found with ballots; entries beyond the cutoff (skin lists)
+// get none.  Then lanes over functions sum each species' run: moments
+// T_b[u][f] = sum e_u Y_f with the four widths in registers (lanes NM .. NM + 3
+// read e_u in place of a function, which gives D_b[u] = sum e_u^2), radial
+// functions with lanes over (entry, function).  With up to SR species every sum
+// stays in registers until the row ends (SR = 0: any number, added up in LDS
+// after every run).  LDS holds one pass, not one row per neighbour, so it does not
+// grow with the widest row.
+// Bound by vector issue, about 1,650 wave instructions' worth of time per water
+// atom.  Against the form that regroups the whole row by species in LDS first
+// (one row of 36 bytes per neighbour), us: 1,048,576 atoms with a skin 5119 ->
+// 4037, 273,561 atoms 820 -> 735, 12,288 atoms 47.4 -> 43.8, 87,912 Li/P/S atoms
+// 200 -> 152, 5.5 k 27.0 -> 18.1.  Two atoms per wavefront: 923 on the 273,561
+// atoms, sums added up in LDS after every run: 829.
+constexpr int kGRegSpecies = 3;         // species with their sums in registers
+
+template <int Z>
+struct GShape {
+    static constexpr int NM = nharm(Z), NX = NM + kMaxUnionEta, NR = NX | 1;
+    static constexpr int NW = NX <= 8 ? 8 : (NX <= 16 ? 16 : (NX <= 32 ? 32 : kWave));   // lanes of one group
+    static constexpr int NG = kWave / NW;
+};
+
+// float4 entries of the wavefront's LDS slice (layout at the top of g_atom)
+__host__ inline int g_units(int Z, int S, int NP, int nrad, int ldg, int rows) {
+    const int NM = nharm(Z), NR = (NM + kMaxUnionEta) | 1;
+    return kWave + S * NM + S + kWave / 2 + (S * nrad + 1) / 2 + rows * NR / 4 + ldg / 4 +
+           (NP * kMaxUnionEta * (Z + 1) + 3) / 4;
+}
+
+template <int Z, int SR>
+__device__ __forceinline__ void g_atom(const SymmArgs& A, const int i, float4* smem4) {
+    constexpr int NM = GShape<Z>::NM, NX = GShape<Z>::NX, NR = GShape<Z>::NR, NW = GShape<Z>::NW, NG = GShape<Z>::NG;
+    constexpr int ZP = Z + 1, U4 = kMaxUnionEta, NB = SR > 0 ? SR : 1;
+    const int lane = threadIdx.x % kWave;
+    const DevModel& Mo = *A.dm;
+    const int S = Mo.S, NP = Mo.NP, ldg = A.ldg, nrad = A.nrad;
+    const int nrow = A.grows;                                   // function rows in LDS at a time (a multiple of 4)
+    float4* ef = smem4;                                         // [64] width factors of the pass
+    float4* T = ef + kWave;                                     // [S][NM] moments, widths in the components
+    float4* D = T + S * NM;                                     // [S]
+    float2* rf = reinterpret_cast<float2*>(D + S);              // [64] distance, cutoff
+    float2* par = rf + kWave;                                   // [S][nrad] radial eta, rs
+    float* rows = reinterpret_cast<float*>(par + ((S * nrad + 1) & ~1));   // [nrow][NR] functions, then e_u
+    float* row = rows + nrow * NR;                              // [ldg]
+    float* Am = row + ldg;                                      // [NP][U4][ZP]
+    const int o0 = A.off[i], o1 = A.off[i + 1], a = A.species[i];
+    float4 gn = make_float4(0.f, 0.f, 0.f, 0.f);
+    int bn = 0;
+    if (o0 + lane < o1) {
+        gn = A.geo[o0 + lane];
+        bn = A.nsp[o0 + lane];
+    }
+    if (SR == 0)
+        for (int x = lane; x < S * NM + S; x += kWave) T[x] = make_float4(0.f, 0.f, 0.f, 0.f);   // T and D
+    for (int x = lane; x < ldg; x += kWave) row[x] = 0.0f;
+    for (int x = lane; x < S * nrad; x += kWave) {
+        const int m = x % nrad, b = x / nrad;
+        const RadBlock rb = Mo.rad[a * S + b];
+        float2 t = make_float2(0.f, 0.f);
+        if (m < rb.n) t = make_float2(A.rad_gauss ? A.rad_etal[rb.par + m] : A.rad_eta[rb.par + m], A.rad_rs[rb.par + m]);
+        par[x] = t;
+    }
+    const float rc = Mo.rc;
+    const int al = lane % NW, grp = lane / NW;
+    float mom[NB][U4], rad[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        rad[b] = 0.0f;
+#pragma unroll
+        for (int u = 0; u < U4; ++u) mom[b][u] = 0.0f;
+    }
+    // the groups of lanes meet, then the sums of species b go to LDS (added: SR = 0)
+    auto put_moments = [&](int b, float (&acc)[U4]) {
+#pragma unroll
+        for (int bit = NW; bit < kWave; bit <<= 1)
+#pragma unroll
+            for (int u = 0; u < U4; ++u) acc[u] += __shfl_xor(acc[u], bit);
+        if (lane < NM) {
+            float4 t = SR == 0 ? T[b * NM + lane] : make_float4(0.f, 0.f, 0.f, 0.f);
+            t.x += acc[0]; t.y += acc[1]; t.z += acc[2]; t.w += acc[3];
+            T[b * NM + lane] = t;
+        } else if (lane < NX) {                                 // lane NM + u: sum of e_u e_u
+            const int u = lane - NM;
+            const float v = u == 0 ? acc[0] : (u == 1 ? acc[1] : (u == 2 ? acc[2] : acc[3]));
+            float* d = reinterpret_cast<float*>(D + b) + u;
+            *d = SR == 0 ? *d + v : v;
+        }
+    };
+    auto put_radial = [&](int b, const RadBlock& rb, float acc) {
+        const int W = rb.n <= 8 ? 8 : (rb.n <= 16 ? 16 : 32);
+        for (int bit = W; bit < kWave; bit <<= 1) acc += __shfl_xor(acc, bit);
+        if (lane < rb.n) row[rb.goff + lane] += acc;
+    };
+    for (int base = o0; base < o1; base += kWave) {
+        const int s = base + lane;
+        const float4 gq = gn;
+        const bool keep = s < o1 && gq.w <= rc;
+        const int key = keep ? bn : -1;
+        if (s + kWave < o1) {
+            gn = A.geo[s + kWave];
+            bn = A.nsp[s + kWave];
+        }
+        int pos = 0, cnt = 0;
+        for (int b = 0; b < S; ++b) {
+            const uint64_t m = __ballot(key == b);
+            if (key == b) pos = cnt + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
+            cnt += __popcll(m);
+        }
+        float y[NM], e[U4];
+        wave_sync();                                            // the previous pass's LDS reads are done
+        if (keep) {
+            const float r = gq.w, ir = __builtin_amdgcn_rcpf(r);   // 1 ulp
+            float C[ZP], Sn[ZP], ql[qidx(Z, Z) + 1];
+            harm_factors<Z, float>(gq.x * ir, gq.y * ir, gq.z * ir, C, Sn, ql);
+            harm_values<Z, float>(C, Sn, ql, y);
+            float fc, gc;
+            cutoff_fg(Mo.cutoff, Mo.rc, Mo.rci, Mo.pirc, r, fc, gc);
+#pragma unroll
+            for (int u = 0; u < U4; ++u) e[u] = u < Mo.nunion[a] ? __expf(-Mo.uieta2[a][u] * r * r) * fc : 0.0f;
+            ef[pos] = make_float4(e[0], e[1], e[2], e[3]);
+            rf[pos] = make_float2(r, fc);
+        }
+        // moments: rows of up to nrow entries at a time
+        for (int c0 = 0; c0 < cnt; c0 += nrow) {
+            if (c0 > 0) wave_sync();                            // the previous rows are read
+            if (keep && pos >= c0 && pos < c0 + nrow) {
+                float* w = rows + (pos - c0) * NR;
+#pragma unroll
+                for (int f = 0; f < NM; ++f) w[f] = y[f];
+#pragma unroll
+                for (int u = 0; u < U4; ++u) w[NM + u] = e[u];
+            }
+            wave_sync();
+            auto run = [&](int j0, int j1, float (&acc)[U4]) {
+                auto step = [&](const float* w, int J) {
+                    const float v = w[al];
+                    const float4 e4 = ef[J];
+                    acc[0] += e4.x * v; acc[1] += e4.y * v; acc[2] += e4.z * v; acc[3] += e4.w * v;
+                };
+                if (al < NX) {
+                    int J = j0 + grp;
+                    // four entries per trip: rows at fixed offsets from one address
+                    for (; J + 3 * NG < j1; J += 4 * NG) {
+                        const float* w = rows + (J - c0) * NR;
+                        step(w, J);
+                        step(w + NG * NR, J + NG);
+                        step(w + 2 * NG * NR, J + 2 * NG);
+                        step(w + 3 * NG * NR, J + 3 * NG);
+                    }
+                    for (; J < j1; J += NG) step(rows + (J - c0) * NR, J);
+                }
+            };
+            int s0 = 0;
+            if constexpr (SR > 0) {
+#pragma unroll
+                for (int b = 0; b < SR; ++b) {
+                    const int n = __popcll(__ballot(key == b));
+                    run(max(s0, c0), min(s0 + n, c0 + nrow), mom[b]);
+                    s0 += n;
+                }
+            } else {
+                for (int b = 0; b < S; ++b) {
+                    const int n = __popcll(__ballot(key == b));
+                    const int j0 = max(s0, c0), j1 = min(s0 + n, c0 + nrow);
+                    s0 += n;
+                    if (j0 >= j1) continue;
+                    float acc[U4] = {0.f, 0.f, 0.f, 0.f};
+                    run(j0, j1, acc);
+                    put_moments(b, acc);
+                }
+            }
+        }
+        // radial: lanes over (entry, function) of every species' run
+        auto radial = [&](int b, const RadBlock& rb, int j0, int j1) {
+            const int sh = rb.n <= 8 ? 3 : (rb.n <= 16 ? 4 : 5), nj = kWave >> sh;
+            const int m = lane & ((1 << sh) - 1);
+            const float2 t = m < rb.n ? par[b * nrad + m] : make_float2(0.f, 0.f);
+            float acc = 0.0f;
+            if (A.rad_gauss) {
+#pragma unroll 4
+                for (int J = j0 + (lane >> sh); J < j1; J += nj) {
+                    const float2 v = rf[J];
+                    const float x = t.x * (v.x - t.y);
+                    acc += __builtin_amdgcn_exp2f(-(x * x)) * v.y;
+                }
+            } else {
+                for (int J = j0 + (lane >> sh); J < j1; J += nj) {
+                    const float2 v = rf[J];
+                    float g, d;
+                    radial_fd(rb.name, t.x, t.y, v.x, v.y, 0.0f, g, d);
+                    acc += g;
+                }
+            }
+            return acc;
+        };
+        int s0 = 0;
+        if constexpr (SR > 0) {
+#pragma unroll
+            for (int b = 0; b < SR; ++b) {
+                const int n = __popcll(__ballot(key == b));
+                if (n > 0) rad[b] += radial(b, Mo.rad[a * S + b], s0, s0 + n);
+                s0 += n;
+            }
+        } else {
+            for (int b = 0; b < S; ++b) {
+                const int n = __popcll(__ballot(key == b));
+                const RadBlock rb = Mo.rad[a * S + b];
+                if (n > 0 && rb.n > 0) put_radial(b, rb, radial(b, rb, s0, s0 + n));
+                s0 += n;
+            }
+        }
+    }
+    wave_sync();
+    if constexpr (SR > 0) {
+#pragma unroll
+        for (int b = 0; b < SR; ++b)
+            if (b < S) {
+                put_moments(b, mom[b]);
+                put_radial(b, Mo.rad[a * S + b], rad[b]);
+            }
+        wave_sync();
+    }
+    if (A.Tout) {
+        float4* out = reinterpret_cast<float4*>(A.Tout) + (size_t)i * S * NM;
+        for (int x = lane; x < S * NM; x += kWave) out[x] = T[x];
+    }
+    // block contractions: lanes over (pair, width, degree); a degree has 2m + 1
+    // functions, every lane runs the length of the highest with the surplus terms
+    // weighted 0, so that the loads issue together
+    for (int x = lane; x < NP * U4 * ZP; x += kWave) {
+        const int m = x % ZP, u = (x / ZP) % U4, p = x / (ZP * U4);
+        int c = 0;
+        while ((c + 1) * (c + 2) / 2 <= p) ++c;
+        const int b = p - c * (c + 1) / 2;
+        const float* Tb = reinterpret_cast<const float*>(T + b * NM) + u;
+        const float* Tc = reinterpret_cast<const float*>(T + c * NM) + u;
+        float v = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 2 * Z + 1; ++j) {
+            const int f = min(m * m + j, NM - 1);
+            const float w = j <= 2 * m ? 1.0f : 0.0f;
+            v += (w * Tb[U4 * f]) * Tc[U4 * f];
+        }
+        if (b == c) v = 0.5f * (v - reinterpret_cast<const float*>(D + b)[u]);
+        Am[x] = v;
+    }
+    wave_sync();
+    // outputs: lanes over (pair, width, combination), loads before the guards that use them
+    for (int x = lane; x < NP * kGridG * kGridK; x += kWave) {
+        const int k = x % kGridK, g = (x / kGridK) % kGridG, p = x / (kGridK * kGridG);
+        const AngBlock& B = Mo.ang[a * NP + p];
+        const int nk = min(max(B.nk, 0), kGridK), goff = B.goff;
+        const bool use = B.n > 0 && g < B.ng && k < nk;
+        const int om = B.outm[g * nk + k];                      // < kGridG * kGridK; used only when use
+        float lc[ZP];
+#pragma unroll
+        for (int l = 0; l < ZP; ++l) lc[l] = B.lcoef[k][l];
+        if (use) {
+            const float* Aq = Am + (p * U4 + g) * ZP;
+            float v = 0.0f;
+#pragma unroll
+            for (int l = 0; l < ZP; ++l) v += lc[l] * Aq[l];
+            row[goff + om] = v;
+        }
+    }
+    wave_sync();
+    for (int x = lane; x < ldg; x += kWave) A.G[(size_t)i * ldg + x] = row[x];
 }
 
 // Grid dispatch: a block holds blockDim.x / 64 atoms (the "atoms per
@@ -1561,15 +1832,14 @@ __global__ __launch_bounds__(256) void k_moment(SymmArgs A) {
     moment_atom<MODE, Z>(A, i, smem_all + (size_t)wave * (A.smem_wave / 16));
 }
 
-// G: the same with registers held to five wavefronts per SIMD (it fits in 96
-// VGPRs without spilling; its LDS per wavefront allows as many)
-template <int Z>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_moment_g(SymmArgs A) {
+// G: one atom per wavefront
+template <int Z, int SR>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_moment_g(SymmArgs A) {
     extern __shared__ float4 smem_all[];
-    const int wave = threadIdx.x / kWave;
-    const int i = blockIdx.x * (blockDim.x / kWave) + wave;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const int i = xcd_block(blockIdx.x, gridDim.x) * (blockDim.x / kWave) + wave;
     if (i >= A.N) return;
-    moment_atom<0, Z>(A, i, smem_all + (size_t)wave * (A.smem_wave / 16));
+    g_atom<Z, SR>(A, i, smem_all + (size_t)wave * (A.smem_wave / 16));
 }
 
 constexpr int kModeAdjT = 4;                                    // the stored-moment adjoint (adjoint_wave)
@@ -1579,7 +1849,7 @@ constexpr int kModeAdjT = 4;                                    // the stored-mo
 // wavefront pulls (first atom, count) items off the queue of its XCD (blocks
 // go to XCD blockIdx.x % 8) until the queue is empty; the items of a batch
 // run largest structure first.
-template <int MODE, int Z>
+template <int MODE, int Z, int SR = 0>
 __global__ __launch_bounds__(256) void k_moment_queue(SymmArgs A) {
     extern __shared__ float4 smem_all[];
     const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
@@ -1596,10 +1866,11 @@ __global__ __launch_bounds__(256) void k_moment_queue(SymmArgs A) {
         int nk = 0;
         if (lane == 0) nk = atomicAdd(ctr, 1);
         const int2 it = A.items[beg + k];
-        if constexpr (MODE == kModeAdjT) {
+        if constexpr (MODE == kModeAdjT || MODE == 0) {
             const int ib = __builtin_amdgcn_readfirstlane(it.x), ie = ib + __builtin_amdgcn_readfirstlane(it.y);
-            for (int a = ib; a < ie; a += A.adjK) {
-                adjoint_wave<Z>(A, a, min(A.adjK, ie - a), smem4);
+            for (int a = ib; a < ie; a += A.atomsK) {
+                if constexpr (MODE == 0) g_atom<Z, SR>(A, a, smem4);
+                else adjoint_wave<Z>(A, a, min(A.atomsK, ie - a), smem4);
                 wave_sync();                                    // the next atoms reuse the LDS slice
             }
         } else {
@@ -1642,10 +1913,6 @@ hipError_t build_items(ann_ctx* ctx) {
     if (!ctx->d_queue) {
         if ((e = hipMalloc(&ctx->d_queue, sizeof(int) * 32 * kXcds)) != hipSuccess) return e;
         if ((e = hipMalloc(&ctx->d_qoff, sizeof(int) * (kXcds + 1))) != hipSuccess) return e;
-        int dev = 0;
-        if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
-        if ((e = hipDeviceGetAttribute(&ctx->num_cu, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess)
-            return e;
     }
     const int resident = std::max(1, ctx->num_cu) * 32;            // wavefronts per CU the kernels can hold
     const int len = std::max(1, std::min(kItemAtoms, ctx->atom_off[S] / (4 * resident)));
@@ -1710,7 +1977,7 @@ static SymmArgs make_args(ann_ctx* ctx) {
     A.rad_gauss = ctx->hm.rad_gauss;
     A.nrad = ctx->hm.nrad;
     A.nrs = A.nrad | 1;
-    A.adjK = 1;
+    A.atomsK = 1;
     return A;
 }
 
@@ -1746,20 +2013,23 @@ static size_t fast_smem(const SymmArgs& A, int mode) {
 
 using MomentKernel = void (*)(SymmArgs);
 template <int MODE, int Z>
-static MomentKernel pick_kernel(bool queued) {
+static MomentKernel pick_kernel(bool queued, int S) {
+    if constexpr (MODE == 0) {
+        if (S <= kGRegSpecies) return queued ? k_moment_queue<0, Z, kGRegSpecies> : k_moment_g<Z, kGRegSpecies>;
+        return queued ? k_moment_queue<0, Z> : k_moment_g<Z, 0>;
+    }
     if (queued) return k_moment_queue<MODE, Z>;
-    if constexpr (MODE == 0) return k_moment_g<Z>;
-    else if constexpr (MODE == kModeAdjT) return k_adjoint<Z>;
+    if constexpr (MODE == kModeAdjT) return k_adjoint<Z>;
     else return k_moment<MODE, Z>;
 }
 template <int MODE>
-static MomentKernel moment_kernel(int z, bool queued) {
+static MomentKernel moment_kernel(int z, bool queued, int S) {
     switch (z) {
-        case 1: return pick_kernel<MODE, 1>(queued);
-        case 2: return pick_kernel<MODE, 2>(queued);
-        case 3: return pick_kernel<MODE, 3>(queued);
-        case 4: return pick_kernel<MODE, 4>(queued);
-        default: return pick_kernel<MODE, 5>(queued);
+        case 1: return pick_kernel<MODE, 1>(queued, S);
+        case 2: return pick_kernel<MODE, 2>(queued, S);
+        case 3: return pick_kernel<MODE, 3>(queued, S);
+        case 4: return pick_kernel<MODE, 4>(queued, S);
+        default: return pick_kernel<MODE, 5>(queued, S);
     }
 }
 
@@ -1781,15 +2051,27 @@ static hipError_t run(ann_ctx* ctx, int form, SymmArgs A) {
         if (MODE == 1 && tfits && ctx->T_gen == ctx->gen) A.Tin = ctx->d_T;
         const bool adjT = MODE == 1 && A.Tin;
         size_t sw = (moment_smem(A, MODE, M.moment_z, M.S, M.NP) + 15) / 16 * 16;
-        if (adjT) {
-            A.adjK = adj_atoms(ctx);
-            while (A.adjK > 1 && adj_units(A.adjK, M.moment_z, M.S, M.NP, A.nrs, A.ldg) > 1024) --A.adjK;   // 16 KiB
-            sw = 16 * (size_t)adj_units(A.adjK, M.moment_z, M.S, M.NP, A.nrs, A.ldg);
+        if (adjT || MODE == 0) {
+            auto units = [&](int K) {
+                return MODE == 0 ? g_units(M.moment_z, M.S, M.NP, A.nrad, A.ldg, A.grows)
+                                 : adj_units(K, M.moment_z, M.S, M.NP, A.nrs, A.ldg);
+            };
+            A.atomsK = MODE == 0 ? 1 : adj_atoms(ctx);
+            // a pass's 64 rows at once where rows are short (degree <= 2) or where the
+            // chip holds every wavefront's slice all the same, else 32 (measured, 32 / 64
+            // rows: 273,561 water atoms 735 / 1010 us, 12,288 43.8 / 53.3, 2,048 20.0 / 18.7,
+            // 87,912 Li/P/S atoms of degree 2 157 / 152)
+            A.grows = kWave;
+            if (MODE == 0 && M.moment_z > 2 &&
+                (int64_t)A.N > (int64_t)ctx->num_cu * ((160 << 10) / (16 * g_units(M.moment_z, M.S, M.NP, A.nrad, A.ldg, kWave))))
+                A.grows = kWave / 2;
+            if (units(A.atomsK) > 1024) A.atomsK = 1;           // above 16 KiB one atom per wavefront
+            sw = 16 * (size_t)units(A.atomsK);
         }
         int apb = ctx->tune_apb[MODE];
         while (apb > 1 && sw * apb > 65536) apb /= 2;          // dynamic LDS of one workgroup
         A.smem_wave = (int)sw;
-        const int per = apb * (adjT ? A.adjK : 1);             // atoms of one workgroup
+        const int per = apb * A.atomsK;                          // atoms of one workgroup
         unsigned grid = (unsigned)((A.N + per - 1) / per), block = 64u * apb;
         const size_t sm = sw * apb;
         const bool queued = ctx->tune_queue == 1;
@@ -1797,7 +2079,8 @@ static hipError_t run(ann_ctx* ctx, int form, SymmArgs A) {
             const hipError_t ei = ensure_items(ctx);
             if (ei != hipSuccess) return ei;
         }
-        MomentKernel kern = adjT ? moment_kernel<kModeAdjT>(M.moment_z, queued) : moment_kernel<MODE>(M.moment_z, queued);
+        MomentKernel kern = adjT ? moment_kernel<kModeAdjT>(M.moment_z, queued, M.S)
+                                 : moment_kernel<MODE>(M.moment_z, queued, M.S);
         if (queued) {
             // persistent: enough workgroups for the most wavefronts a CU can hold
             // (32); those that find no room start later, find the queues empty
