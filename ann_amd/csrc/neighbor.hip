@@ -13,9 +13,9 @@
 // k_a = ceil(rc nb_a / w_a); a wavefront per centre atom walks the flattened
 // candidate set of its search box (lanes over candidates, not over bins),
 // applies the exact FP64 inclusion test in the same operation order as the
-// oracle, compacts accepted keys (j << 30 | packed n) through a ballot into
-// LDS and sorts them (ranks in the staged search, a bitonic network in the
-// wide one).  Integer work; the roofline is
+// oracle and compacts accepted keys (j << 30 | packed n) through a ballot; the
+// staged search meets its candidates in the list's order, the wide one sorts
+// every row with a bitonic network.  Integer work; the roofline is
 // HBM/latency (positions in, 16 B + 13 B per pair out).
 #include <atomic>
 #include <chrono>
@@ -209,47 +209,38 @@ __global__ __launch_bounds__(64) void k_search(
     if (lane == 0) { cnt_out[i] = n; atomicMax(flag + 1, count); }
 }
 
-// Staged search, one block per bin: the candidates of the bin's search box
-// (every atom of the (2k+1)^3 bin images with its image offset) are copied
-// to LDS with one 32-byte load each; each wavefront then tests one centre
-// atom of the bin against them, compacts the accepted keys (j << 30 | packed
-// image) into its own LDS buffer and stores them sorted by rank (no block
-// barriers after the staging).  Bins
-// whose search box holds more than kStageCap candidates or kStageImages
-// images are flagged and left to k_search.  Each block writes the overflow
-// mark (0 or 1) of each of its centre bins exactly once per build, so the
-// marks need no clearing between builds.
+// Staged search, one block per bin or super-bin: the candidates of the search
+// box (every atom of the (2k+1)^3 bin images with its image offset) are copied to
+// LDS with one 32-byte load each, in the list's canonical order (atom index, then
+// image), and each wavefront then tests one centre atom against all of them: the
+// accepted keys (j << 30 | packed image) leave the ballots in order and go
+// straight to the centre's row.  One sort of the box replaces a sort of every row,
+// which was two thirds of the instructions per centre.
+// The sort is a counting sort by bucket of the atom index (one atom per bucket up
+// to kBuckets atoms in the box's index range, else 2^sh neighbouring indices), then
+// each candidate's rank among its bucket's few members; a block that meets a wide
+// index range still sorts, with longer buckets.
+// Boxes with more than kStageCap candidates or kStageImages images are flagged and
+// left to k_search.  Each block writes the overflow mark (0 or 1) of each of its
+// centre bins exactly once per build, so the marks need no clearing between builds.
+// Bound by vector issue: about 25 instructions per 64 candidates and centre, and
+// the staging.  Against one sort per row, us: 1,048,576 atoms (rc 6.5, super-bins
+// now within the capacity) 5767 -> 1579, 273,561 atoms 621 -> 263, 87,912 Li/P/S
+// atoms 213 -> 148, 12,288 atoms 39.5 -> 26.3, 192 atoms 28.6 -> 11.7.
 constexpr int kStageCap = 1280;
 constexpr int kStageImages = 216;
 constexpr int kStageThreads = 512;
-constexpr int kWaveKeys = 256;          // accepted keys per centre in the staged search (more: wide path)
-static_assert(kWaveKeys == 4 * kWave, "the staged sort covers up to four keys per lane");
+constexpr int kBuckets = 1024;
 constexpr int kStageWaves = kStageThreads / kWave;
 constexpr int kStageIt = (kStageCap + kStageThreads - 1) / kStageThreads;
+static_assert(kBuckets == 2 * kStageThreads, "the bucket scan gives every thread two buckets");
 
-// Sorted store of n distinct keys by rank: every lane counts, for the up to R
-// keys it holds, the keys below them (broadcast LDS reads, no dependency
-// between iterations), and writes each key at its rank.
-template <int R>
-__device__ __forceinline__ void rank_and_store(const uint64_t* buf, int n, uint64_t* dst) {
-    const int lane = threadIdx.x % kWave;
-    uint64_t v[R];
-    int rk[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const int e = lane + kWave * r;
-        v[r] = e < n ? buf[e] : ~0ull;
-        rk[r] = 0;
-    }
-#pragma unroll 4
-    for (int m = 0; m < n; ++m) {
-        const uint64_t w = buf[m];
-#pragma unroll
-        for (int r = 0; r < R; ++r) rk[r] += w < v[r] ? 1 : 0;
-    }
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-        if (lane + kWave * r < n) dst[rk[r]] = v[r];
+// the image and wrapped index of unwrapped bin u (|u| is a few cells at most)
+__device__ __forceinline__ int wrap_bin(int u, int nb, int& m) {
+    m = 0;
+    while (u < 0) { u += nb; --m; }
+    while (u >= nb) { u -= nb; ++m; }
+    return u;
 }
 
 __global__ __launch_bounds__(kStageThreads) void k_search_bins(
@@ -259,12 +250,14 @@ __global__ __launch_bounds__(kStageThreads) void k_search_bins(
     __shared__ int im_first[kStageImages];
     __shared__ int im_m[kStageImages];
     __shared__ int im_pre[kStageImages + 1];
-    __shared__ float4 cf[kStageCap];                        // FP32 image position x_j + R (m - shift_j)
-    __shared__ uint64_t cjd[kStageCap];                     // j << 32 | packed (image - shift_j)
-    __shared__ uint64_t wkeys[kStageWaves][kWaveKeys];
-    __shared__ int cen_bin[8], cen_pre[9], cen_img[8];
-    __shared__ int s_ovf[8];                                // centre bins left to the wide search
-    __shared__ int s_total, s_max, s_xmax;
+    __shared__ signed char im_cen[kStageImages];            // centre bin of the image, or -1
+    __shared__ float4 cf[kStageCap];                        // FP32 image position x_j + R (m - shift_j), sorted
+    __shared__ uint64_t ckey[kStageCap];                    // j << 30 | packed (image - shift_j), sorted
+    __shared__ int bucket[kBuckets + 1];
+    __shared__ uint16_t cen_rank[kStageCap];                // sorted place of each centre
+    __shared__ int cen_bin[8], cen_pre[9], wsum[kStageWaves];
+    __shared__ int s_total, s_max, s_xmax, s_jmin, s_jmax;
+    uint64_t* sk = reinterpret_cast<uint64_t*>(cf);         // (j << 32 | image number) by bucket, until the ranks are known
     const int g = xcd_block(blockIdx.x, gridDim.x), t = threadIdx.x;
     const int lane = t % kWave, wave = t / kWave;
     const int s = bin_struc[g];                             // structure of this super-bin
@@ -274,42 +267,53 @@ __global__ __launch_bounds__(kStageThreads) void k_search_bins(
     const int B0 = gi / (c.nsb[1] * c.nsb[2]), B1 = (gi / c.nsb[2]) % c.nsb[1], B2 = gi % c.nsb[2];
     const int lo0 = c.sb * B0, lo1 = c.sb * B1, lo2 = c.sb * B2;
     const int n0b = min(c.sb, c.nb[0] - lo0), n1b = min(c.sb, c.nb[1] - lo1), n2b = min(c.sb, c.nb[2] - lo2);
-    // centre bins of the super-bin and their atom ranges
-    if (t == 0) {
-        int acc = 0, q = 0;
-        for (int d0 = 0; d0 < n0b; ++d0)
-            for (int d1 = 0; d1 < n1b; ++d1)
-                for (int d2 = 0; d2 < n2b; ++d2, ++q) {
-                    const int bg = c.boff + ((lo0 + d0) * c.nb[1] + (lo1 + d1)) * c.nb[2] + (lo2 + d2);
-                    cen_bin[q] = bg;
-                    cen_pre[q] = acc;
-                    cen_img[q] = ((c.k[0] + d0) * (n1b + 2 * c.k[1]) + (c.k[1] + d1)) * (n2b + 2 * c.k[2]) + (c.k[2] + d2);
-                    acc += bin_start[bg + 1] - bin_start[bg];
-                }
-        cen_pre[q] = acc;
-        s_max = 0;
-        s_xmax = 0;
-    }
-    if (t < 8) s_ovf[t] = 0;
     const int ncb = n0b * n1b * n2b;
     const int e0 = n0b + 2 * c.k[0], e1 = n1b + 2 * c.k[1], e2 = n2b + 2 * c.k[2];
     const int nimg = e0 * e1 * e2;
+    for (int q = t; q <= kBuckets; q += kStageThreads) bucket[q] = 0;
+    if (wave == kStageWaves - 1) {
+        // centre bins of the super-bin and their atom ranges (at most eight)
+        int n = 0;
+        if (lane < ncb) {
+            const int d0 = lane / (n1b * n2b), d1 = (lane / n2b) % n1b, d2 = lane % n2b;
+            const int bg = c.boff + ((lo0 + d0) * c.nb[1] + (lo1 + d1)) * c.nb[2] + (lo2 + d2);
+            cen_bin[lane] = bg;
+            n = bin_start[bg + 1] - bin_start[bg];
+        }
+        int inc = n;
+#pragma unroll
+        for (int o = 1; o < 8; o <<= 1) {
+            const int u = __shfl_up(inc, o);
+            if (lane >= o) inc += u;
+        }
+        if (lane < ncb) cen_pre[lane + 1] = inc;
+        if (lane == 0) {
+            cen_pre[0] = 0;
+            s_max = 0;
+            s_xmax = 0;
+            s_jmin = INT32_MAX;
+            s_jmax = -1;
+        }
+    }
     if (nimg > kStageImages) {
         __syncthreads();
         if (t < ncb) bin_ovf[cen_bin[t]] = 1;
         if (t == 0) atomicOr(flag, 8);
         return;
     }
-    for (int q = t; q < nimg; q += kStageThreads) {
-        const int u0 = lo0 - c.k[0] + q / (e1 * e2);
-        const int u1 = lo1 - c.k[1] + (q / e2) % e1;
-        const int u2 = lo2 - c.k[2] + q % e2;
-        const int m0 = floordiv(u0, c.nb[0]), m1 = floordiv(u1, c.nb[1]), m2 = floordiv(u2, c.nb[2]);
-        const int gg = c.boff + ((u0 - m0 * c.nb[0]) * c.nb[1] + (u1 - m1 * c.nb[1])) * c.nb[2] + (u2 - m2 * c.nb[2]);
+    if (t < nimg) {
+        const int x0 = t / (e1 * e2), x1 = (t / e2) % e1, x2 = t % e2;
+        int m0, m1, m2;
+        const int w0 = wrap_bin(lo0 - c.k[0] + x0, c.nb[0], m0), w1 = wrap_bin(lo1 - c.k[1] + x1, c.nb[1], m1),
+                  w2 = wrap_bin(lo2 - c.k[2] + x2, c.nb[2], m2);
+        const int gg = c.boff + (w0 * c.nb[1] + w1) * c.nb[2] + w2;
         const int f = bin_start[gg];
-        im_first[q] = f;
-        im_m[q] = (int)pack_img(m0, m1, m2);
-        im_pre[q + 1] = bin_start[gg + 1] - f;
+        im_first[t] = f;
+        im_m[t] = (int)pack_img(m0, m1, m2);
+        im_pre[t + 1] = bin_start[gg + 1] - f;
+        const int d0 = x0 - c.k[0], d1 = x1 - c.k[1], d2 = x2 - c.k[2];
+        const bool in = d0 >= 0 && d0 < n0b && d1 >= 0 && d1 < n1b && d2 >= 0 && d2 < n2b;
+        im_cen[t] = (signed char)(in ? (d0 * n1b + d1) * n2b + d2 : -1);
     }
     __syncthreads();
     if (t < kWave) {   // inclusive scan of the image counts by the first wavefront
@@ -341,11 +345,12 @@ __global__ __launch_bounds__(kStageThreads) void k_search_bins(
     }
     {
         // every thread resolves all its candidates first, then issues their loads together
-        int src[kStageIt], mq[kStageIt];
+        int src[kStageIt], iq[kStageIt];
 #pragma unroll
         for (int r = 0; r < kStageIt; ++r) {
             const int q = t + r * kStageThreads;
             src[r] = -1;
+            iq[r] = 0;
             if (q < total) {
                 int lo = 0, hi = nimg;
                 while (hi - lo > 1) {
@@ -353,32 +358,107 @@ __global__ __launch_bounds__(kStageThreads) void k_search_bins(
                     if (im_pre[mid] <= q) lo = mid; else hi = mid;
                 }
                 src[r] = im_first[lo] + (q - im_pre[lo]);
-                mq[r] = im_m[lo];
+                iq[r] = lo;
             }
         }
         double4 r4[kStageIt];
 #pragma unroll
         for (int r = 0; r < kStageIt; ++r)
             if (src[r] >= 0) r4[r] = rec[src[r]];
-        float xm = 0.0f;
+        float x[kStageIt], y[kStageIt], z[kStageIt], xm = 0.0f;
+        uint64_t jd[kStageIt];
+        int jlo = INT32_MAX, jhi = -1;
 #pragma unroll
         for (int r = 0; r < kStageIt; ++r) {
-            const int q = t + r * kStageThreads;
             if (src[r] < 0) continue;
             const uint64_t js = (uint64_t)__double_as_longlong(r4[r].w);
             int m0, m1, m2, s0, s1, s2;
-            unpack_img((uint32_t)mq[r], m0, m1, m2);
+            unpack_img((uint32_t)im_m[iq[r]], m0, m1, m2);
             unpack_img((uint32_t)(js & 0xffffffffu), s0, s1, s2);
             const double d0 = m0 - s0, d1 = m1 - s1, d2 = m2 - s2;
-            const float x = (float)(r4[r].x + (R[0] * d0 + R[1] * d1 + R[2] * d2));
-            const float y = (float)(r4[r].y + (R[3] * d0 + R[4] * d1 + R[5] * d2));
-            const float z = (float)(r4[r].z + (R[6] * d0 + R[7] * d1 + R[8] * d2));
-            cf[q] = make_float4(x, y, z, 0.0f);
-            xm = fmaxf(xm, fmaxf(fabsf(x), fmaxf(fabsf(y), fabsf(z))));
-            cjd[q] = (js & 0xffffffff00000000ull) | (uint64_t)pack_img(m0 - s0, m1 - s1, m2 - s2);
+            x[r] = (float)(r4[r].x + (R[0] * d0 + R[1] * d1 + R[2] * d2));
+            y[r] = (float)(r4[r].y + (R[3] * d0 + R[4] * d1 + R[5] * d2));
+            z[r] = (float)(r4[r].z + (R[6] * d0 + R[7] * d1 + R[8] * d2));
+            xm = fmaxf(xm, fmaxf(fabsf(x[r]), fmaxf(fabsf(y[r]), fabsf(z[r]))));
+            jd[r] = (js & 0xffffffff00000000ull) | (uint64_t)pack_img(m0 - s0, m1 - s1, m2 - s2);
+            const int j = (int)(js >> 32);
+            jlo = min(jlo, j);
+            jhi = max(jhi, j);
         }
-        atomicMax(&s_xmax, __float_as_int(xm));             // non-negative floats order as integers
+        int xi = __float_as_int(xm);                        // non-negative floats order as integers
+#pragma unroll
+        for (int o = kWave / 2; o > 0; o >>= 1) {
+            xi = max(xi, __shfl_xor(xi, o));
+            jlo = min(jlo, __shfl_xor(jlo, o));
+            jhi = max(jhi, __shfl_xor(jhi, o));
+        }
+        if (lane == 0) {
+            atomicMax(&s_xmax, xi);
+            atomicMin(&s_jmin, jlo);
+            atomicMax(&s_jmax, jhi);
+        }
+        __syncthreads();
+        // buckets of 2^sh atom indices
+        const int jmin = s_jmin, range = s_jmax - jmin;
+        int sh = 0;
+        while ((range >> sh) >= kBuckets) ++sh;
+        int bk[kStageIt], slot[kStageIt];
+#pragma unroll
+        for (int r = 0; r < kStageIt; ++r) {
+            bk[r] = 0;
+            slot[r] = 0;
+            if (src[r] < 0) continue;
+            bk[r] = ((int)(jd[r] >> 32) - jmin) >> sh;
+            slot[r] = atomicAdd(&bucket[bk[r]], 1);
+        }
+        __syncthreads();
+        {
+            const int v0 = bucket[2 * t], v1 = bucket[2 * t + 1];
+            int inc = v0 + v1;
+#pragma unroll
+            for (int o = 1; o < kWave; o <<= 1) {
+                const int u = __shfl_up(inc, o);
+                if (lane >= o) inc += u;
+            }
+            if (lane == kWave - 1) wsum[wave] = inc;
+            __syncthreads();
+            int before = inc - v0 - v1;
+#pragma unroll
+            for (int w = 0; w < kStageWaves; ++w) before += w < wave ? wsum[w] : 0;
+            bucket[2 * t] = before;
+            bucket[2 * t + 1] = before + v0;
+            if (t == 0) bucket[kBuckets] = total;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kStageIt; ++r)
+            if (src[r] >= 0) sk[bucket[bk[r]] + slot[r]] = (jd[r] & 0xffffffff00000000ull) | (uint64_t)iq[r];
+        __syncthreads();
+        int rank[kStageIt];
+#pragma unroll
+        for (int r = 0; r < kStageIt; ++r) {
+            rank[r] = 0;
+            if (src[r] < 0) continue;
+            const int b0 = bucket[bk[r]], b1 = bucket[bk[r] + 1];
+            const uint64_t me = (jd[r] & 0xffffffff00000000ull) | (uint64_t)iq[r];
+            rank[r] = b0;
+            for (int k = b0; k < b1; ++k) rank[r] += sk[k] < me ? 1 : 0;
+        }
+        __syncthreads();                                    // cf takes the place of sk
+#pragma unroll
+        for (int r = 0; r < kStageIt; ++r) {
+            if (src[r] < 0) continue;
+            cf[rank[r]] = make_float4(x[r], y[r], z[r], 0.0f);
+            ckey[rank[r]] = ((jd[r] >> 32) << 30) | (jd[r] & 0x3fffffffu);
+            const int cb = im_cen[iq[r]];
+            // a centre is the zero image of its own bin, where (image - shift) = -shift
+            if (cb >= 0) cen_rank[cen_pre[cb] + (t + r * kStageThreads - im_pre[iq[r]])] = (uint16_t)rank[r];
+        }
     }
+    // the last chunk of 64 is filled up with NaN places: no comparison accepts their
+    // distance, also where a non-finite position has made the band infinite
+    if (t < kWave && t >= (total & (kWave - 1)) && (total & (kWave - 1)))
+        cf[total / kWave * kWave + t] = make_float4(__int_as_float(0x7fc00000), 0.f, 0.f, 0.f);
     __syncthreads();
     // FP32 pre-test.  With u = 2^-24 and every FP32 coordinate within
     // X = max |x| of its FP64 value to u X, the FP32 squared distance of a
@@ -390,77 +470,51 @@ __global__ __launch_bounds__(kStageThreads) void k_search_bins(
     const double D = 2.0 * uu * (double)__int_as_float(s_xmax) + 1.2 * uu * rc;
     const float band = (float)(4.0 * (3.4641016151377544 * rc * D + 3.0 * D * D + 4.0 * uu * rc2) + 2.0 * uu * rc2);
     const float rc2f = (float)rc2, lo_thr = rc2f - band, hi_thr = rc2f + band;
-    uint64_t* wk = wkeys[wave];
     int wmax = 0;          // largest neighbour count of this wavefront's centres
     for (int cq = wave; cq < ncen; cq += kStageWaves) {
-        int cb = 0;
-        while (cb + 1 < ncb && cq >= cen_pre[cb + 1]) ++cb;
-        // the centre is staged too: its own bin's zero image, where (image - shift) = -shift
-        const int qc = im_pre[cen_img[cb]] + (cq - cen_pre[cb]);
+        const int qc = cen_rank[cq];
         const float4 xi = cf[qc];
-        const uint64_t jsi = cjd[qc];
-        const int i = (int)(jsi >> 32);
-        int si0, si1, si2;
-        unpack_img((uint32_t)(jsi & 0xffffffffu), si0, si1, si2);
-        si0 = -si0;
-        si1 = -si1;
-        si2 = -si2;
+        const uint64_t ki = ckey[qc];
+        const int i = __builtin_amdgcn_readfirstlane((int)(ki >> 30));
+        // the centre's packed image is -shift_i: taking it off a candidate's key
+        // leaves (j << 30 | packed n), field by field (each field carries a bias of 512)
+        const uint64_t koff = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(ki & 0x3fffffffu)) - pack_img(0, 0, 0);
+        uint64_t* dst = keys_out + (size_t)i * kMaxNeigh;
         int count = 0;
         for (int base = 0; base < total; base += kWave) {
             const int q = base + lane;
-            bool ok = false, unsure = false;
-            if (q < total && q != qc) {
-                const float4 xq = cf[q];
-                const float dx = xi.x - xq.x, dy = xi.y - xq.y, dz = xi.z - xq.z;
-                const float d2f = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-                ok = d2f < lo_thr && d2f > band;
-                unsure = d2f <= band || (d2f >= lo_thr && d2f <= hi_thr);
-            }
-            const uint64_t jd = q < total ? cjd[q] : 0ull;
-            const int j = (int)(jd >> 32);
-            int d0, d1, d2i;
-            unpack_img((uint32_t)(jd & 0xffffffffu), d0, d1, d2i);
-            const int n0 = si0 + d0, n1 = si1 + d1, n2 = si2 + d2i;
-            if (__ballot(unsure)) {
-                if (unsure) {
-                    double x, y, z, d2;
-                    pair_vec(pos, i, j, R, n0, n1, n2, x, y, z, d2);
+            const float4 xq = cf[q];
+            const float dx = xi.x - xq.x, dy = xi.y - xq.y, dz = xi.z - xq.z;
+            const float d2f = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+            const bool near = d2f <= hi_thr && q != qc;
+            bool ok = near && d2f < lo_thr && d2f > band;
+            const uint64_t mnear = __ballot(near);
+            if (mnear == 0) continue;
+            const uint64_t key = near ? ckey[q] - koff : 0ull;
+            uint64_t mask = __ballot(ok);
+            if (mask != mnear) {
+                if (near && !ok) {
+                    int n0, n1, n2;
+                    unpack_img((uint32_t)(key & 0x3fffffffu), n0, n1, n2);
+                    double px, py, pz, d2;
+                    pair_vec(pos, i, (int)(key >> 30), R, n0, n1, n2, px, py, pz, d2);
                     ok = d2 > 0.0 && d2 < rc2;
                 }
+                mask = __ballot(ok);
             }
-            const uint64_t key = ((uint64_t)j << 30) | (uint64_t)pack_img(n0, n1, n2);
-            const uint64_t mask = __ballot(ok);
-            const int before = __popcll(mask & ((1ull << lane) - 1ull));
-            if (ok && count + before < kWaveKeys) wk[count + before] = key;
+            const int at = count + __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0));
+            if (ok && at < kMaxNeigh) dst[at] = key;
             count += __popcll(mask);
         }
-        if (count > kWaveKeys) {
-            // more neighbours than the staged buffer holds: the bin goes to the wide search
-            if (lane == 0) {
-                s_ovf[cb] = 1;
-                atomicOr(flag, 8);
-            }
-            continue;
-        }
-        const int n = count;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        uint64_t* dst = keys_out + (size_t)i * kMaxNeigh;
-        if (n <= kWave) rank_and_store<1>(wk, n, dst);
-        else if (n <= 2 * kWave) rank_and_store<2>(wk, n, dst);
-        else rank_and_store<4>(wk, n, dst);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if (lane == 0) cnt_out[i] = n;
+        if (count > kMaxNeigh && lane == 0) atomicOr(flag, 1);
+        if (lane == 0) cnt_out[i] = min(count, kMaxNeigh);
         wmax = max(wmax, count);
     }
     // one global atomic per block (a contended atomic per atom serialises the kernel)
     if (lane == 0) atomicMax(&s_max, wmax);
     __syncthreads();
     if (t == 0) atomicMax(flag + 1, s_max);
-    if (t < ncb) bin_ovf[cen_bin[t]] = s_ovf[t];
+    if (t < ncb) bin_ovf[cen_bin[t]] = 0;
 }
 
 // CSR fill: index, packed image, neighbour species and FP32 pair geometry
@@ -726,11 +780,19 @@ static hipError_t grid_setup(ann_ctx* ctx, double rc) {
         c.nbins = c.nb[0] * c.nb[1] * c.nb[2];
         c.boff = nbins;
         nbins += c.nbins;
-        // 2x2x2 bins per staged block when the enlarged search box still fits
+    }
+    // 2x2x2 bins per staged block share one box of candidates; with few bins one
+    // bin per block spreads the centres over the chip instead (192 atoms in 64 bins:
+    // 12.0 us against 21.8 in super-bins; 2,048 bins and more lose by it, 12,288
+    // atoms 64.5 against 29.2)
+    const bool few = nbins <= 2 * ctx->num_cu;
+    for (int s = 0; s < S; ++s) {
+        CellInfo& c = info[s];
+        // when the enlarged search box still fits
         const double per_bin = (double)(ctx->atom_off[s + 1] - ctx->atom_off[s]) / c.nbins;
         const double box2 = (double)(std::min(2, c.nb[0]) + 2 * c.k[0]) * (std::min(2, c.nb[1]) + 2 * c.k[1]) *
                             (std::min(2, c.nb[2]) + 2 * c.k[2]);
-        c.sb = (ctx->tune_sb != 1 && box2 * per_bin <= 0.7 * kStageCap && box2 <= kStageImages) ? 2 : 1;
+        c.sb = (ctx->tune_sb != 1 && !few && box2 * per_bin <= 0.8 * kStageCap && box2 <= kStageImages) ? 2 : 1;
         for (int a = 0; a < 3; ++a) c.nsb[a] = (c.nb[a] + c.sb - 1) / c.sb;
         const int nsbins = c.nsb[0] * c.nsb[1] * c.nsb[2];
         c.sboff = (int)bin_struc.size();
