@@ -546,7 +546,7 @@ extern "C" int ann_destroy(ann_ctx* ctx) {
     void* ptrs[] = {ctx->d_off_own, ctx->d_cells_own, ctx->d_species_own, ctx->dm, ctx->da.rad_rs, ctx->da.rad_eta, ctx->da.rad_etal, ctx->da.ang_eta, ctx->da.ang_zeta, ctx->da.ang_lam,
                     ctx->da.W, ctx->da.inpw, ctx->da.inpb, ctx->da.params, ctx->da.adam_m, ctx->da.adam_v,
                     ctx->d_struc_of, ctx->d_cellinfo, ctx->d_cellmat, ctx->d_bin_of, ctx->d_shift, ctx->d_bin_cnt,
-                    ctx->d_bin_start, ctx->d_bin_atoms, ctx->d_keys, ctx->d_cnt, ctx->d_flag, ctx->nl.off,
+                    ctx->d_bin_start, ctx->d_bin_atoms, ctx->d_keys, ctx->d_tab, ctx->d_cnt, ctx->d_flag, ctx->nl.off,
                     ctx->nl.idx, ctx->nl.img, ctx->nl.rev, ctx->nl.geo, ctx->nl.nsp, ctx->d_G, ctx->d_dEdG,
                     ctx->d_Eatom, ctx->d_P, ctx->d_u, ctx->d_v, ctx->d_F, ctx->d_E, ctx->d_gE, ctx->d_atomvir,
                     ctx->d_scr, ctx->d_gpart, ctx->d_rank, ctx->d_spcount, ctx->d_rkflag, ctx->d_rkpre, ctx->d_perm, ctx->d_tiles, ctx->d_spend, ctx->d_grad_tiles, ctx->d_gsplit,

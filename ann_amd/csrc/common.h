@@ -274,6 +274,9 @@ struct ann_ctx {
     int rb_seq = 0;                   // completion marker of the last neighbour-build readback
     int* d_rb = nullptr;              // the same words as seen from the device
     int64_t keys_cap = 0;
+    uint64_t* d_tab = nullptr;        // rank tables of the rows (structures of at most 2048 atoms), tab_words each
+    int64_t tab_cap = 0;
+    int tab_words = 0;                // 0: the batch has a larger structure
     // work buffers
     float* d_G = nullptr;
     float* d_dEdG = nullptr;

@@ -39,6 +39,7 @@ constexpr int kMaxImages = 1024;   // bin images searched per atom
 struct CellInfo {
     int nb[3], k[3], nbins, boff;
     int sb, nsb[3], sboff;
+    int single;               // every perpendicular width is at least 2 rc: no partner has two images in a row
 };
 
 __global__ void k_struc_of(const int* __restrict__ off, int nstruc, int* __restrict__ sof) {
@@ -517,33 +518,112 @@ __global__ __launch_bounds__(kStageThreads) void k_search_bins(
     if (t < ncb) bin_ovf[cen_bin[t]] = 0;
 }
 
-// CSR fill: index, packed image, neighbour species and FP32 pair geometry
-__global__ void k_compact(int N, const double* __restrict__ pos, const int* __restrict__ sof,
-                          const double* __restrict__ cells, const int* __restrict__ species,
-                          const uint64_t* __restrict__ keys, const int* __restrict__ off,
-                          int* __restrict__ idx, uint32_t* __restrict__ img, int* __restrict__ rev,
-                          float4* __restrict__ geo, uint8_t* __restrict__ nsp, const int* __restrict__ order,
-                          int cap) {
+// CSR fill: index, packed image, neighbour species and FP32 pair geometry.
+// TAB: also the row's rank table, one 8-byte word per 32 atoms of the structure:
+// which of them the row holds (low half) and how many entries come before them
+// (high half), from which k_rev_table reads any partner's place in the row.
+// Against a binary search of the partner's row per pair (k_rev), us, tables and
+// reverse slots together: 273,561 atoms 286 + 406 -> 289 + 179, 12,288 atoms 14.1 +
+// 19.7 -> 16.4 + 9.3, 87,912 Li/P/S atoms (several images per partner) 44 + 53 ->
+// 50 + 44, 2,048 atoms 10.6 + 15.8 -> 10.7 + 7.3.
+constexpr int kTabAtoms = 2048;              // largest structure with rank tables
+constexpr int kTabWords = kTabAtoms / 32;
+constexpr int kCompactThreads = 128;
+
+template <bool TAB>
+__global__ __launch_bounds__(kCompactThreads) void k_compact(
+    int N, const double* __restrict__ pos, const int* __restrict__ sof, const double* __restrict__ cells,
+    const int* __restrict__ species, const uint64_t* __restrict__ keys, const int* __restrict__ off,
+    int* __restrict__ idx, uint32_t* __restrict__ img, int* __restrict__ rev, float4* __restrict__ geo,
+    uint8_t* __restrict__ nsp, const int* __restrict__ order, int cap, const int* __restrict__ aoff, int tabw,
+    uint64_t* __restrict__ tab) {
+    __shared__ unsigned mask[TAB ? kTabWords : 1];
+    __shared__ int ent[TAB ? kTabWords : 1];
     // centres in bin order: the blocks of one XCD cover one region of space,
     // so the partners they read stay in that XCD's L2
     const int b = xcd_block(blockIdx.x, gridDim.x);
     if (b >= N || off[N] > cap) return;     // a list that does not fit is compacted again after growing
     const int i = order[b];
-    const int o = off[i], n = off[i + 1] - o;
-    const double* R = cells + 9 * sof[i];
-    for (int t = threadIdx.x; t < n; t += blockDim.x) {
+    const int o = off[i], n = off[i + 1] - o, s = sof[i];
+    const double* R = cells + 9 * s;
+    const int a0 = TAB ? aoff[s] : 0;
+    if (TAB) {
+        if (threadIdx.x < kTabWords) {
+            mask[threadIdx.x] = 0;
+            ent[threadIdx.x] = 0;
+        }
+        __syncthreads();
+    }
+    for (int t = threadIdx.x; t < n; t += kCompactThreads) {
         const uint64_t key = keys[(size_t)i * kMaxNeigh + t];
         const int j = (int)(key >> 30);
         const uint32_t p = (uint32_t)(key & 0x3fffffffu);
+        if (TAB) {
+            atomicOr(&mask[(j - a0) >> 5], 1u << ((j - a0) & 31));
+            atomicAdd(&ent[(j - a0) >> 5], 1);
+        }
         int n0, n1, n2;
         unpack_img(p, n0, n1, n2);
         double x, y, z, d2;
         pair_vec(pos, i, j, R, n0, n1, n2, x, y, z, d2);
         idx[o + t] = j;
         img[o + t] = p;
-        rev[o + t] = o + t;
+        if (!TAB) rev[o + t] = o + t;
         geo[o + t] = make_float4((float)x, (float)y, (float)z, (float)sqrt(d2));
         nsp[o + t] = (uint8_t)species[j];
+    }
+    if (TAB) {
+        __syncthreads();
+        const int w = threadIdx.x;
+        if (w < kWave) {
+            const int v = ent[w];            // kTabWords is the wavefront's width
+            int inc = v;
+#pragma unroll
+            for (int q = 1; q < kWave; q <<= 1) {
+                const int u = __shfl_up(inc, q);
+                if (w >= q) inc += u;
+            }
+            if (w < tabw) tab[(size_t)i * tabw + w] = ((uint64_t)(uint32_t)(inc - v) << 32) | mask[w];
+        }
+    }
+}
+static_assert(kTabWords == kWave, "one lane per word of the rank table");
+
+// Reverse slots from the rank tables: the place of centre i in partner j's row is
+// the entries before i's word plus the set bits below i.  Where a partner can
+// appear with several images the bits undercount, and the row is walked on from
+// there to the entry (j -> i, -n).
+__global__ __launch_bounds__(256) void k_rev_table(int N, const int* __restrict__ idx, const uint32_t* __restrict__ img,
+                                                   const int* __restrict__ off, int* __restrict__ rev,
+                                                   int* __restrict__ flag, int cap, const int* __restrict__ sof,
+                                                   const int* __restrict__ aoff, const CellInfo* __restrict__ ci, int tabw,
+                                                   const uint64_t* __restrict__ tab) {
+    const int i = xcd_block(blockIdx.x, gridDim.x) * (blockDim.x / kWave) + threadIdx.x / kWave;
+    if (i >= N || off[N] > cap) return;
+    const int o = off[i], n = off[i + 1] - o, s = sof[i], r = i - aoff[s];
+    const int w = r >> 5;
+    const unsigned below = (1u << (r & 31)) - 1u;
+    const bool single = ci[s].single != 0;
+    for (int t = threadIdx.x % kWave; t < n; t += kWave) {
+        const int j = idx[o + t];
+        const uint64_t e = tab[(size_t)j * tabw + w];
+        const int oj = off[j];
+        int at = oj + (int)(e >> 32) + __popc((unsigned)e & below);
+        if (!single) {
+            const int end = off[j + 1];
+            int n0, n1, n2;
+            unpack_img(img[o + t], n0, n1, n2);
+            const uint32_t want = pack_img(-n0, -n1, -n2);
+            while (at < end && (idx[at] < i || (idx[at] == i && img[at] < want))) ++at;
+            if (at >= end || idx[at] != i || img[at] != want) {   // impossible for the symmetric FP64 test
+                atomicOr(flag, 4);
+                at = o + t;
+            }
+        } else if (!((unsigned)e >> (r & 31) & 1u)) {
+            atomicOr(flag, 4);
+            at = o + t;
+        }
+        rev[o + t] = at;
     }
 }
 
@@ -776,6 +856,7 @@ static hipError_t grid_setup(ann_ctx* ctx, double rc) {
             c.nb[a] = std::max(1, (int)std::floor(2.0 * w / rc * (1.0 - 1e-12)));
             c.nb[a] = std::min(c.nb[a], 256);
             c.k[a] = (int)std::ceil(rc * c.nb[a] / w * (1.0 + 1e-12));
+            c.single = (a == 0 || c.single) && w >= 2.0 * rc * (1.0 + 1e-9);
         }
         c.nbins = c.nb[0] * c.nb[1] * c.nb[2];
         c.boff = nbins;
@@ -856,17 +937,26 @@ static void launch_compact(ann_ctx* ctx, int cap) {
     const int N = ctx->natoms;
     hipStream_t st = ctx->stream;
     NList& nl = ctx->nl;
+    // rank tables where every structure fits one (8 bytes per 32 atoms and row);
+    // larger structures search their partners' rows
+    const bool tab = ctx->tab_words > 0;
     {
         Launch L(ctx, "nb_compact");
-        k_compact<<<N, 128, 0, st>>>(N, ctx->d_pos, ctx->d_struc_of, ctx->d_cells, ctx->d_species, ctx->d_keys,
-                                     nl.off, nl.idx, nl.img, nl.rev, nl.geo, nl.nsp, ctx->d_bin_atoms, cap);
+        (tab ? k_compact<true> : k_compact<false>)<<<N, kCompactThreads, 0, st>>>(
+            N, ctx->d_pos, ctx->d_struc_of, ctx->d_cells, ctx->d_species, ctx->d_keys, nl.off, nl.idx, nl.img, nl.rev,
+            nl.geo, nl.nsp, ctx->d_bin_atoms, cap, ctx->d_atom_off, ctx->tab_words, ctx->d_tab);
     }
     // a missing reverse slot (impossible for the symmetric FP64 test) is
     // reported by the next synchronising call (ann_nlist_size, next build)
     Launch L(ctx, "nb_rev");
     constexpr int kRevRows = 4;                 // centres (wavefronts) per workgroup
-    k_rev<<<(N + kRevRows - 1) / kRevRows, kRevRows * kWave, 0, st>>>(N, nl.idx, nl.img, nl.off, nl.rev, ctx->d_flag + 2,
-                                                                      ctx->d_bin_atoms, cap);
+    if (tab)
+        k_rev_table<<<(N + kRevRows - 1) / kRevRows, kRevRows * kWave, 0, st>>>(
+            N, nl.idx, nl.img, nl.off, nl.rev, ctx->d_flag + 2, cap, ctx->d_struc_of, ctx->d_atom_off,
+            reinterpret_cast<const CellInfo*>(ctx->d_cellinfo), ctx->tab_words, ctx->d_tab);
+    else
+        k_rev<<<(N + kRevRows - 1) / kRevRows, kRevRows * kWave, 0, st>>>(N, nl.idx, nl.img, nl.off, nl.rev,
+                                                                          ctx->d_flag + 2, ctx->d_bin_atoms, cap);
 }
 
 hipError_t neighbors_build(ann_ctx* ctx, double rc) {
@@ -877,6 +967,13 @@ hipError_t neighbors_build(ann_ctx* ctx, double rc) {
     int64_t kc = ctx->keys_cap;
     HIPCHK(grow(ctx->d_keys, kc, (int64_t)N * kMaxNeigh));
     ctx->keys_cap = kc;
+    ctx->tab_words = 0;
+    int most = 0;                               // atoms of the largest structure
+    for (int s = 0; s < ctx->nstruc; ++s) most = std::max(most, ctx->atom_off[s + 1] - ctx->atom_off[s]);
+    if (most <= kTabAtoms) {
+        ctx->tab_words = (most + 31) / 32;
+        HIPCHK(grow(ctx->d_tab, ctx->tab_cap, (int64_t)N * ctx->tab_words));
+    }
     int64_t rcap = ctx->binrec_cap;
     HIPCHK(grow(ctx->d_binrec, rcap, (int64_t)N));
     ctx->binrec_cap = rcap;
