@@ -2,9 +2,9 @@
 //
 // Same mathematics as ANN::fpbp + DODZ::grad (src/ml/nn.cpp:1367-1389,
 // 1801-1830).  Atoms are grouped by species (a species-sorted permutation of
-// the batch) into tiles of 16 rows; one wavefront owns a tile and runs every
+// the batch) into tiles of 16 rows; four wavefronts share a tile and run every
 // layer as 16 x N x K products on the matrix cores (BF16 operands split into
-// three terms, FP32 accumulation; mm_bf16x3 below):
+// three terms, FP32 accumulation; Operands below):
 //   forward:  Z_l = A_{l-1} W_l^T (+ b_l), activation on the accumulator;
 //   backward: g_{L-1} = outw W_L^T . sigma'_{L-1}, g_{l-1} = (g_l W_l) . sigma'_{l-1},
 //             dE/dG = (g_0 W_0) . inpw.
@@ -39,14 +39,12 @@ struct MfmaArgs {
     const uint4* wtab;     // BF16x3 operand tables of the hidden-layer weights
 };
 
-// acc[ct] += X (16 x K, rows = atoms, from LDS) * B (K x 16 columns of tile ct)
-// for every column tile at once on v_mfma_f32_16x16x32_bf16.  BF16 carries 8
+// acc += X (16 x K, rows = atoms, from LDS) * B (K x 16 columns of one tile)
+// on v_mfma_f32_16x16x32_bf16.  BF16 carries 8
 // mantissa bits, so both operands are split into three BF16 terms
 // x = x0 + x1 + x2 (x0 = bf16(x), x1 = bf16(x - x0), x2 = bf16(x - x0 - x1)) and
 // the six products with i + j <= 2 are accumulated in FP32: truncation
-// ~2^-24 relative, the FP32 level the 1e-5 force bar needs.  The activation
-// operand is split once per k block and reused by every column tile; the
-// tiles advance together so one block's weight loads are in flight together.
+// ~2^-24 relative, the FP32 level the 1e-5 force bar needs.
 // Lane l supplies row l % 16 of X and column l % 16 of B for k block
 // 8 (l / 16) .. +7 and receives D rows 4 (l / 16) .. +3 of column l % 16.
 __device__ __forceinline__ void split3(float x, __bf16& a, __bf16& b, __bf16& c) {
@@ -64,39 +62,60 @@ __device__ __forceinline__ bf16x8 as_bf16x8(uint4 u) {
 
 // The right operands come pre-split from a table (k_wtables): for k block kk
 // and column tile ct, the three BF16 terms of lane l are the 16-byte entries
-// ((kk * nt + ct) * 3 + p) * 64 + l, p = 0, 1, 2.
-template <int NT>
-__device__ __forceinline__ void mm_bf16x3(int K, int ncol, const float (*X)[kMaxK + 1], const uint4* __restrict__ tab,
-                                          f32x4 (&acc)[NT], int wv) {
-    const int lane = threadIdx.x % kWave;
-    const int row = lane % 16, kb = 8 * (lane / 16);
-    const int nt = (ncol + 15) / 16;
-    for (int k0 = 0, kk = 0; k0 < K; k0 += 32, ++kk) {
-        bf16x8 a0, a1, a2;
+// ((kk * nt + ct) * 3 + p) * 64 + l, p = 0, 1, 2.  The left operands are split
+// once, by the thread that writes them, into three BF16 planes of the tile.
+constexpr int kNetWaves = 4;                // wavefronts per tile; column tile ct belongs to wavefront ct % 4
+constexpr int kPlaneK = kMaxK + 8;          // row stride of a plane: 16-byte rows, all banks in a 16-row read
+typedef __bf16 PlaneRow[kPlaneK];
+
+// This wavefront's operands of a product with NH own column tiles and up to KB k
+// blocks.  Loaded a phase ahead, so that the loads' latency runs beside the phase
+// before (they depend on nothing but the tile's species).
+template <int NH, int KB>
+struct Operands {
+    uint4 w[NH][KB][3];
+    __device__ __forceinline__ void load(const uint4* __restrict__ tab, int K, int ncol, int wv) {
+        const int lane = threadIdx.x % kWave, nt = (ncol + 15) / 16, nkb = (K + 31) / 32;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int k = k0 + kb + j;
-            __bf16 x0, x1, x2;
-            split3(k < K ? X[row][k] : 0.0f, x0, x1, x2);
-            a0[j] = x0; a1[j] = x1; a2[j] = x2;
-        }
+        for (int h = 0; h < NH; ++h)
 #pragma unroll
-        for (int ct = 0; ct < NT; ++ct) {
-            if (ct >= nt) break;
-            if ((ct & 1) != wv) continue;           // column tiles alternate between the two wavefronts
-            const uint4* e = tab + (size_t)((kk * nt + ct) * 3) * kWave + lane;
-            const bf16x8 b0 = as_bf16x8(e[0]), b1 = as_bf16x8(e[kWave]), b2 = as_bf16x8(e[2 * kWave]);
-            f32x4 c = acc[ct];
-            c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, b0, c, 0, 0, 0);
-            c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b1, c, 0, 0, 0);
-            c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b2, c, 0, 0, 0);
-            c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b0, c, 0, 0, 0);
-            c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b1, c, 0, 0, 0);
-            c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b0, c, 0, 0, 0);
-            acc[ct] = c;
+            for (int kk = 0; kk < KB; ++kk) {
+                const int ct = h * kNetWaves + wv;
+                if (ct < nt && kk < nkb) {
+                    const uint4* e = tab + (size_t)((kk * nt + ct) * 3) * kWave + lane;
+#pragma unroll
+                    for (int p = 0; p < 3; ++p) w[h][kk][p] = e[p * kWave];
+                }
+            }
+    }
+    // acc[h] += X (16 x K planes) * (own column tile h)
+    __device__ __forceinline__ void mul(const PlaneRow* X0, const PlaneRow* X1, const PlaneRow* X2, int K, int ncol,
+                                        int wv, f32x4 (&acc)[NH]) const {
+        const int lane = threadIdx.x % kWave, row = lane % 16, kb = 8 * (lane / 16);
+        const int nt = (ncol + 15) / 16, nkb = (K + 31) / 32;
+        if (wv >= nt) return;
+#pragma unroll
+        for (int kk = 0; kk < KB; ++kk) {
+            if (kk >= nkb) break;
+            const bf16x8 a0 = *reinterpret_cast<const bf16x8*>(&X0[row][32 * kk + kb]);
+            const bf16x8 a1 = *reinterpret_cast<const bf16x8*>(&X1[row][32 * kk + kb]);
+            const bf16x8 a2 = *reinterpret_cast<const bf16x8*>(&X2[row][32 * kk + kb]);
+#pragma unroll
+            for (int h = 0; h < NH; ++h) {
+                if (h * kNetWaves + wv >= nt) break;
+                const bf16x8 b0 = as_bf16x8(w[h][kk][0]), b1 = as_bf16x8(w[h][kk][1]), b2 = as_bf16x8(w[h][kk][2]);
+                f32x4 c = acc[h];
+                c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, b0, c, 0, 0, 0);
+                c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b1, c, 0, 0, 0);
+                c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b2, c, 0, 0, 0);
+                c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b0, c, 0, 0, 0);
+                c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b1, c, 0, 0, 0);
+                c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b0, c, 0, 0, 0);
+                acc[h] = c;
+            }
         }
     }
-}
+};
 
 // The weight tables, all read from the FP32 weights W and rewritten after
 // every parameter update, in one launch (grid row = role and segment):
@@ -228,165 +247,195 @@ hipError_t split_weights(ann_ctx* ctx, int* tick) {
     return weight_tables(ctx, tick, true);
 }
 
-// two wavefronts per 16-atom single-species tile: the column tiles of every
-// product alternate between them (the launch has fewer tiles than SIMDs).
+// Four wavefronts per 16-atom single-species tile, the column tiles of every
+// product dealt round.  A batch of small structures has fewer tiles than the chip
+// has SIMDs and a tile is a chain of short products, so latency is what counts:
+// every product's weight operands are loaded a phase ahead, the inputs come
+// straight into the split planes, and the output neuron and the first gradient
+// share a phase.
 // NT: column tiles of 16 of the widest hidden layer (4 up to 64 neurons, 8 up
 // to 128), so narrow networks keep their registers and LDS.
+// Against two wavefronts per tile that split the left operand at every product and
+// loaded each operand where it was used, us: 192 atoms 22.6 -> 12.1, 2,048 atoms 22
+// -> 12.4, 12,288 atoms 28.8 -> 17.3, 273,561 atoms 308 -> 248 (water 80-32-32-1),
+// 21,872 Li/P/S atoms (96-48-48-1) 35.4 -> 25.6.
 template <int NT>
-__global__ __launch_bounds__(128) void k_net_mfma(MfmaArgs A) {
+__global__ __launch_bounds__(kNetWaves * kWave) void k_net_mfma(MfmaArgs A) {
     constexpr int W = 16 * NT;                  // widest hidden layer of this instance
-    __shared__ float act[kTile][kMaxK + 1];     // activations / gradients, operand side
+    constexpr int NH = NT / kNetWaves;          // own column tiles of a hidden layer
+    constexpr int NB = kMaxK / 16 / kNetWaves;  // own column tiles of the input side
+    constexpr int KH = W / 32;                  // k blocks of a hidden layer
+    constexpr int kThreads = kNetWaves * kWave;
+    __shared__ __align__(16) PlaneRow X0[kTile], X1[kTile], X2[kTile];   // left operand, split
+    __shared__ float act[kTile][W + 1];         // activations of the last hidden layer
     __shared__ float sdz[kMaxLayers - 1][kTile][W + 1];
-    __shared__ int atoms[kTile];
-    const int t = blockIdx.x, tid = threadIdx.x, lane = tid % kWave, wv = tid / kWave;
-    constexpr int kThreads = 2 * kWave;
-    if (t >= A.ntiles) return;
+    const int t = blockIdx.x, tid = threadIdx.x, lane = tid % kWave;
+    const int wv = __builtin_amdgcn_readfirstlane(tid / kWave);
     const int2 tl = A.tiles[t];
     const int a = tl.x;
     const int nrow = min(kTile, A.spend[a] - tl.y);
     const NetDesc& D = A.dm->net[a];
-    const int L = D.nlayer;
+    const int L = D.nlayer, nin = D.nin;
     const float* iw = A.inpw + D.inoff;
     const float* ib = A.inpb + D.inoff;
-    if (tid < kTile) atoms[tid] = tid < nrow ? A.perm[tl.y + tid] : -1;
-    __syncthreads();
-    // scaled input s = inpw (G + inpb) into LDS: lanes over the inputs, rows unrolled
+    Operands<NH, kMaxK / 32> wf;
+    if (L > 1) wf.load(A.wtab + D.wsf[0], nin, D.nodes[0], wv);
+    // a value and its right neighbour, split, into the planes
+    auto put2 = [&](int r, int k, float x, float y) {
+        __bf16 p[3], q[3];
+        split3(x, p[0], p[1], p[2]);
+        split3(y, q[0], q[1], q[2]);
+        X0[r][k] = p[0]; X0[r][k + 1] = q[0];
+        X1[r][k] = p[1]; X1[r][k + 1] = q[1];
+        X2[r][k] = p[2]; X2[r][k + 1] = q[2];
+    };
+    auto put1 = [&](int r, int k, float x) {
+        __bf16 p, q, u;
+        split3(x, p, q, u);
+        X0[r][k] = p;
+        X1[r][k] = q;
+        X2[r][k] = u;
+    };
+    // scaled input s = inpw (G + inpb): a wavefront takes every fourth row, lanes two inputs each
     {
-        float w2[kMaxK / kWave], b2[kMaxK / kWave];
+        const int k = 2 * lane;
+        const bool in0 = k < nin, in1 = k + 1 < nin;
+        const float w0 = in0 ? iw[k] : 0.0f, w1 = in1 ? iw[k + 1] : 0.0f;
+        const float b0 = in0 ? ib[k] : 0.0f, b1 = in1 ? ib[k + 1] : 0.0f;
+        float g0[kTile / kNetWaves], g1[kTile / kNetWaves];
 #pragma unroll
-        for (int h = 0; h < kMaxK / kWave; ++h) {
-            const int k = lane + h * kWave;
-            w2[h] = k < D.nin ? iw[k] : 0.0f;
-            b2[h] = k < D.nin ? ib[k] : 0.0f;
+        for (int q = 0; q < kTile / kNetWaves; ++q) {
+            const int r = wv + q * kNetWaves;
+            const float* G = A.G + (size_t)A.perm[tl.y + min(r, nrow - 1)] * A.ldg;
+            g0[q] = in0 ? G[k] : 0.0f;
+            g1[q] = in1 ? G[k + 1] : 0.0f;
         }
 #pragma unroll
-        for (int r = wv; r < kTile; r += 2) {
-            const int ai = atoms[r];
-#pragma unroll
-            for (int h = 0; h < kMaxK / kWave; ++h) {
-                const int k = lane + h * kWave;
-                act[r][k] = (ai >= 0 && k < D.nin) ? w2[h] * (A.G[(size_t)ai * A.ldg + k] + b2[h]) : 0.0f;
-            }
+        for (int q = 0; q < kTile / kNetWaves; ++q) {
+            const int r = wv + q * kNetWaves;
+            const float x = r < nrow ? w0 * (g0[q] + b0) : 0.0f, y = r < nrow ? w1 * (g1[q] + b1) : 0.0f;
+            put2(r, k, x, y);                               // zero past the inputs, up to kMaxK
         }
     }
-    __syncthreads();
     const int col = lane % 16, rb = 4 * (lane / 16);
-    int ni = D.nin;
-    for (int l = 0; l < L - 1; ++l) {
-        const int no = D.nodes[l];
-        const float* bl = A.W + D.boff[l];
-        float out[NT][4];
-        f32x4 accs[NT];
-#pragma unroll
-        for (int ct = 0; ct < NT; ++ct) accs[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
-        mm_bf16x3<NT>(ni, no, act, A.wtab + D.wsf[l], accs, wv);
-#pragma unroll
-        for (int ct = 0; ct < NT; ++ct) {
-            if (ct * 16 >= no) break;
-            if ((ct & 1) != wv) continue;
-            const f32x4 acc = accs[ct];
-            const int n = ct * 16 + col;
-            const float bn = n < no ? bl[n] : 0.0f;
-            float z[4], av[4], dv[4], d2[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) z[i] = acc[i] + bn;
-            act_many<false, 4>(D.neuron, D.c, z, av, dv, d2);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                out[ct][i] = n < no ? av[i] : 0.0f;
-                sdz[l][rb + i][n < W ? n : W] = n < no ? dv[i] : 0.0f;
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int ct = 0; ct < NT; ++ct) {
-            if (ct * 16 >= no) break;
-            if ((ct & 1) != wv) continue;
-            const int n = ct * 16 + col;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) act[rb + i][n] = n < no ? out[ct][i] : 0.0f;
-        }
-        // zero the padding up to the next multiple of 32
-        for (int q = tid; q < kTile * 32; q += kThreads) {
-            const int r = q / 32, k = no + q % 32;
-            if (k < kMaxK) act[r][k] = 0.0f;
-        }
-        __syncthreads();
-        ni = no;
-    }
-    // linear output layer (1 neuron) on the vector ALU
+    // thread (row, slot of 16) of the phases that run over a row's neurons
+    const int orow = tid / 16, osl = tid % 16;
     const float* WL = A.W + D.woff[L - 1];
-    const float bL = A.W[D.boff[L - 1]];
-    if (tid < nrow) {
-        float z = bL;
-        for (int m = 0; m < ni; ++m) z += WL[m] * act[tid][m];
-        A.Eatom[atoms[tid]] = D.outb + D.outw * z;
-    }
-    if (!A.dEdG) return;
     if (L == 1) {
+        // no hidden layer: the output neuron reads the scaled inputs
+        float z = 0.0f;
+        if (orow < nrow) {
+            const float* G = A.G + (size_t)A.perm[tl.y + orow] * A.ldg;
+            for (int m = osl; m < nin; m += 16) z += WL[m] * (iw[m] * (G[m] + ib[m]));
+        }
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) z += __shfl_xor(z, o);
+        if (orow < nrow && osl == 0) A.Eatom[A.perm[tl.y + orow]] = D.outb + D.outw * (A.W[D.boff[0]] + z);
+        if (!A.dEdG) return;
         for (int q = tid; q < kTile * A.ldg; q += kThreads) {
             const int r = q / A.ldg, m = q % A.ldg;
-            if (r < nrow) A.dEdG[(size_t)atoms[r] * A.ldg + m] = m < D.nin ? D.outw * WL[m] * iw[m] : 0.0f;
+            if (r < nrow) A.dEdG[(size_t)A.perm[tl.y + r] * A.ldg + m] = m < nin ? D.outw * WL[m] * iw[m] : 0.0f;
         }
         return;
     }
-    __syncthreads();
-    // g_{L-1} = outw W_L . sigma'_{L-1}  (operand layout, rows = atoms)
-    for (int q = tid; q < kTile * kMaxK; q += kThreads) {
-        const int r = q / kMaxK, m = q % kMaxK;
-        act[r][m] = m < ni ? D.outw * WL[m] * sdz[L - 2][r][m] : 0.0f;
-    }
-    __syncthreads();
-    for (int l = L - 2; l >= 0; --l) {
+    int ni = nin;
+    for (int l = 0; l < L - 1; ++l) {
         const int no = D.nodes[l];
-        const int nprev = l == 0 ? D.nin : D.nodes[l - 1];
-        float out[kMaxK / 16][4];
-        f32x4 accs[kMaxK / 16];
+        const float* bl = A.W + D.boff[l];
+        float bias[NH];
 #pragma unroll
-        for (int ct = 0; ct < kMaxK / 16; ++ct) accs[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
-        mm_bf16x3<kMaxK / 16>(no, nprev, act, A.wtab + D.wsb[l], accs, wv);
+        for (int h = 0; h < NH; ++h) {
+            const int n = (h * kNetWaves + wv) * 16 + col;
+            bias[h] = n < no ? bl[n] : 0.0f;
+        }
+        __syncthreads();                                    // the planes are written
+        f32x4 acc[NH];
 #pragma unroll
-        for (int ct = 0; ct < kMaxK / 16; ++ct) {
-            if (ct * 16 >= nprev) break;
-            if ((ct & 1) != wv) continue;
-            const f32x4 acc = accs[ct];
-            const int m = ct * 16 + col;
+        for (int h = 0; h < NH; ++h) acc[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+        wf.mul(X0, X1, X2, ni, no, wv, acc);
+        if (l + 1 < L - 1) wf.load(A.wtab + D.wsf[l + 1], no, D.nodes[l + 1], wv);
+        __syncthreads();                                    // the planes are read
+#pragma unroll
+        for (int h = 0; h < NH; ++h) {
+            const int n = (h * kNetWaves + wv) * 16 + col;
+            float av[4] = {0.f, 0.f, 0.f, 0.f}, dv[4] = {0.f, 0.f, 0.f, 0.f}, d2[4];
+            if ((h * kNetWaves + wv) * 16 < no) {
+                float z[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) z[i] = acc[h][i] + bias[h];
+                act_many<false, 4>(D.neuron, D.c, z, av, dv, d2);
+            }
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                float v = acc[i];
-                if (l > 0) v *= (m < nprev) ? sdz[l - 1][rb + i][m] : 0.0f;
-                out[ct][i] = v;
+                const float x = n < no ? av[i] : 0.0f;
+                put1(rb + i, n, x);                         // zero past the neurons, up to W
+                act[rb + i][n] = x;
+                sdz[l][rb + i][n] = n < no ? dv[i] : 0.0f;
             }
         }
+        ni = no;
+    }
+    Operands<NH, KH> wbh;                                   // backward through hidden layers
+    Operands<NB, KH> wb0;                                   // and through the input layer
+    const bool grad = A.dEdG != nullptr;
+    if (grad) {
+        if (L > 2) wbh.load(A.wtab + D.wsb[L - 2], ni, D.nodes[L - 3], wv);
+        else wb0.load(A.wtab + D.wsb[0], ni, nin, wv);
+    }
+    __syncthreads();
+    // linear output neuron, and g_{L-1} = outw W_L . sigma'_{L-1} into the planes
+    {
+        float z = 0.0f;
+        for (int m = osl; m < W; m += 16) {
+            const float w = m < ni ? WL[m] : 0.0f;
+            z += w * act[orow][m];
+            if (grad) put1(orow, m, m < ni ? D.outw * w * sdz[L - 2][orow][m] : 0.0f);
+        }
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) z += __shfl_xor(z, o);
+        if (orow < nrow && osl == 0) A.Eatom[A.perm[tl.y + orow]] = D.outb + D.outw * (A.W[D.boff[L - 1]] + z);
+    }
+    if (!grad) return;
+    for (int l = L - 2; l >= 1; --l) {
+        const int no = D.nodes[l], nprev = D.nodes[l - 1];
         __syncthreads();
-        if (l > 0) {
+        f32x4 acc[NH];
 #pragma unroll
-            for (int ct = 0; ct < kMaxK / 16; ++ct) {
-                if (ct * 16 >= nprev) break;
-                if ((ct & 1) != wv) continue;
-                const int m = ct * 16 + col;
+        for (int h = 0; h < NH; ++h) acc[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+        wbh.mul(X0, X1, X2, no, nprev, wv, acc);
+        if (l > 1) wbh.load(A.wtab + D.wsb[l - 1], nprev, D.nodes[l - 2], wv);
+        else wb0.load(A.wtab + D.wsb[0], nprev, nin, wv);
+        __syncthreads();
 #pragma unroll
-                for (int i = 0; i < 4; ++i) act[rb + i][m] = m < nprev ? out[ct][i] : 0.0f;
-            }
-            for (int q = tid; q < kTile * 32; q += kThreads) {
-                const int r = q / 32, k = nprev + q % 32;
-                if (k < kMaxK) act[r][k] = 0.0f;
-            }
-        } else {
+        for (int h = 0; h < NH; ++h) {
+            const int m = (h * kNetWaves + wv) * 16 + col;
 #pragma unroll
-            for (int ct = 0; ct < kMaxK / 16; ++ct) {
-                if (ct * 16 >= A.ldg) break;
-                if ((ct & 1) != wv) continue;
-                const int m = ct * 16 + col;
+            for (int i = 0; i < 4; ++i) put1(rb + i, m, m < nprev ? acc[h][i] * sdz[l - 1][rb + i][m] : 0.0f);
+        }
+    }
+    {
+        float iwm[NB];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int r = rb + i;
-                    if (r < nrow && m < A.ldg)
-                        A.dEdG[(size_t)atoms[r] * A.ldg + m] = (m < D.nin && ct * 16 < nprev) ? out[ct][i] * iw[m] : 0.0f;
-                }
-            }
+        for (int h = 0; h < NB; ++h) {
+            const int m = (h * kNetWaves + wv) * 16 + col;
+            iwm[h] = m < nin ? iw[m] : 0.0f;
         }
         __syncthreads();
+        f32x4 acc[NB];
+#pragma unroll
+        for (int h = 0; h < NB; ++h) acc[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+        wb0.mul(X0, X1, X2, D.nodes[0], nin, wv, acc);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = rb + i;
+            if (r >= nrow) continue;
+            float* out = A.dEdG + (size_t)A.perm[tl.y + r] * A.ldg;
+#pragma unroll
+            for (int h = 0; h < NB; ++h) {
+                const int m = (h * kNetWaves + wv) * 16 + col;
+                if (m < A.ldg) out[m] = m < nin ? acc[h][i] * iwm[h] : 0.0f;
+            }
+        }
     }
 }
 
@@ -413,8 +462,8 @@ hipError_t net_fwd_mfma(ann_ctx* ctx, const float* G, float* Eatom, float* dEdG,
     for (int a = 0; a < ctx->hm.S; ++a)
         for (int l = 0; l < ctx->hm.net[a].nlayer - 1; ++l) wmax = std::max(wmax, ctx->hm.net[a].nodes[l]);
     Launch L(ctx, "net_mfma");
-    if (wmax <= 64) k_net_mfma<4><<<A.ntiles, 128, 0, ctx->stream>>>(A);
-    else k_net_mfma<8><<<A.ntiles, 128, 0, ctx->stream>>>(A);
+    if (wmax <= 64) k_net_mfma<4><<<A.ntiles, kNetWaves * kWave, 0, ctx->stream>>>(A);
+    else k_net_mfma<8><<<A.ntiles, kNetWaves * kWave, 0, ctx->stream>>>(A);
     return hipGetLastError();
 }
 
