@@ -1169,40 +1169,40 @@ __global__ void k_neigh_species(int64_t P, const int* __restrict__ idx, const in
     if (s < P) nsp[s] = (uint8_t)species[idx[s]];
 }
 
-// Host CSR (off [N+1], idx [P], img [P][3]) of the current batch into the
-// context's list: packed images, reverse slots found by sorting the entries,
-// neighbour species and pair geometry on the device.  Returns an ANN status.
-int set_neighbors_host(ann_ctx* ctx, const int* off, const int* idx, const int* img, double rc) {
-    const int N = ctx->natoms;
-    if (off[0] != 0) return fail(ANN_ERR_ARG, "neighbour list: off[0] must be 0");
-    int maxn = 0;
-    for (int i = 0; i < N; ++i) {
-        if (off[i + 1] < off[i]) return fail(ANN_ERR_ARG, "neighbour list: offsets must not decrease");
-        maxn = std::max(maxn, off[i + 1] - off[i]);
-    }
-    if (maxn > kMaxNeigh)
-        return fail(ANN_ERR_CAPACITY, "an atom has " + std::to_string(maxn) + " neighbours; capacity is " +
-                                          std::to_string(kMaxNeigh));
-    const int64_t P = off[N];
-    std::vector<uint32_t> pimg(std::max<int64_t>(P, 1));
-    std::vector<int> rev(std::max<int64_t>(P, 1), -1), owner(std::max<int64_t>(P, 1));
-    int s = 0;
-    for (int i = 0; i < N; ++i) {
-        while (ctx->atom_off[s + 1] <= i) ++s;
-        for (int q = off[i]; q < off[i + 1]; ++q) {
-            const int j = idx[q];
-            if (j < ctx->atom_off[s] || j >= ctx->atom_off[s + 1])
-                return fail(ANN_ERR_ARG, "neighbour list: partner outside the centre's structure");
-            for (int x = 0; x < 3; ++x)
-                if (img[3 * (int64_t)q + x] < -511 || img[3 * (int64_t)q + x] > 511)
-                    return fail(ANN_ERR_UNSUPPORTED, "neighbour list: image vector beyond +-511 cells");
-            pimg[q] = pack_img(img[3 * (int64_t)q], img[3 * (int64_t)q + 1], img[3 * (int64_t)q + 2]);
-            owner[q] = i;
-            if (j == i && pimg[q] == pack_img(0, 0, 0))
-                return fail(ANN_ERR_ARG, "neighbour list: atom " + std::to_string(i) + " lists itself in its own cell");
+// Reverse slots of a list whose rows have any order: a lane per entry walks the
+// partner's whole row and counts the entries (j -> i, -n).  Exactly one for every
+// entry of the list means that it is symmetric and holds nothing twice; anything
+// else raises the flag.  Entries times row length loads (1,536 atoms with 91
+// partners: 13 M, about 0.1 ms) against sorting the list on the host (17 ms).
+__global__ __launch_bounds__(256) void k_rev_scan(int N, const int* __restrict__ off, const int* __restrict__ idx,
+                                                  const uint32_t* __restrict__ img, int* __restrict__ rev,
+                                                  int* __restrict__ flag) {
+    const int i = blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
+    if (i >= N) return;
+    for (int s = off[i] + threadIdx.x % kWave; s < off[i + 1]; s += kWave) {
+        const int j = idx[s];
+        int n0, n1, n2;
+        unpack_img(img[s], n0, n1, n2);
+        const uint32_t want = pack_img(-n0, -n1, -n2);
+        int found = 0, at = s;
+        const int e = off[j + 1];
+#pragma unroll 8
+        for (int q = off[j]; q < e; ++q) {
+            const bool hit = idx[q] == i && img[q] == want;
+            found += hit ? 1 : 0;
+            at = hit ? q : at;
         }
+        rev[s] = at;
+        if (found != 1) atomicOr(flag, 1);
     }
-    // reverse slots: entry (i -> j, n) pairs with (j -> i, -n); sort by (centre, partner, image)
+}
+
+// The fault of a list that k_rev_scan refused, found on the host by sorting it
+static int list_fault(const int* off, const int* idx, const uint32_t* pimg, int N) {
+    const int64_t P = off[N];
+    std::vector<int> owner(std::max<int64_t>(P, 1));
+    for (int i = 0; i < N; ++i)
+        for (int q = off[i]; q < off[i + 1]; ++q) owner[q] = i;
     std::vector<int64_t> order(P);
     for (int64_t q = 0; q < P; ++q) order[q] = q;
     auto key = [&](int64_t q) { return std::make_tuple(owner[q], idx[q], pimg[q]); };
@@ -1221,7 +1221,40 @@ int set_neighbors_host(ann_ctx* ctx, const int* off, const int* idx, const int* 
             return fail(ANN_ERR_ARG, "neighbour list is not symmetric: entry " + std::to_string(q) + " (atom " +
                                          std::to_string(owner[q]) + " -> " + std::to_string(idx[q]) +
                                          ") has no reverse entry");
-        rev[q] = (int)*it;
+    }
+    return fail(ANN_ERR_HIP, "neighbour list: reverse slots not found");
+}
+
+// Host CSR (off [N+1], idx [P], img [P][3]) of the current batch into the
+// context's list: packed images, reverse slots found by walking the partners'
+// rows, neighbour species and pair geometry on the device.  Returns an ANN status.
+int set_neighbors_host(ann_ctx* ctx, const int* off, const int* idx, const int* img, double rc) {
+    const int N = ctx->natoms;
+    if (off[0] != 0) return fail(ANN_ERR_ARG, "neighbour list: off[0] must be 0");
+    int maxn = 0;
+    for (int i = 0; i < N; ++i) {
+        if (off[i + 1] < off[i]) return fail(ANN_ERR_ARG, "neighbour list: offsets must not decrease");
+        maxn = std::max(maxn, off[i + 1] - off[i]);
+    }
+    if (maxn > kMaxNeigh)
+        return fail(ANN_ERR_CAPACITY, "an atom has " + std::to_string(maxn) + " neighbours; capacity is " +
+                                          std::to_string(kMaxNeigh));
+    const int64_t P = off[N];
+    std::vector<uint32_t> pimg(std::max<int64_t>(P, 1));
+    int s = 0;
+    for (int i = 0; i < N; ++i) {
+        while (ctx->atom_off[s + 1] <= i) ++s;
+        for (int q = off[i]; q < off[i + 1]; ++q) {
+            const int j = idx[q];
+            if (j < ctx->atom_off[s] || j >= ctx->atom_off[s + 1])
+                return fail(ANN_ERR_ARG, "neighbour list: partner outside the centre's structure");
+            for (int x = 0; x < 3; ++x)
+                if (img[3 * (int64_t)q + x] < -511 || img[3 * (int64_t)q + x] > 511)
+                    return fail(ANN_ERR_UNSUPPORTED, "neighbour list: image vector beyond +-511 cells");
+            pimg[q] = pack_img(img[3 * (int64_t)q], img[3 * (int64_t)q + 1], img[3 * (int64_t)q + 2]);
+            if (j == i && pimg[q] == pack_img(0, 0, 0))
+                return fail(ANN_ERR_ARG, "neighbour list: atom " + std::to_string(i) + " lists itself in its own cell");
+        }
     }
     NList& nl = ctx->nl;
     hipStream_t st = ctx->stream;
@@ -1239,15 +1272,20 @@ int set_neighbors_host(ann_ctx* ctx, const int* off, const int* idx, const int* 
     if (P > 0) {
         ANN_HIP(hipMemcpyAsync(nl.idx, idx, sizeof(int) * P, hipMemcpyHostToDevice, st));
         ANN_HIP(hipMemcpyAsync(nl.img, pimg.data(), sizeof(uint32_t) * P, hipMemcpyHostToDevice, st));
-        ANN_HIP(hipMemcpyAsync(nl.rev, rev.data(), sizeof(int) * P, hipMemcpyHostToDevice, st));
+        k_rev_scan<<<(N + 3) / 4, 256, 0, st>>>(N, nl.off, nl.idx, nl.img, nl.rev, ctx->d_flag + 3);
+        ANN_HIP(hipGetLastError());
         k_neigh_species<<<(unsigned)((P + 255) / 256), 256, 0, st>>>(P, nl.idx, ctx->d_species, nl.nsp);
         ANN_HIP(hipGetLastError());
     }
     nl.npairs = P;
     nl.maxn = maxn;
     ANN_HIP(refresh_geometry(ctx));
+    // the refusal flag to the host words, cleared once read
+    k_readback<<<1, kWave, 0, st>>>(ctx->d_flag + 3, 1, ctx->d_rb + 9, 0, 1);
+    ANN_HIP(hipGetLastError());
     ANN_HIP(hipStreamSynchronize(st));       // the host vectors go out of scope
     (void)rc;
+    if (((volatile const int*)ctx->h_rb)[9]) return list_fault(off, idx, pimg.data(), N);
     return ANN_OK;
 }
 

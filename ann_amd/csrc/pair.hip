@@ -17,6 +17,7 @@
 // geometry is refreshed from them.  Host code; the device work is
 // ann_energy_forces.
 #include <cmath>
+#include <cstring>
 #include <string>
 #include <vector>
 
@@ -34,8 +35,11 @@ struct PairState {
     int hoff[2] = {0, 0};
     int nlocal = 0;
     bool have_list = false;
-    std::vector<double> h_out;
-    std::vector<float> h_ea;
+    // pinned host copies: positions and cell in, results out (a call ends with a
+    // synchronisation, so one set serves them all)
+    double* h_in = nullptr;     // [3 cap + 9]
+    double* h_out = nullptr;    // [10 + 3 cap]
+    float* h_ea = nullptr;      // [cap]
 };
 
 void pair_free(ann_ctx* ctx) {
@@ -44,6 +48,9 @@ void pair_free(ann_ctx* ctx) {
     void* ptrs[] = {p->pos, p->cell, p->species, p->off, p->out};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
+    void* pins[] = {p->h_in, p->h_out, p->h_ea};
+    for (void* q : pins)
+        if (q) (void)hipHostFree(q);
     delete p;
     ctx->pair = nullptr;
 }
@@ -81,6 +88,11 @@ extern "C" int ann_pair_compute(ann_ctx* ctx, int form, int new_list, int nlocal
         void* ptrs[] = {P.pos, P.cell, P.species, P.off, P.out};
         for (void* q : ptrs)
             if (q) ANN_HIP(hipFree(q));
+        void* pins[] = {P.h_in, P.h_out, P.h_ea};
+        for (void* q : pins)
+            if (q) ANN_HIP(hipHostFree(q));
+        P.h_in = P.h_out = nullptr;
+        P.h_ea = nullptr;
         P.pos = P.cell = P.out = nullptr;
         P.species = P.off = nullptr;
         P.cap = 0;
@@ -90,11 +102,16 @@ extern "C" int ann_pair_compute(ann_ctx* ctx, int form, int new_list, int nlocal
         ANN_HIP(hipMalloc(&P.species, sizeof(int) * (size_t)nlocal));
         ANN_HIP(hipMalloc(&P.off, sizeof(int) * 2));
         ANN_HIP(hipMalloc(&P.out, sizeof(double) * (10 + 3 * (size_t)nlocal)));
+        ANN_HIP(hipHostMalloc((void**)&P.h_in, sizeof(double) * (3 * (size_t)nlocal + 9), 0));
+        ANN_HIP(hipHostMalloc((void**)&P.h_out, sizeof(double) * (10 + 3 * (size_t)nlocal), 0));
+        ANN_HIP(hipHostMalloc((void**)&P.h_ea, sizeof(float) * (size_t)nlocal, 0));
         P.cap = nlocal;
     }
     hipStream_t st = ctx->stream;
-    ANN_HIP(hipMemcpyAsync(P.pos, x, sizeof(double) * 3 * (size_t)nlocal, hipMemcpyHostToDevice, st));
-    ANN_HIP(hipMemcpyAsync(P.cell, cell, sizeof(double) * 9, hipMemcpyHostToDevice, st));
+    std::memcpy(P.h_in, x, sizeof(double) * 3 * (size_t)nlocal);
+    std::memcpy(P.h_in + 3 * (size_t)nlocal, cell, sizeof(double) * 9);
+    ANN_HIP(hipMemcpyAsync(P.pos, P.h_in, sizeof(double) * 3 * (size_t)nlocal, hipMemcpyHostToDevice, st));
+    ANN_HIP(hipMemcpyAsync(P.cell, P.h_in + 3 * (size_t)nlocal, sizeof(double) * 9, hipMemcpyHostToDevice, st));
     if (new_list) {
         P.have_list = false;
         P.hoff[0] = 0;
@@ -116,32 +133,48 @@ extern "C" int ann_pair_compute(ann_ctx* ctx, int form, int new_list, int nlocal
             if (numneigh[i] > 0 && !firstneigh[i]) return fail(ANN_ERR_ARG, "null neighbour row");
             off[i + 1] = off[i] + numneigh[i];
         }
+        // every ghost's owner and image once: the list names it many times
+        struct Ghost { int owner, n[3], state; };           // state 0 good, 1 no local owner, 2 no image of it
+        std::vector<Ghost> ghost(nghost);
+        for (int k = 0; k < nghost; ++k) {
+            Ghost& G = ghost[k];
+            G.owner = owner[k];
+            G.n[0] = G.n[1] = G.n[2] = 0;
+            G.state = G.owner < 0 || G.owner >= nlocal ? 1 : 0;
+            if (G.state) continue;
+            const size_t gx = 3 * ((size_t)nlocal + k), ox = 3 * (size_t)G.owner;
+            const double dx[3] = {x[gx] - x[ox], x[gx + 1] - x[ox + 1], x[gx + 2] - x[ox + 2]};
+            for (int t = 0; t < 3; ++t) {
+                const double fr = Ri[3 * t] * dx[0] + Ri[3 * t + 1] * dx[1] + Ri[3 * t + 2] * dx[2];
+                const double rn = std::nearbyint(fr);
+                if (!(std::fabs(fr - rn) <= 1e-6 * std::fmax(1.0, std::fabs(fr)))) { G.state = 2; break; }
+                G.n[t] = rn < -1e9 || rn > 1e9 ? 1 << 30 : (int)rn;
+            }
+        }
         idx.resize(off[nlocal]);
         img.resize(3 * (size_t)off[nlocal]);
-        for (int i = 0; i < nlocal; ++i)
+        for (int i = 0; i < nlocal; ++i) {
+            const int* row = firstneigh[i];
             for (int q = 0; q < numneigh[i]; ++q) {
-                const int j = firstneigh[i][q];
+                const int j = row[q];
                 if (j < 0 || j >= nall) return fail(ANN_ERR_ARG, "neighbour index outside the local and ghost atoms");
-                const int o = j < nlocal ? j : owner[j - nlocal];
-                if (o < 0 || o >= nlocal)
-                    return fail(ANN_ERR_ARG, "ghost " + std::to_string(j) + " has no local owner");
-                int n[3] = {0, 0, 0};
-                if (j >= nlocal) {
-                    const double dx[3] = {x[3 * (size_t)j] - x[3 * (size_t)o], x[3 * (size_t)j + 1] - x[3 * (size_t)o + 1],
-                                          x[3 * (size_t)j + 2] - x[3 * (size_t)o + 2]};
-                    for (int t = 0; t < 3; ++t) {
-                        const double fr = Ri[3 * t] * dx[0] + Ri[3 * t + 1] * dx[1] + Ri[3 * t + 2] * dx[2];
-                        const double rn = std::nearbyint(fr);
-                        if (!(std::fabs(fr - rn) <= 1e-6 * std::fmax(1.0, std::fabs(fr))))
-                            return fail(ANN_ERR_ARG, "ghost " + std::to_string(j) +
-                                                         " is not a lattice image of its owner");
-                        n[t] = (int)rn;
-                    }
-                }
                 const size_t s = (size_t)off[i] + q;
-                idx[s] = o;
-                for (int t = 0; t < 3; ++t) img[3 * s + t] = n[t];
+                int* n = &img[3 * s];
+                if (j < nlocal) {
+                    idx[s] = j;
+                    n[0] = n[1] = n[2] = 0;
+                    continue;
+                }
+                const Ghost& G = ghost[j - nlocal];
+                if (G.state == 1) return fail(ANN_ERR_ARG, "ghost " + std::to_string(j) + " has no local owner");
+                if (G.state == 2)
+                    return fail(ANN_ERR_ARG, "ghost " + std::to_string(j) + " is not a lattice image of its owner");
+                idx[s] = G.owner;
+                n[0] = G.n[0];
+                n[1] = G.n[1];
+                n[2] = G.n[2];
             }
+        }
         if ((r = ann_set_neighbors(ctx, off.data(), idx.data(), img.data(), rc)) != ANN_OK) return r;
         P.have_list = true;
         P.nlocal = nlocal;
@@ -154,11 +187,9 @@ extern "C" int ann_pair_compute(ann_ctx* ctx, int form, int new_list, int nlocal
     double* dF = P.out + 10;
     int r = ann_energy_forces(ctx, form, 1, dE, dF, virial ? dV : nullptr);
     if (r != ANN_OK) return r;
-    P.h_out.resize(10 + 3 * (size_t)nlocal);
-    ANN_HIP(hipMemcpyAsync(P.h_out.data(), P.out, sizeof(double) * P.h_out.size(), hipMemcpyDeviceToHost, st));
+    ANN_HIP(hipMemcpyAsync(P.h_out, P.out, sizeof(double) * (10 + 3 * (size_t)nlocal), hipMemcpyDeviceToHost, st));
     if (eatom) {
-        P.h_ea.resize(nlocal);
-        ANN_HIP(hipMemcpyAsync(P.h_ea.data(), ctx->d_Eatom, sizeof(float) * (size_t)nlocal, hipMemcpyDeviceToHost, st));
+        ANN_HIP(hipMemcpyAsync(P.h_ea, ctx->d_Eatom, sizeof(float) * (size_t)nlocal, hipMemcpyDeviceToHost, st));
     }
     ANN_HIP(hipStreamSynchronize(st));
     for (size_t q = 0; q < 3 * (size_t)nlocal; ++q) f[q] += P.h_out[10 + q];
@@ -166,7 +197,7 @@ extern "C" int ann_pair_compute(ann_ctx* ctx, int form, int new_list, int nlocal
     if (eatom)
         for (int i = 0; i < nlocal; ++i) eatom[i] += (double)P.h_ea[i] + ctx->hm.net[species[i]].evac;
     if (virial) {
-        const double* V = P.h_out.data() + 1;
+        const double* V = P.h_out + 1;
         virial[0] += V[0];
         virial[1] += V[4];
         virial[2] += V[8];

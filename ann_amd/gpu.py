@@ -404,16 +404,23 @@ class Engine:
         cell = np.ascontiguousarray(cell, dtype=np.float64)
         own = np.ascontiguousarray(owner, dtype=np.int32)
         nghost = len(x) - nlocal
-        rows = [np.ascontiguousarray(r, dtype=np.int32) for r in neigh] if neigh is not None else None
-        num = np.array([len(r) for r in rows], np.int32) if rows is not None else None
-        ptrs = (P_I * nlocal)(*[r.ctypes.data_as(P_I) for r in rows]) if rows is not None else None
+        num = rows = ptrs = None
+        if neigh is not None:
+            # one flat array and the address of every row in it
+            if len(neigh) != nlocal:
+                raise ValueError("pair_compute: one neighbour row per local atom")
+            num = np.fromiter(map(len, neigh), np.int32, nlocal)
+            rows = np.concatenate(neigh, dtype=np.int32, casting="unsafe") if nlocal else np.zeros(0, np.int32)
+            first = np.concatenate([[0], np.cumsum(num[:-1], dtype=np.int64)])
+            ptrs = (rows.ctypes.data + 4 * first).astype(np.uintp)
         f = np.zeros((nlocal, 3))
         e = C.c_double(0.0)
         ea = np.zeros(nlocal) if per_atom else None
         vir = np.zeros(6)
         _check(lib().ann_pair_compute(self.h, form, int(new_list), nlocal, nghost, x.ctypes.data_as(P_D),
                                       sp.ctypes.data_as(P_I), cell.ctypes.data_as(P_D), own.ctypes.data_as(P_I),
-                                      num.ctypes.data_as(P_I) if num is not None else None, ptrs,
+                                      num.ctypes.data_as(P_I) if num is not None else None,
+                                      C.c_void_p(ptrs.ctypes.data) if ptrs is not None else None,
                                       C.c_double(rc), f.ctypes.data_as(P_D), C.byref(e),
                                       ea.ctypes.data_as(P_D) if ea is not None else None, vir.ctypes.data_as(P_D)))
         return e.value, f, ea, vir
