@@ -59,7 +59,7 @@ struct SymmArgs {
     const float* u;
     float* v;
     float* Tout;              // moment form, G: store each atom's moments T here (or null)
-    const float* Tin;         // moment form, adjoint: moments of the same geometry (or null: recompute)
+    const float* Tin;         // moment form, adjoint and tangent: moments of the same geometry (or null: recompute)
     const float* rad_etal;    // rad_eta times sqrt(log2 e)
     int rad_gauss;            // every radial block is GAUSSIAN
     int nrad, nrs;            // widest radial block; its row stride in the adjoint's tables (odd)
@@ -1569,40 +1569,58 @@ constexpr int kGRegSpecies = 3;         // species with their sums in registers
 
 template <int Z>
 struct GShape {
-    static constexpr int NM = nharm(Z), NX = NM + kMaxUnionEta, NR = NX | 1;
+    static constexpr int NM = nharm(Z), NX = NM + kMaxUnionEta;
     static constexpr int NW = NX <= 8 ? 8 : (NX <= 16 ? 16 : (NX <= 32 ? 32 : kWave));   // lanes of one group
     static constexpr int NG = kWave / NW;
 };
 
 // float4 entries of the wavefront's LDS slice (layout at the top of g_atom)
-__host__ inline int g_units(int Z, int S, int NP, int nrad, int ldg, int rows) {
-    const int NM = nharm(Z), NR = (NM + kMaxUnionEta) | 1;
-    return kWave + S * NM + S + kWave / 2 + (S * nrad + 1) / 2 + rows * NR / 4 + ldg / 4 +
+__host__ inline int g_units(bool tan, int Z, int S, int NP, int nrad, int ldg, int rows) {
+    const int NM = nharm(Z), NX = NM + kMaxUnionEta, NR = (tan ? 2 * NX : NX) | 1, t = tan ? 2 : 1;
+    return t * kWave + t * S * NM + S + t * kWave / 2 + (S * nrad + 1) / 2 + rows * NR / 4 + ldg / 4 +
            (NP * kMaxUnionEta * (Z + 1) + 3) / 4;
 }
 
-template <int Z, int SR>
+// TAN: the tangent v = dG/dr . u along the atoms' displacements u, with the
+// moments T that the G kernel stored: the runs then sum
+// dT_b[u][f] = sum (w de_u/dr Y_f + e_u dY_f), w = r^ . (u_i - u_j), and the
+// contraction is its product rule.  Against the form that regroups the row in LDS
+// and sums the moments again, Li/P/S: 21,872 atoms 89 -> 64 us (rows 24 / 32 / 48 /
+// 64 at a time: 64.5 / 67.3 / 70.2 / 85.5), 5.5 k 32 -> 25 us.
+template <int Z, int SR, bool TAN>
 __device__ __forceinline__ void g_atom(const SymmArgs& A, const int i, float4* smem4) {
-    constexpr int NM = GShape<Z>::NM, NX = GShape<Z>::NX, NR = GShape<Z>::NR, NW = GShape<Z>::NW, NG = GShape<Z>::NG;
+    constexpr int NM = GShape<Z>::NM, NX = GShape<Z>::NX, NW = GShape<Z>::NW, NG = GShape<Z>::NG;
+    constexpr int NR = (TAN ? 2 * NX : NX) | 1;                 // functions and e_u (TAN: then their derivatives), odd
     constexpr int ZP = Z + 1, U4 = kMaxUnionEta, NB = SR > 0 ? SR : 1;
     const int lane = threadIdx.x % kWave;
     const DevModel& Mo = *A.dm;
     const int S = Mo.S, NP = Mo.NP, ldg = A.ldg, nrad = A.nrad;
     const int nrow = A.grows;                                   // function rows in LDS at a time (a multiple of 4)
     float4* ef = smem4;                                         // [64] width factors of the pass
-    float4* T = ef + kWave;                                     // [S][NM] moments, widths in the components
+    float4* fw = ef + (TAN ? kWave : 0);                        // [64] TAN: w de_u/dr
+    float4* T = fw + kWave;                                     // [S][NM] sums (moments or dT), widths in the components
     float4* D = T + S * NM;                                     // [S]
-    float2* rf = reinterpret_cast<float2*>(D + S);              // [64] distance, cutoff
-    float2* par = rf + kWave;                                   // [S][nrad] radial eta, rs
+    float4* Ts = D + S;                                         // [S][NM] TAN: stored moments
+    float2* rf = reinterpret_cast<float2*>(Ts + (TAN ? S * NM : 0));   // [64] distance, cutoff (TAN: also its derivative, w)
+    float2* par = rf + (TAN ? 2 : 1) * kWave;                   // [S][nrad] radial eta, rs
     float* rows = reinterpret_cast<float*>(par + ((S * nrad + 1) & ~1));   // [nrow][NR] functions, then e_u
     float* row = rows + nrow * NR;                              // [ldg]
     float* Am = row + ldg;                                      // [NP][U4][ZP]
     const int o0 = A.off[i], o1 = A.off[i + 1], a = A.species[i];
     float4 gn = make_float4(0.f, 0.f, 0.f, 0.f);
-    int bn = 0;
+    int bn = 0, jn = 0;
     if (o0 + lane < o1) {
         gn = A.geo[o0 + lane];
         bn = A.nsp[o0 + lane];
+        if (TAN) jn = A.nidx[o0 + lane];
+    }
+    float uix = 0.f, uiy = 0.f, uiz = 0.f;
+    if (TAN) {
+        uix = A.u[3 * (size_t)i];
+        uiy = A.u[3 * (size_t)i + 1];
+        uiz = A.u[3 * (size_t)i + 2];
+        const float4* gT = reinterpret_cast<const float4*>(A.Tin) + (size_t)i * S * NM;
+        for (int x = lane; x < S * NM; x += kWave) Ts[x] = gT[x];
     }
     if (SR == 0)
         for (int x = lane; x < S * NM + S; x += kWave) T[x] = make_float4(0.f, 0.f, 0.f, 0.f);   // T and D
@@ -1650,9 +1668,16 @@ __device__ __forceinline__ void g_atom(const SymmArgs& A, const int i, float4* s
         const float4 gq = gn;
         const bool keep = s < o1 && gq.w <= rc;
         const int key = keep ? bn : -1;
+        float tx = 0.f, ty = 0.f, tz = 0.f;
+        if (TAN && keep) {
+            tx = uix - A.u[3 * (size_t)jn];
+            ty = uiy - A.u[3 * (size_t)jn + 1];
+            tz = uiz - A.u[3 * (size_t)jn + 2];
+        }
         if (s + kWave < o1) {
             gn = A.geo[s + kWave];
             bn = A.nsp[s + kWave];
+            if (TAN) jn = A.nidx[s + kWave];
         }
         int pos = 0, cnt = 0;
         for (int b = 0; b < S; ++b) {
@@ -1660,19 +1685,35 @@ __device__ __forceinline__ void g_atom(const SymmArgs& A, const int i, float4* s
             if (key == b) pos = cnt + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0));
             cnt += __popcll(m);
         }
-        float y[NM], e[U4];
+        float y[NM], e[U4], dy[TAN ? NM : 1], d[U4];
         wave_sync();                                            // the previous pass's LDS reads are done
         if (keep) {
             const float r = gq.w, ir = __builtin_amdgcn_rcpf(r);   // 1 ulp
+            const float hx = gq.x * ir, hy = gq.y * ir, hz = gq.z * ir;
             float C[ZP], Sn[ZP], ql[qidx(Z, Z) + 1];
-            harm_factors<Z, float>(gq.x * ir, gq.y * ir, gq.z * ir, C, Sn, ql);
+            harm_factors<Z, float>(hx, hy, hz, C, Sn, ql);
             harm_values<Z, float>(C, Sn, ql, y);
+            float w = 0.0f;
+            if constexpr (TAN) {
+                w = hx * tx + hy * ty + hz * tz;
+                harm_along<Z, float>(C, Sn, ql, (tx - hx * w) * ir, (ty - hy * w) * ir, (tz - hz * w) * ir, dy);
+            }
             float fc, gc;
             cutoff_fg(Mo.cutoff, Mo.rc, Mo.rci, Mo.pirc, r, fc, gc);
 #pragma unroll
-            for (int u = 0; u < U4; ++u) e[u] = u < Mo.nunion[a] ? __expf(-Mo.uieta2[a][u] * r * r) * fc : 0.0f;
+            for (int u = 0; u < U4; ++u) {
+                const float k = Mo.uieta2[a][u], x = u < Mo.nunion[a] ? __expf(-k * r * r) : 0.0f;
+                e[u] = x * fc;
+                d[u] = x * (-2.0f * r * k * fc + gc) * w;       // TAN
+            }
             ef[pos] = make_float4(e[0], e[1], e[2], e[3]);
-            rf[pos] = make_float2(r, fc);
+            if constexpr (TAN) {
+                fw[pos] = make_float4(d[0], d[1], d[2], d[3]);
+                rf[2 * pos] = make_float2(r, fc);
+                rf[2 * pos + 1] = make_float2(gc, w);
+            } else {
+                rf[pos] = make_float2(r, fc);
+            }
         }
         // moments: rows of up to nrow entries at a time
         for (int c0 = 0; c0 < cnt; c0 += nrow) {
@@ -1683,13 +1724,26 @@ __device__ __forceinline__ void g_atom(const SymmArgs& A, const int i, float4* s
                 for (int f = 0; f < NM; ++f) w[f] = y[f];
 #pragma unroll
                 for (int u = 0; u < U4; ++u) w[NM + u] = e[u];
+                if constexpr (TAN) {
+#pragma unroll
+                    for (int f = 0; f < NM; ++f) w[NX + f] = dy[f];
+#pragma unroll
+                    for (int u = 0; u < U4; ++u) w[NX + NM + u] = d[u];
+                }
             }
             wave_sync();
             auto run = [&](int j0, int j1, float (&acc)[U4]) {
                 auto step = [&](const float* w, int J) {
                     const float v = w[al];
                     const float4 e4 = ef[J];
-                    acc[0] += e4.x * v; acc[1] += e4.y * v; acc[2] += e4.z * v; acc[3] += e4.w * v;
+                    if constexpr (TAN) {
+                        const float dv = w[NX + al];
+                        const float4 f4 = fw[J];
+                        acc[0] += f4.x * v + e4.x * dv; acc[1] += f4.y * v + e4.y * dv;
+                        acc[2] += f4.z * v + e4.z * dv; acc[3] += f4.w * v + e4.w * dv;
+                    } else {
+                        acc[0] += e4.x * v; acc[1] += e4.y * v; acc[2] += e4.z * v; acc[3] += e4.w * v;
+                    }
                 };
                 if (al < NX) {
                     int J = j0 + grp;
@@ -1733,16 +1787,24 @@ __device__ __forceinline__ void g_atom(const SymmArgs& A, const int i, float4* s
             if (A.rad_gauss) {
 #pragma unroll 4
                 for (int J = j0 + (lane >> sh); J < j1; J += nj) {
-                    const float2 v = rf[J];
+                    const float2 v = rf[TAN ? 2 * J : J];
                     const float x = t.x * (v.x - t.y);
-                    acc += __builtin_amdgcn_exp2f(-(x * x)) * v.y;
+                    const float ex = __builtin_amdgcn_exp2f(-(x * x));
+                    if constexpr (TAN) {
+                        // d/dr [e fc] = e (gc - 2 eta^2 (r - rs) fc); eta carries sqrt(log2 e)
+                        const float2 gw = rf[2 * J + 1];
+                        acc += ex * (gw.x - 1.3862943611198906f * (t.x * x) * v.y) * gw.y;
+                    } else {
+                        acc += ex * v.y;
+                    }
                 }
             } else {
                 for (int J = j0 + (lane >> sh); J < j1; J += nj) {
-                    const float2 v = rf[J];
-                    float g, d;
-                    radial_fd(rb.name, t.x, t.y, v.x, v.y, 0.0f, g, d);
-                    acc += g;
+                    const float2 v = rf[TAN ? 2 * J : J];
+                    const float2 gw = TAN ? rf[2 * J + 1] : make_float2(0.f, 0.f);
+                    float g, dr;
+                    radial_fd(rb.name, t.x, t.y, v.x, v.y, gw.x, g, dr);
+                    acc += TAN ? dr * gw.y : g;
                 }
             }
             return acc;
@@ -1774,7 +1836,7 @@ __device__ __forceinline__ void g_atom(const SymmArgs& A, const int i, float4* s
             }
         wave_sync();
     }
-    if (A.Tout) {
+    if (!TAN && A.Tout) {
         float4* out = reinterpret_cast<float4*>(A.Tout) + (size_t)i * S * NM;
         for (int x = lane; x < S * NM; x += kWave) out[x] = T[x];
     }
@@ -1793,7 +1855,13 @@ __device__ __forceinline__ void g_atom(const SymmArgs& A, const int i, float4* s
         for (int j = 0; j < 2 * Z + 1; ++j) {
             const int f = min(m * m + j, NM - 1);
             const float w = j <= 2 * m ? 1.0f : 0.0f;
-            v += (w * Tb[U4 * f]) * Tc[U4 * f];
+            if constexpr (TAN) {
+                const float* Sb = reinterpret_cast<const float*>(Ts + b * NM) + u;
+                const float* Sc = reinterpret_cast<const float*>(Ts + c * NM) + u;
+                v += w * (Tb[U4 * f] * Sc[U4 * f] + Sb[U4 * f] * Tc[U4 * f]);
+            } else {
+                v += (w * Tb[U4 * f]) * Tc[U4 * f];
+            }
         }
         if (b == c) v = 0.5f * (v - reinterpret_cast<const float*>(D + b)[u]);
         Am[x] = v;
@@ -1818,7 +1886,8 @@ __device__ __forceinline__ void g_atom(const SymmArgs& A, const int i, float4* s
         }
     }
     wave_sync();
-    for (int x = lane; x < ldg; x += kWave) A.G[(size_t)i * ldg + x] = row[x];
+    float* out = TAN ? A.v : A.G;
+    for (int x = lane; x < ldg; x += kWave) out[(size_t)i * ldg + x] = row[x];
 }
 
 // Grid dispatch: a block holds blockDim.x / 64 atoms (the "atoms per
@@ -1832,17 +1901,17 @@ __global__ __launch_bounds__(256) void k_moment(SymmArgs A) {
     moment_atom<MODE, Z>(A, i, smem_all + (size_t)wave * (A.smem_wave / 16));
 }
 
-// G: one atom per wavefront
-template <int Z, int SR>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_moment_g(SymmArgs A) {
+// G and the tangent with stored moments: one atom per wavefront
+template <int Z, int SR, bool TAN>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(Z <= 2 ? 5 : 4))) void k_moment_g(SymmArgs A) {
     extern __shared__ float4 smem_all[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int i = xcd_block(blockIdx.x, gridDim.x) * (blockDim.x / kWave) + wave;
     if (i >= A.N) return;
-    g_atom<Z, SR>(A, i, smem_all + (size_t)wave * (A.smem_wave / 16));
+    g_atom<Z, SR, TAN>(A, i, smem_all + (size_t)wave * (A.smem_wave / 16));
 }
 
-constexpr int kModeAdjT = 4;                                    // the stored-moment adjoint (adjoint_wave)
+constexpr int kModeAdjT = 4, kModeTanT = 5;                     // the stored-moment adjoint and tangent
 
 // Persistent dispatch (a separate kernel, so that the grid kernel keeps its
 // own register allocation): a grid sized to the resident capacity, every
@@ -1866,10 +1935,11 @@ __global__ __launch_bounds__(256) void k_moment_queue(SymmArgs A) {
         int nk = 0;
         if (lane == 0) nk = atomicAdd(ctr, 1);
         const int2 it = A.items[beg + k];
-        if constexpr (MODE == kModeAdjT || MODE == 0) {
+        if constexpr (MODE == kModeAdjT || MODE == 0 || MODE == kModeTanT) {
             const int ib = __builtin_amdgcn_readfirstlane(it.x), ie = ib + __builtin_amdgcn_readfirstlane(it.y);
             for (int a = ib; a < ie; a += A.atomsK) {
-                if constexpr (MODE == 0) g_atom<Z, SR>(A, a, smem4);
+                if constexpr (MODE == 0) g_atom<Z, SR, false>(A, a, smem4);
+                else if constexpr (MODE == kModeTanT) g_atom<Z, SR, true>(A, a, smem4);
                 else adjoint_wave<Z>(A, a, min(A.atomsK, ie - a), smem4);
                 wave_sync();                                    // the next atoms reuse the LDS slice
             }
@@ -2014,13 +2084,15 @@ static size_t fast_smem(const SymmArgs& A, int mode) {
 using MomentKernel = void (*)(SymmArgs);
 template <int MODE, int Z>
 static MomentKernel pick_kernel(bool queued, int S) {
-    if constexpr (MODE == 0) {
-        if (S <= kGRegSpecies) return queued ? k_moment_queue<0, Z, kGRegSpecies> : k_moment_g<Z, kGRegSpecies>;
-        return queued ? k_moment_queue<0, Z> : k_moment_g<Z, 0>;
+    if constexpr (MODE == 0 || MODE == kModeTanT) {
+        constexpr bool tan = MODE == kModeTanT;
+        if (S <= kGRegSpecies) return queued ? k_moment_queue<MODE, Z, kGRegSpecies> : k_moment_g<Z, kGRegSpecies, tan>;
+        return queued ? k_moment_queue<MODE, Z> : k_moment_g<Z, 0, tan>;
+    } else if constexpr (MODE == kModeAdjT) {
+        return queued ? k_moment_queue<MODE, Z> : k_adjoint<Z>;
+    } else {
+        return queued ? k_moment_queue<MODE, Z> : k_moment<MODE, Z>;
     }
-    if (queued) return k_moment_queue<MODE, Z>;
-    if constexpr (MODE == kModeAdjT) return k_adjoint<Z>;
-    else return k_moment<MODE, Z>;
 }
 template <int MODE>
 static MomentKernel moment_kernel(int z, bool queued, int S) {
@@ -2048,25 +2120,22 @@ static hipError_t run(ann_ctx* ctx, int form, SymmArgs A) {
         // fits (a forward call on a grown batch before any fused call skips it)
         const bool tfits = ctx->d_T && ctx->work_atoms >= A.N;
         if (MODE == 0 && tfits) A.Tout = ctx->d_T;
-        if (MODE == 1 && tfits && ctx->T_gen == ctx->gen) A.Tin = ctx->d_T;
-        const bool adjT = MODE == 1 && A.Tin;
+        if (MODE != 0 && tfits && ctx->T_gen == ctx->gen) A.Tin = ctx->d_T;
+        const bool adjT = MODE == 1 && A.Tin, tanT = MODE == 2 && A.Tin;
         size_t sw = (moment_smem(A, MODE, M.moment_z, M.S, M.NP) + 15) / 16 * 16;
-        if (adjT || MODE == 0) {
-            auto units = [&](int K) {
-                return MODE == 0 ? g_units(M.moment_z, M.S, M.NP, A.nrad, A.ldg, A.grows)
-                                 : adj_units(K, M.moment_z, M.S, M.NP, A.nrs, A.ldg);
-            };
-            A.atomsK = MODE == 0 ? 1 : adj_atoms(ctx);
-            // a pass's 64 rows at once where rows are short (degree <= 2) or where the
+        if (adjT) {
+            A.atomsK = adj_atoms(ctx);
+            if (adj_units(A.atomsK, M.moment_z, M.S, M.NP, A.nrs, A.ldg) > 1024) A.atomsK = 1;   // above 16 KiB
+            sw = 16 * (size_t)adj_units(A.atomsK, M.moment_z, M.S, M.NP, A.nrs, A.ldg);
+        } else if (MODE == 0 || tanT) {
+            // a pass's 64 rows at once where rows are short (G up to degree 2) or where the
             // chip holds every wavefront's slice all the same, else 32 (measured, 32 / 64
             // rows: 273,561 water atoms 735 / 1010 us, 12,288 43.8 / 53.3, 2,048 20.0 / 18.7,
             // 87,912 Li/P/S atoms of degree 2 157 / 152)
-            A.grows = kWave;
-            if (MODE == 0 && M.moment_z > 2 &&
-                (int64_t)A.N > (int64_t)ctx->num_cu * ((160 << 10) / (16 * g_units(M.moment_z, M.S, M.NP, A.nrad, A.ldg, kWave))))
-                A.grows = kWave / 2;
-            if (units(A.atomsK) > 1024) A.atomsK = 1;           // above 16 KiB one atom per wavefront
-            sw = 16 * (size_t)units(A.atomsK);
+            auto units = [&](int rows) { return g_units(tanT, M.moment_z, M.S, M.NP, A.nrad, A.ldg, rows); };
+            const bool fits = (int64_t)A.N <= (int64_t)ctx->num_cu * ((160 << 10) / (16 * units(kWave)));
+            A.grows = (MODE == 0 && M.moment_z <= 2) || fits ? kWave : (tanT && M.moment_z <= 2 ? 24 : kWave / 2);
+            sw = 16 * (size_t)units(A.grows);
         }
         int apb = ctx->tune_apb[MODE];
         while (apb > 1 && sw * apb > 65536) apb /= 2;          // dynamic LDS of one workgroup
@@ -2079,8 +2148,9 @@ static hipError_t run(ann_ctx* ctx, int form, SymmArgs A) {
             const hipError_t ei = ensure_items(ctx);
             if (ei != hipSuccess) return ei;
         }
-        MomentKernel kern = adjT ? moment_kernel<kModeAdjT>(M.moment_z, queued, M.S)
-                                 : moment_kernel<MODE>(M.moment_z, queued, M.S);
+        MomentKernel kern = adjT   ? moment_kernel<kModeAdjT>(M.moment_z, queued, M.S)
+                            : tanT ? moment_kernel<kModeTanT>(M.moment_z, queued, M.S)
+                                   : moment_kernel<MODE>(M.moment_z, queued, M.S);
         if (queued) {
             // persistent: enough workgroups for the most wavefronts a CU can hold
             // (32); those that find no room start later, find the queues empty
