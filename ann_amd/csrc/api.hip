@@ -206,7 +206,7 @@ static int upload_model(ann_ctx* ctx, const ann_model_desc* d) {
     M.rci = (float)(1.0 / d->rc);
     M.pirc = (float)(3.141592653589793 / d->rc);
     M.rad_gauss = 1;
-    std::vector<float> rrs, reta, retal, aeta, azeta, alam;
+    std::vector<float> rrs, reta, aeta, azeta, alam;
     std::vector<double> rrs64, reta64, aeta64, azeta64;   // the same tables in FP64 (FP64-evaluated inputs)
     ctx->rc64 = d->rc;
     // radial blocks
@@ -227,7 +227,6 @@ static int upload_model(ann_ctx* ctx, const ann_model_desc* d) {
             for (int m = 0; m < n; ++m) {
                 rrs.push_back((float)d->rad_rs[d->rad_off[t] + m]);
                 reta.push_back((float)d->rad_eta[d->rad_off[t] + m]);
-                retal.push_back((float)(d->rad_eta[d->rad_off[t] + m] * 1.2011224087864498));   // sqrt(log2 e)
                 rrs64.push_back(d->rad_rs[d->rad_off[t] + m]);
                 reta64.push_back(d->rad_eta[d->rad_off[t] + m]);
             }
@@ -469,7 +468,6 @@ static int upload_model(ann_ctx* ctx, const ann_model_desc* d) {
     };
     ANN_HIP(up(ctx->da.rad_rs, rrs));
     ANN_HIP(up(ctx->da.rad_eta, reta));
-    ANN_HIP(up(ctx->da.rad_etal, retal));
     ANN_HIP(up(ctx->da.ang_eta, aeta));
     ANN_HIP(up(ctx->da.ang_zeta, azeta));
     ANN_HIP(up(ctx->da.ang_lam, alam));
@@ -543,7 +541,7 @@ extern "C" int ann_destroy(ann_ctx* ctx) {
     if (!ctx) return ANN_OK;
     hipDeviceSynchronize();
     pair_free(ctx);
-    void* ptrs[] = {ctx->d_off_own, ctx->d_cells_own, ctx->d_species_own, ctx->dm, ctx->da.rad_rs, ctx->da.rad_eta, ctx->da.rad_etal, ctx->da.ang_eta, ctx->da.ang_zeta, ctx->da.ang_lam,
+    void* ptrs[] = {ctx->d_off_own, ctx->d_cells_own, ctx->d_species_own, ctx->dm, ctx->da.rad_rs, ctx->da.rad_eta, ctx->da.ang_eta, ctx->da.ang_zeta, ctx->da.ang_lam,
                     ctx->da.W, ctx->da.inpw, ctx->da.inpb, ctx->da.params, ctx->da.adam_m, ctx->da.adam_v,
                     ctx->d_struc_of, ctx->d_cellinfo, ctx->d_cellmat, ctx->d_bin_of, ctx->d_shift, ctx->d_bin_cnt,
                     ctx->d_bin_start, ctx->d_bin_atoms, ctx->d_keys, ctx->d_tab, ctx->d_cnt, ctx->d_flag, ctx->nl.off,

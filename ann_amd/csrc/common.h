@@ -111,7 +111,6 @@ struct PreItem {
 struct DevArrays {
     float* rad_rs = nullptr;
     float* rad_eta = nullptr;
-    float* rad_etal = nullptr;   // rad_eta times sqrt(log2 e)
     float* ang_eta = nullptr;
     float* ang_zeta = nullptr;
     float* ang_lam = nullptr;

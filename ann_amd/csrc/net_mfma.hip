@@ -385,15 +385,15 @@ __global__ __launch_bounds__(kNetWaves * kWave) void k_net_mfma(MfmaArgs A) {
     __syncthreads();
     // linear output neuron, and g_{L-1} = outw W_L . sigma'_{L-1} into the planes
     {
-        float z = 0.0f;
-        for (int m = osl; m < W; m += 16) {
-            const float w = m < ni ? WL[m] : 0.0f;
-            z += w * act[orow][m];
-            if (grad) put1(orow, m, m < ni ? D.outw * w * sdz[L - 2][orow][m] : 0.0f);
+        if (grad)
+            for (int m = osl; m < W; m += 16) put1(orow, m, m < ni ? D.outw * WL[m] * sdz[L - 2][orow][m] : 0.0f);
+        // one lane per atom, terms in order: atoms in like environments round alike, so
+        // the order of this sum shows in a structure's energy
+        if (tid < nrow) {
+            float z = A.W[D.boff[L - 1]];
+            for (int m = 0; m < ni; ++m) z += WL[m] * act[tid][m];
+            A.Eatom[A.perm[tl.y + tid]] = D.outb + D.outw * z;
         }
-#pragma unroll
-        for (int o = 8; o > 0; o >>= 1) z += __shfl_xor(z, o);
-        if (orow < nrow && osl == 0) A.Eatom[A.perm[tl.y + orow]] = D.outb + D.outw * (A.W[D.boff[L - 1]] + z);
     }
     if (!grad) return;
     for (int l = L - 2; l >= 1; --l) {

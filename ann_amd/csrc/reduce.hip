@@ -116,9 +116,11 @@ __global__ __launch_bounds__(256) void k_chunk_sums(const int* __restrict__ chun
         }
         if (qmask & 4) acc[10] += keatom[a];
     }
-    // wavefront butterflies, then the four wavefront partials in order
+    // wavefront butterflies of the quantities asked for, then the four wavefront
+    // partials in order
 #pragma unroll
     for (int q = 0; q < kSumQ; ++q) {
+        if (!(qmask & (q == 0 ? 1 : (q < 10 ? 2 : 4)))) continue;
         double v = acc[q];
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);

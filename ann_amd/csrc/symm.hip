@@ -60,7 +60,6 @@ struct SymmArgs {
     float* v;
     float* Tout;              // moment form, G: store each atom's moments T here (or null)
     const float* Tin;         // moment form, adjoint and tangent: moments of the same geometry (or null: recompute)
-    const float* rad_etal;    // rad_eta times sqrt(log2 e)
     int rad_gauss;            // every radial block is GAUSSIAN
     int nrad, nrs;            // widest radial block; its row stride in the adjoint's tables (odd)
     int grows;                // function rows in LDS of the G kernel
@@ -1365,8 +1364,8 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
 // Bound by vector issue: about 1,300 wave instructions per atom (water, two atoms
 // per wavefront) against 2,800 of the form with one LDS row per neighbour.
 // Measured against it: 1,048,576 atoms, list with a skin, 8.57 -> 3.15 ms;
-// 273,561 atoms 1285 -> 576 us; 12,288 atoms 54 -> 36 us; Li/P/S, 21,872 atoms,
-// 67 -> 37 us.
+// 273,561 atoms 1285 -> 554 us; 12,288 atoms 54 -> 36 us; Li/P/S, 21,872 atoms,
+// 67 -> 36 us.
 constexpr int kAdjAtoms = 2;
 
 // float4 entries of the wavefront's LDS slice (layout at the top of adjoint_wave)
@@ -1422,7 +1421,7 @@ __device__ __forceinline__ void adjoint_wave(const SymmArgs& A, const int i0, co
         const RadBlock rb = Mo.rad[spec(q) * S + b];
         float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
         if (m < rb.n) {
-            const float e = A.rad_gauss ? A.rad_etal[rb.par + m] : A.rad_eta[rb.par + m], g = row[q * ldg + rb.goff + m];
+            const float e = A.rad_eta[rb.par + m], g = row[q * ldg + rb.goff + m];
             t = make_float4(e, A.rad_rs[rb.par + m], g, g * e);
         }
         R[x] = t;
@@ -1471,7 +1470,15 @@ __device__ __forceinline__ void adjoint_wave(const SymmArgs& A, const int i0, co
         reinterpret_cast<float*>(dD)[x] = -0.5f * v;
     }
     wave_sync();
-    const float rc = Mo.rc;
+    const float rc = Mo.rc, rci = Mo.rci, pirc = Mo.pirc;
+    const int cut = Mo.cutoff;
+    // 1/eta^2 of the atoms' widths (0 past them: their dE/dT is 0), in scalars: a lane
+    // picks its atom's by a select instead of four loads per pass
+    float ke[kAdjAtoms][U4];
+#pragma unroll
+    for (int q = 0; q < kAdjAtoms; ++q)
+#pragma unroll
+        for (int u = 0; u < U4; ++u) ke[q][u] = Mo.uieta2[sp[q]][u];
     for (; s < s_end; s += kWave) {
         const float4 gq = gn;
         const int b = bn;
@@ -1488,21 +1495,21 @@ __device__ __forceinline__ void adjoint_wave(const SymmArgs& A, const int i0, co
             const float r = gq.w, ir = __builtin_amdgcn_rcpf(r);   // 1 ulp
             const float hx = gq.x * ir, hy = gq.y * ir, hz = gq.z * ir;
             float fc, gc;
-            cutoff_fg(Mo.cutoff, Mo.rc, Mo.rci, Mo.pirc, r, fc, gc);
+            cutoff_fg(cut, rc, rci, pirc, r, fc, gc);
             const int qb = q * S + b;
             const float4* Rq = R + qb * nrs;
             float amp;
             if (A.rad_gauss) {
-                // d/dr [e fc] = e (gc - 2 eta^2 (r - rs) fc); eta carries sqrt(log2 e)
+                // d/dr [e fc] = e (gc - 2 eta^2 (r - rs) fc)
                 float se = 0.0f, sx = 0.0f;
 #pragma unroll 4
                 for (int m = 0; m < A.nrad; ++m) {
                     const float4 t = Rq[m];
-                    const float x = t.x * (r - t.y), e = __builtin_amdgcn_exp2f(-(x * x));
+                    const float x = t.x * (r - t.y), e = __expf(-x * x);
                     se += t.z * e;
                     sx += t.w * (x * e);
                 }
-                amp = se * gc - 1.3862943611198906f * fc * sx;  // 2 / log2 e
+                amp = se * gc - 2.0f * fc * sx;
             } else {
                 const RadBlock rb = Mo.rad[a * S + b];
                 amp = 0.0f;
@@ -1516,7 +1523,9 @@ __device__ __forceinline__ void adjoint_wave(const SymmArgs& A, const int i0, co
             float e[U4], d[U4];
 #pragma unroll
             for (int u = 0; u < U4; ++u) {
-                const float k = Mo.uieta2[a][u];                // 0 past the centre's widths: their dE/dT is 0
+                float k = ke[0][u];
+#pragma unroll
+                for (int x = 1; x < kAdjAtoms; ++x) k = q == x ? ke[x][u] : k;
                 const float x = __expf(-k * r * r);
                 e[u] = x * fc;
                 d[u] = x * (-2.0f * r * k * fc + gc);
@@ -1629,7 +1638,7 @@ __device__ __forceinline__ void g_atom(const SymmArgs& A, const int i, float4* s
         const int m = x % nrad, b = x / nrad;
         const RadBlock rb = Mo.rad[a * S + b];
         float2 t = make_float2(0.f, 0.f);
-        if (m < rb.n) t = make_float2(A.rad_gauss ? A.rad_etal[rb.par + m] : A.rad_eta[rb.par + m], A.rad_rs[rb.par + m]);
+        if (m < rb.n) t = make_float2(A.rad_eta[rb.par + m], A.rad_rs[rb.par + m]);
         par[x] = t;
     }
     const float rc = Mo.rc;
@@ -1788,12 +1797,10 @@ __device__ __forceinline__ void g_atom(const SymmArgs& A, const int i, float4* s
 #pragma unroll 4
                 for (int J = j0 + (lane >> sh); J < j1; J += nj) {
                     const float2 v = rf[TAN ? 2 * J : J];
-                    const float x = t.x * (v.x - t.y);
-                    const float ex = __builtin_amdgcn_exp2f(-(x * x));
+                    const float x = t.x * (v.x - t.y), ex = __expf(-x * x);
                     if constexpr (TAN) {
-                        // d/dr [e fc] = e (gc - 2 eta^2 (r - rs) fc); eta carries sqrt(log2 e)
                         const float2 gw = rf[2 * J + 1];
-                        acc += ex * (gw.x - 1.3862943611198906f * (t.x * x) * v.y) * gw.y;
+                        acc += ex * (gw.x - 2.0f * (t.x * x) * v.y) * gw.y;
                     } else {
                         acc += ex * v.y;
                     }
@@ -2043,7 +2050,6 @@ static SymmArgs make_args(ann_ctx* ctx) {
     A.geo = ctx->nl.geo;
     A.nsp = ctx->nl.nsp;
     A.nidx = ctx->nl.idx;
-    A.rad_etal = ctx->da.rad_etal;
     A.rad_gauss = ctx->hm.rad_gauss;
     A.nrad = ctx->hm.nrad;
     A.nrs = A.nrad | 1;
