@@ -1110,6 +1110,12 @@ hipError_t neighbors_build(ann_ctx* ctx, double rc) {
         set_error("the previous neighbour list was not symmetric (reverse slot missing)");
         return hipErrorInvalidValue;
     }
+    // Rows that the search left out or cut short have no reverse slots: what the
+    // compaction beside this wait found missing there is no fault of a list
+    auto forget_rev = [&]() {
+        return spec_cap > 0 && flags[0] ? hipMemsetAsync(ctx->d_flag + 2, 0, sizeof(int), st) : hipSuccess;
+    };
+    HIPCHK(forget_rev());
     if (flags[0] & 8) {
         // bins with a search box too large to stage: one wavefront per centre atom
         ctx->nb_dirty = true;
@@ -1130,6 +1136,7 @@ hipError_t neighbors_build(ann_ctx* ctx, double rc) {
         flags[0] |= rb[0];
         flags[1] = std::max(flags[1], (int)rb[1]);
         total = rb[4];
+        if (flags[0] & ~8) HIPCHK(forget_rev());
     }
     if (flags[0] & 16) {
         ctx->nb_status = ANN_ERR_ARG;

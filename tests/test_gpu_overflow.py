@@ -1,0 +1,81 @@
+"""Neighbour lists of structures in which only part of the bins fit the staged
+search, bit for bit against the FP64 oracle's list: built, moved and built again
+on the same context, so that the fill that runs beside the wait for the list size
+meets rows the first search pass left out."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _model():
+    from ann_amd import configs
+    return configs.model_ar256()
+
+
+def _slab(L, height, fill, spacing, seed):
+    """Atoms on a jittered grid in the lower part of an L x L x height cell, a few above it."""
+    from ann_amd import configs
+    rng = np.random.default_rng(seed)
+    axes = [np.arange(int(x / spacing)) * spacing for x in (L, L, fill)]
+    pos = np.stack(np.meshgrid(*axes, indexing="ij"), -1).reshape(-1, 3)
+    pos = pos + rng.normal(0.0, 0.05 * spacing, size=pos.shape)
+    gas = rng.uniform([0, 0, fill], [L, L, height], size=(40, 3))
+    pos = rng.permutation(np.concatenate([pos, gas]))
+    return configs.single(pos, np.diag([L, L, height]), np.zeros(len(pos), np.int32))
+
+
+def _check(eng, pos, batch, orc, rc):
+    nl = eng.nlist()
+    ref = orc.nlist(pos, batch.cells[0].reshape(3, 3), batch.species, rc)
+    for k in ("off", "idx", "img", "rev"):
+        assert np.array_equal(nl[k], getattr(ref, k)), k
+
+
+# L, height, filled height, spacing, cutoff: a slab whose dense part overflows even the
+# smallest search box (atoms above it have short rows), one below and one above the
+# largest structure with rank tables; water-like slabs whose mean density admits
+# 2 x 2 x 2 bins that the dense part overflows
+CASES = [(11.0, 24.0, 11.0, 0.92, 4.0), (13.0, 24.0, 12.0, 0.875, 4.0), (40.0, 40.0, 28.0, 2.15, 7.5),
+         (50.0, 50.0, 30.0, 2.15, 8.0)]
+
+
+@pytest.mark.parametrize("L,height,fill,spacing,rc", CASES)
+def test_partly_overflowed_bins(oracle_mod, L, height, fill, spacing, rc):
+    import torch
+    from ann_amd.gpu import Engine
+    model, batch = _model(), _slab(L, height, fill, spacing, 70)
+    orc = oracle_mod.Oracle(model)
+    eng = Engine(model, "cuda:0")
+    eng.set_batch(batch)
+    rng = np.random.default_rng(71)
+    pos = batch.pos.copy()
+    for step in range(4):                       # the first build allocates, the others fill beside the wait
+        eng.neighbors(rc)
+        widest = eng.nlist_size()[1]
+        _check(eng, pos, batch, orc, rc)
+        pos = pos + rng.normal(0.0, 0.02, size=pos.shape)
+        eng.d_pos.copy_(torch.from_numpy(pos))
+    print(f"  {batch.ntotal} atoms, rc {rc}: widest row {widest}", flush=True)
+
+
+@pytest.mark.parametrize("n", [700, 2500])
+def test_refused_then_good(oracle_mod, n):
+    """A build refused for rows above the capacity leaves no fault behind for the next one."""
+    import torch
+    from ann_amd import configs
+    from ann_amd.gpu import AnnError, Engine
+    L, rc = (n / 0.1) ** (1.0 / 3.0), 5.0
+    pos = np.random.default_rng(72).uniform(0, L, size=(n, 3))
+    batch = configs.single(pos, np.eye(3) * L, np.zeros(n, np.int32))
+    orc = oracle_mod.Oracle(_model())
+    eng = Engine(_model(), "cuda:0")
+    eng.set_batch(batch)
+    eng.neighbors(rc)
+    for _ in range(2):
+        eng.d_pos.copy_(torch.from_numpy(pos * (3.0 / L)))      # every atom within rc of every other
+        with pytest.raises(AnnError):
+            eng.neighbors(rc)
+        eng.d_pos.copy_(torch.from_numpy(pos))
+        eng.neighbors(rc)
+        _check(eng, pos, batch, orc, rc)
