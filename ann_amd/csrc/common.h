@@ -144,8 +144,17 @@ struct NList {
     int64_t cap = 0;
 };
 
+// Image vectors in 10-bit fields, n + 512 modulo 1024: a value out of range stays in
+// its own field and never reaches a neighbouring one or the atom index above it.
 inline __host__ __device__ uint32_t pack_img(int n0, int n1, int n2) {
-    return ((uint32_t)(n0 + 512) << 20) | ((uint32_t)(n1 + 512) << 10) | (uint32_t)(n2 + 512);
+    return ((uint32_t)(n0 + 512) & 1023u) << 20 | ((uint32_t)(n1 + 512) & 1023u) << 10 | ((uint32_t)(n2 + 512) & 1023u);
+}
+// Packed difference of two packed images, every field modulo 1024 on its own (the
+// fields' top bits are set before the subtraction, so no borrow leaves a field,
+// and put right after it).  Bits 30 and 31 of a pass through.
+inline __host__ __device__ uint32_t img_minus(uint32_t a, uint32_t b) {
+    constexpr uint32_t top = 0x20080200u;
+    return ((a | top) - (b & ~top & 0x3fffffffu)) ^ ((a ^ b) & top);
 }
 inline __host__ __device__ void unpack_img(uint32_t p, int& n0, int& n1, int& n2) {
     n0 = (int)((p >> 20) & 1023) - 512;

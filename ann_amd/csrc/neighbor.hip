@@ -549,8 +549,9 @@ __global__ __launch_bounds__(kStageThreads) void k_search_bins(
         const uint64_t ki = ckey[qc];
         const int i = __builtin_amdgcn_readfirstlane((int)(ki >> 30));
         // the centre's packed image is -shift_i: taking it off a candidate's key
-        // leaves (j << 30 | packed n), field by field (each field carries a bias of 512)
-        const uint64_t koff = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(ki & 0x3fffffffu)) - pack_img(0, 0, 0);
+        // leaves (j << 30 | packed n).  Fields wrap one by one: shifts beyond +-511
+        // (a structure far from its cell) must not reach the index in the high bits
+        const uint32_t si = (uint32_t)__builtin_amdgcn_readfirstlane((int)(ki & 0x3fffffffu));
         uint64_t* dst = keys_out + (size_t)i * kMaxNeigh;
         int count = 0;
         for (int base = 0; base < total; base += kWave) {
@@ -562,7 +563,8 @@ __global__ __launch_bounds__(kStageThreads) void k_search_bins(
             bool ok = near && d2f < lo_thr && d2f > band;
             const uint64_t mnear = __ballot(near);
             if (mnear == 0) continue;
-            const uint64_t key = near ? ckey[q] - koff : 0ull;
+            const uint64_t kq = near ? ckey[q] : 0ull;
+            const uint64_t key = (kq & 0xffffffff00000000ull) | img_minus((uint32_t)kq, si);
             uint64_t mask = __ballot(ok);
             if (mask != mnear) {
                 if (near && !ok) {

@@ -79,3 +79,27 @@ def test_refused_then_good(oracle_mod, n):
         eng.d_pos.copy_(torch.from_numpy(pos))
         eng.neighbors(rc)
         _check(eng, pos, batch, orc, rc)
+
+
+@pytest.mark.parametrize("n,L,rc", [(2, 4.0, 6.0), (301, 16.0, 6.0), (2601, 32.0, 6.0)])
+def test_far_from_the_cell(oracle_mod, n, L, rc):
+    """A structure moved by whole cells, also past the +-511 that a packed image holds,
+    keeps its list.  Coordinates are multiples of 2^-10, so the move is exact."""
+    import torch
+    from ann_amd import configs
+    from ann_amd.gpu import Engine
+    rng = np.random.default_rng(73)
+    pos = rng.integers(0, int(L * 1024), size=(n, 3)) / 1024.0
+    batch = configs.single(pos, np.eye(3) * L, np.zeros(n, np.int32))
+    eng = Engine(_model(), "cuda:0")
+    eng.set_batch(batch)
+    eng.neighbors(rc)
+    _check(eng, pos, batch, oracle_mod.Oracle(_model()), rc)
+    home = eng.nlist()
+    for k in (511, -511, 512, -512, -513, 1000, -1024, 5000):
+        for axis in ((1, 0, 0), (0, 1, 0), (0, 0, 1), (1, 1, 1)):
+            eng.d_pos.copy_(torch.from_numpy(pos + np.array(axis) * (k * L)))
+            eng.neighbors(rc)
+            away = eng.nlist()
+            for q in ("off", "idx", "img", "rev", "geo"):
+                assert np.array_equal(away[q], home[q]), (k, axis, q)
