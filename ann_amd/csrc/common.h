@@ -261,6 +261,7 @@ struct ann_ctx {
     double grid_rc = 0;
     int grid_nbins = 0, grid_nsb = 0;  // bins and staged-search super-bins
     int grid_maxbins = 0;              // bins of the structure with the most
+    bool nb_split = false;            // super-bins overflowed in the last build: their bins are searched beside them
     bool pos_ref_valid = false;       // d_pos_ref holds the positions of the last build
     int* d_bin_atoms = nullptr;
     int bin_cap = 0;

@@ -292,9 +292,11 @@ __global__ __launch_bounds__(64) void k_search(
 // to kBuckets atoms in the box's index range, else 2^sh neighbouring indices), then
 // each candidate's rank among its bucket's few members; a block that meets a wide
 // index range still sorts, with longer buckets.
-// Boxes with more than kStageCap candidates or kStageImages images are flagged and
-// left to k_search.  Each block writes the overflow mark (0 or 1) of each of its
-// centre bins exactly once per build, so the marks need no clearing between builds.
+// Boxes with more than kStageCap candidates or kStageImages images are flagged: the
+// bins of a super-bin are searched one by one by the SPLIT instance (one block per
+// marked bin), bins that do not fit either are left to k_search.  Each block writes
+// the overflow mark (0 or 1) of each of its centre bins exactly once per build, so
+// the marks need no clearing between builds.
 // Bound by vector issue: about 25 instructions per 64 candidates and centre, and
 // the staging.  Against one sort per row, us: 1,048,576 atoms (rc 6.5, super-bins
 // now within the capacity) 5767 -> 1579, 273,561 atoms 621 -> 263, 87,912 Li/P/S
@@ -303,6 +305,7 @@ constexpr int kStageCap = 1280;
 constexpr int kStageImages = 216;
 constexpr int kStageThreads = 512;
 constexpr int kBuckets = 1024;
+constexpr int kOvfBin = 8, kOvfSuper = 32;                  // build flags: a bin's or a super-bin's box did not fit
 constexpr int kStageWaves = kStageThreads / kWave;
 constexpr int kStageIt = (kStageCap + kStageThreads - 1) / kStageThreads;
 static_assert(kBuckets == 2 * kStageThreads, "the bucket scan gives every thread two buckets");
@@ -315,10 +318,12 @@ __device__ __forceinline__ int wrap_bin(int u, int nb, int& m) {
     return u;
 }
 
+template <bool SPLIT>
 __global__ __launch_bounds__(kStageThreads) void k_search_bins(
     const CellInfo* __restrict__ ci, const double* __restrict__ cells, const int* __restrict__ bin_struc,
     const int* __restrict__ bin_start, const double4* __restrict__ rec, const double* __restrict__ pos, double rc2,
-    uint64_t* __restrict__ keys_out, int* __restrict__ cnt_out, int* __restrict__ flag, int* __restrict__ bin_ovf) {
+    uint64_t* __restrict__ keys_out, int* __restrict__ cnt_out, int* __restrict__ flag, int* __restrict__ bin_ovf,
+    const int* __restrict__ bin_atoms, const int* __restrict__ sof) {
     __shared__ int im_first[kStageImages];
     __shared__ int im_m[kStageImages];
     __shared__ int im_pre[kStageImages + 1];
@@ -332,13 +337,16 @@ __global__ __launch_bounds__(kStageThreads) void k_search_bins(
     uint64_t* sk = reinterpret_cast<uint64_t*>(cf);         // (j << 32 | image number) by bucket, until the ranks are known
     const int g = xcd_block(blockIdx.x, gridDim.x), t = threadIdx.x;
     const int lane = t % kWave, wave = t / kWave;
-    const int s = bin_struc[g];                             // structure of this super-bin
+    if (SPLIT && (!bin_ovf[g] || bin_start[g] == bin_start[g + 1])) return;
+    const int s = SPLIT ? sof[bin_atoms[bin_start[g]]] : bin_struc[g];   // structure of this bin or super-bin
     const CellInfo c = ci[s];
+    if (SPLIT && c.sb == 1) return;                         // a single bin's box did not fit: left to k_search
     const double* R = cells + 9 * s;
-    const int gi = g - c.sboff;
-    const int B0 = gi / (c.nsb[1] * c.nsb[2]), B1 = (gi / c.nsb[2]) % c.nsb[1], B2 = gi % c.nsb[2];
-    const int lo0 = c.sb * B0, lo1 = c.sb * B1, lo2 = c.sb * B2;
-    const int n0b = min(c.sb, c.nb[0] - lo0), n1b = min(c.sb, c.nb[1] - lo1), n2b = min(c.sb, c.nb[2] - lo2);
+    const int gi = SPLIT ? g - c.boff : g - c.sboff, sb = SPLIT ? 1 : c.sb;
+    const int w1 = SPLIT ? c.nb[1] : c.nsb[1], w2 = SPLIT ? c.nb[2] : c.nsb[2];
+    const int B0 = gi / (w1 * w2), B1 = (gi / w2) % w1, B2 = gi % w2;
+    const int lo0 = sb * B0, lo1 = sb * B1, lo2 = sb * B2;
+    const int n0b = min(sb, c.nb[0] - lo0), n1b = min(sb, c.nb[1] - lo1), n2b = min(sb, c.nb[2] - lo2);
     const int ncb = n0b * n1b * n2b;
     const int e0 = n0b + 2 * c.k[0], e1 = n1b + 2 * c.k[1], e2 = n2b + 2 * c.k[2];
     const int nimg = e0 * e1 * e2;
@@ -370,7 +378,7 @@ __global__ __launch_bounds__(kStageThreads) void k_search_bins(
     if (nimg > kStageImages) {
         __syncthreads();
         if (t < ncb) bin_ovf[cen_bin[t]] = 1;
-        if (t == 0) atomicOr(flag, 8);
+        if (t == 0) atomicOr(flag, sb > 1 ? kOvfSuper : kOvfBin);
         return;
     }
     if (t < nimg) {
@@ -412,7 +420,7 @@ __global__ __launch_bounds__(kStageThreads) void k_search_bins(
     }
     if (total > kStageCap) {
         if (t < ncb) bin_ovf[cen_bin[t]] = 1;
-        if (t == 0) atomicOr(flag, 8);
+        if (t == 0) atomicOr(flag, sb > 1 ? kOvfSuper : kOvfBin);
         return;
     }
     {
@@ -1085,10 +1093,25 @@ hipError_t neighbors_build(ann_ctx* ctx, double rc) {
     }
     {
         Launch L(ctx, "nb_search");
-        k_search_bins<<<ctx->grid_nsb, kStageThreads, 0, st>>>(dci, ctx->d_cells, ctx->d_bin_struc, ctx->d_bin_start,
+        k_search_bins<false><<<ctx->grid_nsb, kStageThreads, 0, st>>>(dci, ctx->d_cells, ctx->d_bin_struc, ctx->d_bin_start,
                                                       ctx->d_binrec, ctx->d_pos, rc * rc, ctx->d_keys, ctx->d_cnt,
-                                                      ctx->d_flag, ctx->d_bin_ovf);
+                                                      ctx->d_flag, ctx->d_bin_ovf, ctx->d_bin_atoms, ctx->d_struc_of);
     }
+    // Super-bins are chosen on a structure's mean density; where its dense part (a
+    // slab, a droplet) does not fit them, their bins are searched one by one.  A
+    // context that met this in its last build launches that pass at once instead of
+    // after the wait.  Whole builds, us, against leaving such bins to k_search: 4,212
+    // atoms 153 -> 86, 33,696 atoms 504 -> 218, 57,132 atoms 1746 -> 632 (a loop over
+    // the bins inside the block that found them costs every search registers: 1,048,576
+    // uniform atoms 1.57 -> 2.66 ms).
+    auto search_split = [&]() {
+        Launch L(ctx, "nb_search_split");
+        k_search_bins<true><<<nbins, kStageThreads, 0, st>>>(dci, ctx->d_cells, ctx->d_bin_struc, ctx->d_bin_start,
+                                                             ctx->d_binrec, ctx->d_pos, rc * rc, ctx->d_keys, ctx->d_cnt,
+                                                             ctx->d_flag, ctx->d_bin_ovf, ctx->d_bin_atoms, ctx->d_struc_of);
+    };
+    const bool ahead = ctx->nb_split;
+    if (ahead) search_split();
     HIPCHK(hipGetLastError());
     NList& nl = ctx->nl;
     // Offsets, then flags, pair count and a completion marker to pinned host
@@ -1112,15 +1135,18 @@ hipError_t neighbors_build(ann_ctx* ctx, double rc) {
         set_error("the previous neighbour list was not symmetric (reverse slot missing)");
         return hipErrorInvalidValue;
     }
+    ctx->nb_split = flags[0] & kOvfSuper;
+    const bool behind = ctx->nb_split && !ahead;
     // Rows that the search left out or cut short have no reverse slots: what the
     // compaction beside this wait found missing there is no fault of a list
     auto forget_rev = [&]() {
-        return spec_cap > 0 && flags[0] ? hipMemsetAsync(ctx->d_flag + 2, 0, sizeof(int), st) : hipSuccess;
+        return spec_cap > 0 ? hipMemsetAsync(ctx->d_flag + 2, 0, sizeof(int), st) : hipSuccess;
     };
-    HIPCHK(forget_rev());
-    if (flags[0] & 8) {
-        // bins with a search box too large to stage: one wavefront per centre atom
+    if (behind || (flags[0] & ~kOvfSuper)) HIPCHK(forget_rev());
+    if (behind || (flags[0] & kOvfBin)) {
         ctx->nb_dirty = true;
+        if (behind) search_split();
+        // bins with a search box too large to stage: one wavefront per centre atom
         {
             Launch L(ctx, "nb_search_wide");
             k_search<<<N, 64, 0, st>>>(N, ctx->d_pos, ctx->d_struc_of, dci, ctx->d_cells, ctx->d_bin_of,
@@ -1138,7 +1164,7 @@ hipError_t neighbors_build(ann_ctx* ctx, double rc) {
         flags[0] |= rb[0];
         flags[1] = std::max(flags[1], (int)rb[1]);
         total = rb[4];
-        if (flags[0] & ~8) HIPCHK(forget_rev());
+        if (flags[0] & ~(kOvfBin | kOvfSuper)) HIPCHK(forget_rev());
     }
     if (flags[0] & 16) {
         ctx->nb_status = ANN_ERR_ARG;

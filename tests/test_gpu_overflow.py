@@ -36,12 +36,12 @@ def _check(eng, pos, batch, orc, rc):
 # smallest search box (atoms above it have short rows), one below and one above the
 # largest structure with rank tables; water-like slabs whose mean density admits
 # 2 x 2 x 2 bins that the dense part overflows
-CASES = [(11.0, 24.0, 11.0, 0.92, 4.0), (13.0, 24.0, 12.0, 0.875, 4.0), (40.0, 40.0, 28.0, 2.15, 7.5),
-         (50.0, 50.0, 30.0, 2.15, 8.0)]
+CASES = [(11.0, 24.0, 10.5, 0.875, 4.0, 4), (13.0, 24.0, 12.0, 0.875, 4.0, 4), (40.0, 40.0, 28.0, 2.15, 7.5, 1),
+         (50.0, 50.0, 30.0, 2.15, 8.0, 1)]
 
 
-@pytest.mark.parametrize("L,height,fill,spacing,rc", CASES)
-def test_partly_overflowed_bins(oracle_mod, L, height, fill, spacing, rc):
+@pytest.mark.parametrize("L,height,fill,spacing,rc,wide", CASES)
+def test_partly_overflowed_bins(oracle_mod, L, height, fill, spacing, rc, wide):
     import torch
     from ann_amd.gpu import Engine
     model, batch = _model(), _slab(L, height, fill, spacing, 70)
@@ -50,30 +50,36 @@ def test_partly_overflowed_bins(oracle_mod, L, height, fill, spacing, rc):
     eng.set_batch(batch)
     rng = np.random.default_rng(71)
     pos = batch.pos.copy()
+    eng.profile(True)
     for step in range(4):                       # the first build allocates, the others fill beside the wait
         eng.neighbors(rc)
         widest = eng.nlist_size()[1]
         _check(eng, pos, batch, orc, rc)
         pos = pos + rng.normal(0.0, 0.02, size=pos.shape)
         eng.d_pos.copy_(torch.from_numpy(pos))
+    # 2 x 2 x 2 bins that do not fit are searched one by one, after the first build without a second pass
+    assert eng.profile_get("nb_search_wide")[1] == wide
+    assert eng.profile_get("nb_search_split")[1] == (4 if wide == 1 else 0)
     print(f"  {batch.ntotal} atoms, rc {rc}: widest row {widest}", flush=True)
 
 
-@pytest.mark.parametrize("n", [700, 2500])
+@pytest.mark.parametrize("n", [1900, 2600])
 def test_refused_then_good(oracle_mod, n):
     """A build refused for rows above the capacity leaves no fault behind for the next one."""
     import torch
     from ann_amd import configs
     from ann_amd.gpu import AnnError, Engine
-    L, rc = (n / 0.1) ** (1.0 / 3.0), 5.0
+    L, rc = (n / 0.57) ** (1.0 / 3.0), 5.0
     pos = np.random.default_rng(72).uniform(0, L, size=(n, 3))
+    bad = pos.copy()
+    bad[-560:] = L / 2 + (pos[-560:] - L / 2) * (2.0 / L)       # 560 atoms within rc of each other, fewer pairs in all
     batch = configs.single(pos, np.eye(3) * L, np.zeros(n, np.int32))
     orc = oracle_mod.Oracle(_model())
     eng = Engine(_model(), "cuda:0")
     eng.set_batch(batch)
     eng.neighbors(rc)
     for _ in range(2):
-        eng.d_pos.copy_(torch.from_numpy(pos * (3.0 / L)))      # every atom within rc of every other
+        eng.d_pos.copy_(torch.from_numpy(bad))
         with pytest.raises(AnnError):
             eng.neighbors(rc)
         eng.d_pos.copy_(torch.from_numpy(pos))
