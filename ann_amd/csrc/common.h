@@ -261,6 +261,7 @@ struct ann_ctx {
     double grid_rc = 0;
     int grid_nbins = 0, grid_nsb = 0;  // bins and staged-search super-bins
     int grid_maxbins = 0;              // bins of the structure with the most
+    bool grid_tab = false;            // rank tables pay for most pairs of the batch
     bool nb_split = false;            // super-bins overflowed in the last build: their bins are searched beside them
     bool pos_ref_valid = false;       // d_pos_ref holds the positions of the last build
     int* d_bin_atoms = nullptr;
@@ -286,7 +287,7 @@ struct ann_ctx {
     int64_t keys_cap = 0;
     uint64_t* d_tab = nullptr;        // rank tables of the rows (structures of at most 2048 atoms), tab_words each
     int64_t tab_cap = 0;
-    int tab_words = 0;                // 0: the batch has a larger structure
+    int tab_words = 0;                // 0: no tables (a larger structure, or they do not pay)
     // work buffers
     float* d_G = nullptr;
     float* d_dEdG = nullptr;

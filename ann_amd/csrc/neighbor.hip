@@ -947,10 +947,24 @@ static hipError_t grid_setup(ann_ctx* ctx, double rc) {
     // 12.0 us against 21.8 in super-bins; 2,048 bins and more lose by it, 12,288
     // atoms 64.5 against 29.2)
     const bool few = nbins <= 2 * ctx->num_cu;
+    // rank tables pay in structures of 64 atoms or more (below, rows are short and the
+    // table is one more thing to write) whose rows rarely hold several images of a
+    // partner (the images that the table's bits leave out are walked one by one): the
+    // cutoff sphere at most 0.85 of the cell.  Fill and reverse slots together, us,
+    // search / tables: 20,000 structures of 4 atoms 69 / 81, 4,096 of 16 65 / 71, 1,024
+    // sparse ones of 64 67.5 / 67.5, 512 of 200 198 / 121; dense cells by sphere / cell:
+    // 2.9 150 / 371, 1.4 136 / 184, 0.93 107 / 113, 0.80 125 / 115, 0.70 144 / 134
+    double tab_pairs = 0.0, all_pairs = 0.0;                // in proportion to the pairs expected
     for (int s = 0; s < S; ++s) {
         CellInfo& c = info[s];
+        const double* r = &cells[9 * s];
+        const double vol = std::fabs(r[0] * (r[4] * r[8] - r[5] * r[7]) - r[1] * (r[3] * r[8] - r[5] * r[6]) +
+                                     r[2] * (r[3] * r[7] - r[4] * r[6]));
+        const int n = ctx->atom_off[s + 1] - ctx->atom_off[s];
+        all_pairs += (double)n * n / vol;
+        if (n >= 64 && 4.18879 * rc * rc * rc <= 0.85 * vol) tab_pairs += (double)n * n / vol;
         // when the enlarged search box still fits
-        const double per_bin = (double)(ctx->atom_off[s + 1] - ctx->atom_off[s]) / c.nbins;
+        const double per_bin = (double)n / c.nbins;
         const double box2 = (double)(std::min(2, c.nb[0]) + 2 * c.k[0]) * (std::min(2, c.nb[1]) + 2 * c.k[1]) *
                             (std::min(2, c.nb[2]) + 2 * c.k[2]);
         c.sb = (ctx->tune_sb != 1 && !few && box2 * per_bin <= 0.8 * kStageCap && box2 <= kStageImages) ? 2 : 1;
@@ -983,6 +997,7 @@ static hipError_t grid_setup(ann_ctx* ctx, double rc) {
     ctx->grid_valid = true;
     ctx->grid_rc = rc;
     ctx->grid_nbins = nbins;
+    ctx->grid_tab = 2.0 * tab_pairs >= all_pairs;           // most pairs are in such structures
     ctx->grid_maxbins = 0;
     for (const CellInfo& c : info) ctx->grid_maxbins = std::max(ctx->grid_maxbins, c.nbins);
     ctx->grid_nsb = (int)bin_struc.size();
@@ -1019,8 +1034,8 @@ static void launch_compact(ann_ctx* ctx, int cap) {
     const int N = ctx->natoms;
     hipStream_t st = ctx->stream;
     NList& nl = ctx->nl;
-    // rank tables where every structure fits one (8 bytes per 32 atoms and row);
-    // larger structures search their partners' rows
+    // rank tables where every structure fits one (8 bytes per 32 atoms and row) and
+    // they pay (grid_setup); else the partners' rows are searched
     const bool tab = ctx->tab_words > 0;
     {
         Launch L(ctx, "nb_compact");
@@ -1052,7 +1067,7 @@ hipError_t neighbors_build(ann_ctx* ctx, double rc) {
     ctx->tab_words = 0;
     int most = 0;                               // atoms of the largest structure
     for (int s = 0; s < ctx->nstruc; ++s) most = std::max(most, ctx->atom_off[s + 1] - ctx->atom_off[s]);
-    if (most <= kTabAtoms) {
+    if (most <= kTabAtoms && ctx->grid_tab) {
         ctx->tab_words = (most + 31) / 32;
         HIPCHK(grow(ctx->d_tab, ctx->tab_cap, (int64_t)N * ctx->tab_words));
     }

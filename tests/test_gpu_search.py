@@ -71,3 +71,20 @@ def test_nonfinite_then_good(oracle_mod):
     eng.set_batch(batch)
     eng.neighbors(5.0)
     _check(eng, batch, oracle_mod.Oracle(model), 5.0)
+
+
+# atoms, box, cutoff, copies around the rule for rank tables: structures of 63 and 64
+# atoms, the cutoff sphere 0.84 and 0.86 of the cell, small cells with many images of
+# a partner; and a batch whose pairs are half in either kind
+@pytest.mark.parametrize("n,L,rc,copies", [(63, 12.0, 6.0, 4), (64, 12.0, 6.0, 4), (64, (905.0 / 0.84) ** (1 / 3), 6.0, 3),
+                                           (64, (905.0 / 0.86) ** (1 / 3), 6.0, 3), (32, 6.8, 6.0, 4), (96, 9.9, 6.0, 3)])
+def test_rank_table_rule(oracle_mod, n, L, rc, copies):
+    from ann_amd.configs import Batch
+    from ann_amd.gpu import Engine
+    eng, orc = Engine(_model(), "cuda:0"), oracle_mod.Oracle(_model())
+    same = Batch.concat([_gas(n, L, 80 + c) for c in range(copies)])
+    mixed = Batch.concat([same, _gas(200, 14.0, 90), _gas(3, 9.0, 91)])
+    for batch in (same, mixed, same):
+        eng.set_batch(batch)
+        eng.neighbors(rc)
+        _check(eng, batch, orc, rc)
