@@ -116,24 +116,30 @@ __global__ void k_fill_bins(int N, const int* __restrict__ bin_of, const int* __
 // fill (three launches) in batches of such structures: E+F of one water box 82.4 ->
 // 76.4 us, of 64 boxes 185 -> 173 us, energies of 512 Li/P/S cells 496 -> 464 us
 // (with the two-barrier scan of the row offsets).
+// T threads take structures of up to 4 T atoms and bins.  Blocks of one wavefront
+// where structures are many (kSBinMany on) and small, else blocks of eight: us, eight
+// wavefronts / one, 500 structures of 192 atoms 8.3 / 11.1, 1,500 14.1 / 14.1, 3,000
+// 21.9 / 19.1; of four atoms 1,500 8.9 / 6.7, 20,000 62 / 17.
 constexpr int kSBinThreads = 512;
-constexpr int kSBinAtoms = 2048;            // largest structure (atoms, bins) of this path
-constexpr int kSBinIt = kSBinAtoms / kSBinThreads;
+constexpr int kSBinIt = 4;
+constexpr int kSBinAtoms = kSBinIt * kSBinThreads;   // largest structure (atoms, bins) of this path
+constexpr int kSBinMany = 1536;
 
-__global__ __launch_bounds__(kSBinThreads) void k_bin_struc(
+template <int T>
+__global__ __launch_bounds__(T) void k_bin_struc(
     int nstruc, const int* __restrict__ aoff, const double* __restrict__ pos, const int* __restrict__ sof,
     const CellInfo* __restrict__ ci, const double* __restrict__ rinv, int* __restrict__ bin_of, int* __restrict__ shift,
     int* __restrict__ bin_start, int* __restrict__ bin_atoms, double4* __restrict__ rec, int* __restrict__ flag) {
-    __shared__ int cnt[kSBinAtoms];
-    __shared__ int wsum[kSBinThreads / kWave];
+    __shared__ int cnt[kSBinIt * T];
+    __shared__ int wsum[T / kWave];
     const int s = blockIdx.x, t = threadIdx.x, lane = t % kWave, w = t / kWave;
     const int a0 = aoff[s], n = aoff[s + 1] - a0, nb = ci[s].nbins, boff = ci[s].boff;
-    for (int q = t; q < kSBinAtoms; q += kSBinThreads) cnt[q] = 0;
+    for (int q = t; q < kSBinIt * T; q += T) cnt[q] = 0;
     __syncthreads();
     int g[kSBinIt], slot[kSBinIt];
 #pragma unroll
     for (int r = 0; r < kSBinIt; ++r) {
-        const int a = t + r * kSBinThreads;
+        const int a = t + r * T;
         g[r] = -1;
         slot[r] = 0;
         if (a < n) {
@@ -161,7 +167,7 @@ __global__ __launch_bounds__(kSBinThreads) void k_bin_struc(
     __syncthreads();
     int run = inc - sum;
 #pragma unroll
-    for (int k = 0; k < kSBinThreads / kWave; ++k) run += k < w ? wsum[k] : 0;
+    for (int k = 0; k < T / kWave; ++k) run += k < w ? wsum[k] : 0;
 #pragma unroll
     for (int r = 0; r < kSBinIt; ++r) {
         const int q = kSBinIt * t + r;
@@ -174,7 +180,7 @@ __global__ __launch_bounds__(kSBinThreads) void k_bin_struc(
 #pragma unroll
     for (int r = 0; r < kSBinIt; ++r)
         if (g[r] >= 0) {
-            const int i = a0 + t + r * kSBinThreads, at = a0 + cnt[g[r]] + slot[r];
+            const int i = a0 + t + r * T, at = a0 + cnt[g[r]] + slot[r];
             bin_atoms[at] = i;
             rec[at] = bin_record(i, pos, shift);
         }
@@ -1089,10 +1095,10 @@ hipError_t neighbors_build(ann_ctx* ctx, double rc) {
         if (most <= kSBinAtoms && ctx->grid_maxbins <= kSBinAtoms) {
             // one launch instead of three where every structure fits a block
             Launch L(ctx, "nb_bin");
-            k_bin_struc<<<ctx->nstruc, kSBinThreads, 0, st>>>(ctx->nstruc, ctx->d_atom_off, ctx->d_pos, ctx->d_struc_of, dci,
-                                                              ctx->d_cellmat, ctx->d_bin_of, ctx->d_shift,
-                                                              ctx->d_bin_start, ctx->d_bin_atoms, ctx->d_binrec,
-                                                              ctx->d_flag);
+            const bool wave = ctx->nstruc >= kSBinMany && std::max(most, ctx->grid_maxbins) <= kSBinIt * kWave;
+            (wave ? k_bin_struc<kWave> : k_bin_struc<kSBinThreads>)<<<ctx->nstruc, wave ? kWave : kSBinThreads, 0, st>>>(
+                ctx->nstruc, ctx->d_atom_off, ctx->d_pos, ctx->d_struc_of, dci, ctx->d_cellmat, ctx->d_bin_of, ctx->d_shift,
+                ctx->d_bin_start, ctx->d_bin_atoms, ctx->d_binrec, ctx->d_flag);
         } else {
         {
             Launch L(ctx, "nb_bin");

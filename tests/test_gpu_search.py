@@ -88,3 +88,17 @@ def test_rank_table_rule(oracle_mod, n, L, rc, copies):
         eng.set_batch(batch)
         eng.neighbors(rc)
         _check(eng, batch, orc, rc)
+
+
+# the largest structure among many: up to 256 atoms and 216 bins a structure is binned
+# by one wavefront, 257 atoms or 343 bins take eight
+@pytest.mark.parametrize("n,L", [(2, 9.0), (255, 20.0), (256, 20.0), (257, 20.0), (200, 21.5)])
+def test_many_structures(oracle_mod, n, L):
+    from ann_amd.configs import Batch
+    from ann_amd.gpu import Engine
+    eng, orc = Engine(_model(), "cuda:0"), oracle_mod.Oracle(_model())
+    batch = Batch.concat([_gas(1 + c % 5, 8.0 + 0.5 * (c % 3), 100 + c) for c in range(1540)] + [_gas(n, L, 99)])
+    for _ in range(2):
+        eng.set_batch(batch)
+        eng.neighbors(6.0)
+        _check(eng, batch, orc, 6.0)
