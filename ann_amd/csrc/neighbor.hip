@@ -295,9 +295,10 @@ __global__ __launch_bounds__(64) void k_search(
 // straight to the centre's row.  One sort of the box replaces a sort of every row,
 // which was two thirds of the instructions per centre.
 // The sort is a counting sort by bucket of the atom index (one atom per bucket up
-// to kBuckets atoms in the box's index range, else 2^sh neighbouring indices), then
-// each candidate's rank among its bucket's few members; a block that meets a wide
-// index range still sorts, with longer buckets.
+// to kBuckets atoms in the box's index range, else 2^sh neighbouring indices; few
+// atoms, which then have many images each, take several buckets per atom), then each
+// candidate's rank among its bucket's few members; a block that meets a wide index
+// range still sorts, with longer buckets.
 // Boxes with more than kStageCap candidates or kStageImages images are flagged: the
 // bins of a super-bin are searched one by one by the SPLIT instance (one block per
 // marked bin), bins that do not fit either are left to k_search.  Each block writes
@@ -314,6 +315,8 @@ constexpr int kBuckets = 1024;
 constexpr int kOvfBin = 8, kOvfSuper = 32;                  // build flags: a bin's or a super-bin's box did not fit
 constexpr int kStageWaves = kStageThreads / kWave;
 constexpr int kStageIt = (kStageCap + kStageThreads - 1) / kStageThreads;
+constexpr int kImageBits = 8;
+static_assert(kStageImages <= 1 << kImageBits, "image numbers in kImageBits");
 static_assert(kBuckets == 2 * kStageThreads, "the bucket scan gives every thread two buckets");
 
 // the image and wrapped index of unwrapped bin u (|u| is a few cells at most)
@@ -484,17 +487,18 @@ __global__ __launch_bounds__(kStageThreads) void k_search_bins(
             atomicMax(&s_jmax, jhi);
         }
         __syncthreads();
-        // buckets of 2^sh atom indices
+        // buckets of 2^sh atom indices, or 2^ib buckets per index split by image number
         const int jmin = s_jmin, range = s_jmax - jmin;
-        int sh = 0;
+        int sh = 0, ib = 0;
         while ((range >> sh) >= kBuckets) ++sh;
+        while (ib < kImageBits && ((range + 1) << (ib + 1)) <= kBuckets) ++ib;
         int bk[kStageIt], slot[kStageIt];
 #pragma unroll
         for (int r = 0; r < kStageIt; ++r) {
             bk[r] = 0;
             slot[r] = 0;
             if (src[r] < 0) continue;
-            bk[r] = ((int)(jd[r] >> 32) - jmin) >> sh;
+            bk[r] = (((int)(jd[r] >> 32) - jmin) >> sh) << ib | iq[r] >> (kImageBits - ib);
             slot[r] = atomicAdd(&bucket[bk[r]], 1);
         }
         __syncthreads();
