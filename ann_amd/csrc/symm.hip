@@ -1564,17 +1564,21 @@ __global__ __launch_bounds__(256) void k_adjoint(SymmArgs A) {
 // get none.  Then lanes over functions sum each species' run: moments
 // T_b[u][f] = sum e_u Y_f with the four widths in registers (lanes NM .. NM + 3
 // read e_u in place of a function, which gives D_b[u] = sum e_u^2), radial
-// functions with lanes over (entry, function).  With up to SR species every sum
-// stays in registers until the row ends (SR = 0: any number, added up in LDS
-// after every run).  LDS holds one pass, not one row per neighbour, so it does not
-// grow with the widest row.
+// functions with lanes over (entry, function).  Every sum stays
+// in registers until the row ends, for three species or for all eight.  LDS holds
+// one pass, not one row per neighbour, so it does not grow with the widest row.
 // Bound by vector issue, about 1,650 wave instructions' worth of time per water
 // atom.  Against the form that regroups the whole row by species in LDS first
 // (one row of 36 bytes per neighbour), us: 1,048,576 atoms with a skin 5119 ->
 // 4037, 273,561 atoms 820 -> 735, 12,288 atoms 47.4 -> 43.8, 87,912 Li/P/S atoms
 // 200 -> 152, 5.5 k 27.0 -> 18.1.  Two atoms per wavefront: 923 on the 273,561
-// atoms, sums added up in LDS after every run: 829.
+// atoms, sums added up in LDS after every run: 829.  More species, 100,000 atoms, us,
+// whole row regrouped / sums in LDS / in registers: four (degree 4) 557 / 534 / 481,
+// five (degree 2) 402 / 440 / 387, eight (degree 2) 767 / 847 / 743; tangent with
+// stored moments, LDS / registers: 1073 / 997, 653 / 624, 1212 / 1094 (its eight-species
+// instances at one wavefront per SIMD less, or their sums spill: 1061, 688, 1219).
 constexpr int kGRegSpecies = 3;         // species with their sums in registers
+constexpr int kGRegMany = kMaxSpecies;  // of the instances for more species
 
 template <int Z>
 struct GShape {
@@ -1600,7 +1604,7 @@ template <int Z, int SR, bool TAN>
 __device__ __forceinline__ void g_atom(const SymmArgs& A, const int i, float4* smem4) {
     constexpr int NM = GShape<Z>::NM, NX = GShape<Z>::NX, NW = GShape<Z>::NW, NG = GShape<Z>::NG;
     constexpr int NR = (TAN ? 2 * NX : NX) | 1;                 // functions and e_u (TAN: then their derivatives), odd
-    constexpr int ZP = Z + 1, U4 = kMaxUnionEta, NB = SR > 0 ? SR : 1;
+    constexpr int ZP = Z + 1, U4 = kMaxUnionEta;
     const int lane = threadIdx.x % kWave;
     const DevModel& Mo = *A.dm;
     const int S = Mo.S, NP = Mo.NP, ldg = A.ldg, nrad = A.nrad;
@@ -1631,8 +1635,6 @@ __device__ __forceinline__ void g_atom(const SymmArgs& A, const int i, float4* s
         const float4* gT = reinterpret_cast<const float4*>(A.Tin) + (size_t)i * S * NM;
         for (int x = lane; x < S * NM; x += kWave) Ts[x] = gT[x];
     }
-    if (SR == 0)
-        for (int x = lane; x < S * NM + S; x += kWave) T[x] = make_float4(0.f, 0.f, 0.f, 0.f);   // T and D
     for (int x = lane; x < ldg; x += kWave) row[x] = 0.0f;
     for (int x = lane; x < S * nrad; x += kWave) {
         const int m = x % nrad, b = x / nrad;
@@ -1643,31 +1645,27 @@ __device__ __forceinline__ void g_atom(const SymmArgs& A, const int i, float4* s
     }
     const float rc = Mo.rc;
     const int al = lane % NW, grp = lane / NW;
-    float mom[NB][U4], rad[NB];
+    float mom[SR][U4], rad[SR];
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
+    for (int b = 0; b < SR; ++b) {
         rad[b] = 0.0f;
 #pragma unroll
         for (int u = 0; u < U4; ++u) mom[b][u] = 0.0f;
     }
-    // the groups of lanes meet, then the sums of species b go to LDS (added: SR = 0)
+    // the groups of lanes meet, then the sums of species b go to LDS
     auto put_moments = [&](int b, float (&acc)[U4]) {
 #pragma unroll
         for (int bit = NW; bit < kWave; bit <<= 1)
 #pragma unroll
             for (int u = 0; u < U4; ++u) acc[u] += __shfl_xor(acc[u], bit);
         if (lane < NM) {
-            float4 t = SR == 0 ? T[b * NM + lane] : make_float4(0.f, 0.f, 0.f, 0.f);
-            t.x += acc[0]; t.y += acc[1]; t.z += acc[2]; t.w += acc[3];
-            T[b * NM + lane] = t;
+            T[b * NM + lane] = make_float4(acc[0], acc[1], acc[2], acc[3]);
         } else if (lane < NX) {                                 // lane NM + u: sum of e_u e_u
             const int u = lane - NM;
-            const float v = u == 0 ? acc[0] : (u == 1 ? acc[1] : (u == 2 ? acc[2] : acc[3]));
-            float* d = reinterpret_cast<float*>(D + b) + u;
-            *d = SR == 0 ? *d + v : v;
+            reinterpret_cast<float*>(D + b)[u] = u == 0 ? acc[0] : (u == 1 ? acc[1] : (u == 2 ? acc[2] : acc[3]));
         }
     };
-    auto put_radial = [&](int b, const RadBlock& rb, float acc) {
+    auto put_radial = [&](const RadBlock& rb, float acc) {
         const int W = rb.n <= 8 ? 8 : (rb.n <= 16 ? 16 : 32);
         for (int bit = W; bit < kWave; bit <<= 1) acc += __shfl_xor(acc, bit);
         if (lane < rb.n) row[rb.goff + lane] += acc;
@@ -1768,23 +1766,12 @@ __device__ __forceinline__ void g_atom(const SymmArgs& A, const int i, float4* s
                 }
             };
             int s0 = 0;
-            if constexpr (SR > 0) {
 #pragma unroll
-                for (int b = 0; b < SR; ++b) {
-                    const int n = __popcll(__ballot(key == b));
-                    run(max(s0, c0), min(s0 + n, c0 + nrow), mom[b]);
-                    s0 += n;
-                }
-            } else {
-                for (int b = 0; b < S; ++b) {
-                    const int n = __popcll(__ballot(key == b));
-                    const int j0 = max(s0, c0), j1 = min(s0 + n, c0 + nrow);
-                    s0 += n;
-                    if (j0 >= j1) continue;
-                    float acc[U4] = {0.f, 0.f, 0.f, 0.f};
-                    run(j0, j1, acc);
-                    put_moments(b, acc);
-                }
+            for (int b = 0; b < SR; ++b) {
+                if (SR > kGRegSpecies && b >= S) break;
+                const int n = __popcll(__ballot(key == b));
+                run(max(s0, c0), min(s0 + n, c0 + nrow), mom[b]);
+                s0 += n;
             }
         }
         // radial: lanes over (entry, function) of every species' run
@@ -1817,32 +1804,22 @@ __device__ __forceinline__ void g_atom(const SymmArgs& A, const int i, float4* s
             return acc;
         };
         int s0 = 0;
-        if constexpr (SR > 0) {
 #pragma unroll
-            for (int b = 0; b < SR; ++b) {
-                const int n = __popcll(__ballot(key == b));
-                if (n > 0) rad[b] += radial(b, Mo.rad[a * S + b], s0, s0 + n);
-                s0 += n;
-            }
-        } else {
-            for (int b = 0; b < S; ++b) {
-                const int n = __popcll(__ballot(key == b));
-                const RadBlock rb = Mo.rad[a * S + b];
-                if (n > 0 && rb.n > 0) put_radial(b, rb, radial(b, rb, s0, s0 + n));
-                s0 += n;
-            }
+        for (int b = 0; b < SR; ++b) {
+            if (SR > kGRegSpecies && b >= S) break;
+            const int n = __popcll(__ballot(key == b));
+            if (n > 0) rad[b] += radial(b, Mo.rad[a * S + b], s0, s0 + n);
+            s0 += n;
         }
     }
     wave_sync();
-    if constexpr (SR > 0) {
 #pragma unroll
-        for (int b = 0; b < SR; ++b)
-            if (b < S) {
-                put_moments(b, mom[b]);
-                put_radial(b, Mo.rad[a * S + b], rad[b]);
-            }
-        wave_sync();
-    }
+    for (int b = 0; b < SR; ++b)
+        if (b < S) {
+            put_moments(b, mom[b]);
+            put_radial(Mo.rad[a * S + b], rad[b]);
+        }
+    wave_sync();
     if (!TAN && A.Tout) {
         float4* out = reinterpret_cast<float4*>(A.Tout) + (size_t)i * S * NM;
         for (int x = lane; x < S * NM; x += kWave) out[x] = T[x];
@@ -1910,7 +1887,8 @@ __global__ __launch_bounds__(256) void k_moment(SymmArgs A) {
 
 // G and the tangent with stored moments: one atom per wavefront
 template <int Z, int SR, bool TAN>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(Z <= 2 ? 5 : 4))) void k_moment_g(SymmArgs A) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
+    (Z <= 2 ? 5 : 4) - (TAN && SR > kGRegSpecies && Z != 3 ? 1 : 0)))) void k_moment_g(SymmArgs A) {
     extern __shared__ float4 smem_all[];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int i = xcd_block(blockIdx.x, gridDim.x) * (blockDim.x / kWave) + wave;
@@ -2093,7 +2071,7 @@ static MomentKernel pick_kernel(bool queued, int S) {
     if constexpr (MODE == 0 || MODE == kModeTanT) {
         constexpr bool tan = MODE == kModeTanT;
         if (S <= kGRegSpecies) return queued ? k_moment_queue<MODE, Z, kGRegSpecies> : k_moment_g<Z, kGRegSpecies, tan>;
-        return queued ? k_moment_queue<MODE, Z> : k_moment_g<Z, 0, tan>;
+        return queued ? k_moment_queue<MODE, Z, kGRegMany> : k_moment_g<Z, kGRegMany, tan>;
     } else if constexpr (MODE == kModeAdjT) {
         return queued ? k_moment_queue<MODE, Z> : k_adjoint<Z>;
     } else {
