@@ -2119,6 +2119,7 @@ static hipError_t run(ann_ctx* ctx, int form, SymmArgs A) {
             auto units = [&](int rows) { return g_units(tanT, M.moment_z, M.S, M.NP, A.nrad, A.ldg, rows); };
             const bool fits = (int64_t)A.N <= (int64_t)ctx->num_cu * ((160 << 10) / (16 * units(kWave)));
             A.grows = (MODE == 0 && M.moment_z <= 2) || fits ? kWave : (tanT && M.moment_z <= 2 ? 24 : kWave / 2);
+            A.grows = std::min(A.grows, A.maxn);                // no more than the widest row has (a multiple of 4)
             sw = 16 * (size_t)units(A.grows);
         }
         int apb = ctx->tune_apb[MODE];

@@ -87,3 +87,36 @@ def test_many_species(oracle_mod, S, z, nr):
         print(f"  S {S} z {z} queue {queue}: E {eE:.1e} F {eF:.1e} V {eV:.1e} G {eG:.1e} G64 {eG64:.1e} "
               f"tangent {eT:.1e} {eT0:.1e}", flush=True)
         assert eE <= 1e-6 and eF <= 1e-5 and eV <= 1e-5 and eG <= 2e-5 and eG64 <= 1e-10 and eT <= 1e-5 and eT0 <= 1e-5
+
+
+# widest rows around the function rows held in LDS at a time (4, 8, 24, 32)
+@pytest.mark.parametrize("z", [2, 4])
+@pytest.mark.parametrize("n", [1, 4, 5, 6, 9, 25, 26, 33, 34])
+def test_short_rows(oracle_mod, n, z):
+    """n atoms within one cutoff of each other (rows of n - 1), twice, and a lone atom."""
+    import torch
+    from ann_amd import configs
+    from ann_amd.configs import Batch
+    from ann_amd.gpu import FAST, Engine
+    rng = np.random.default_rng(500 + n)
+    g = np.stack(np.meshgrid(*[np.arange(4)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    def one(k):
+        p = g[rng.permutation(64)[:k]] * 1.1 + rng.normal(0.0, 0.08, size=(k, 3))
+        return configs.single(p, np.eye(3) * 30.0, rng.integers(0, 4, k).astype(np.int32))
+    batch = Batch.concat([one(n), one(1), one(n)])
+    model = _model(4, z, 8)
+    orc, eng = oracle_mod.Oracle(model), Engine(model, "cuda:0")
+    eng.set_batch(batch)
+    eng.neighbors()
+    assert eng.nlist_size()[1] == n - 1
+    u = rng.normal(size=(batch.ntotal, 3))
+    eng.energy_forces(FAST)
+    v = eng.tangent(torch.tensor(u, device="cuda:0"), FAST).cpu().numpy()
+    G = eng.symm(FAST).cpu().numpy().astype(np.float64)
+    for k in range(batch.nstruc):
+        pos, cell, sp = batch.struc(k)
+        s = slice(batch.atom_off[k], batch.atom_off[k + 1])
+        Go, vr = orc.symm(pos, cell, sp), orc.tangent(pos, cell, sp, u[s])
+        m = Go.shape[1]
+        assert np.max(np.abs(G[s, :m] - Go)) <= 2e-5 * max(np.abs(Go).max(), 1e-30)
+        assert np.linalg.norm(v[s, :m] - vr) <= 1e-5 * np.linalg.norm(vr)
