@@ -714,6 +714,7 @@ extern "C" int ann_set_batch(ann_ctx* ctx, const ann_batch* b) {
     ctx->have_nlist = false;
     ctx->grid_valid = false;
     ctx->gen++;
+    ctx->geo_gen++;
     ctx->G_valid = false;
     ctx->rank_valid = false;
     ctx->perm_valid = false;
@@ -773,6 +774,7 @@ extern "C" int ann_neighbors(ann_ctx* ctx, double rc) {
     ctx->nl_rc = r;
     ctx->pos_ref_valid = false;   // the skin reference is taken by the next MD step
     ctx->gen++;
+    ctx->geo_gen++;
     return ANN_OK;
 }
 
@@ -789,6 +791,7 @@ extern "C" int ann_set_neighbors(ann_ctx* ctx, const int* off, const int* idx, c
     ctx->nl_rc = rc;
     ctx->pos_ref_valid = false;
     ctx->gen++;
+    ctx->geo_gen++;
     return ANN_OK;
 }
 
@@ -799,6 +802,7 @@ extern "C" int ann_refresh_geometry(ann_ctx* ctx) {
     if (e != hipSuccess) return fail(ANN_ERR_HIP, std::string("refresh_geometry: ") + hipGetErrorString(e));
     ctx->G_valid = false;
     ctx->gen++;
+    ctx->geo_gen++;
     return ANN_OK;
 }
 
@@ -810,6 +814,7 @@ extern "C" int ann_wrap_positions(ann_ctx* ctx) {
     ctx->have_nlist = false;      // image vectors of the old list refer to the unwrapped positions
     ctx->G_valid = false;
     ctx->gen++;
+    ctx->geo_gen++;
     return ANN_OK;
 }
 
@@ -1101,6 +1106,7 @@ extern "C" int ann_md_step(ann_ctx* ctx, int form, double dt, const double* mass
     RET_HIP(refresh_geometry(ctx), "refresh_geometry");
     ctx->G_valid = false;
     ctx->gen++;
+    ctx->geo_gen++;
     RET_HIP(network_rows(ctx, form, ctx->d_G), "symm_fwd");
     RET_HIP(net_fwd(ctx, form, ctx->d_G, ctx->d_Eatom, ctx->d_dEdG, true), "net_fwd");
     RET_HIP(symm_bwd(ctx, form, ctx->d_dEdG, ctx->d_P), "symm_bwd");
@@ -1331,6 +1337,7 @@ extern "C" int ann_autotune(ann_ctx* ctx, int form) {
     ctx->G_valid = false;
     ctx->pos_ref_valid = false;
     ctx->gen++;
+    ctx->geo_gen++;
     return ANN_OK;
 }
 

@@ -325,9 +325,10 @@ struct ann_ctx {
     hipStream_t gstream = nullptr;    // private non-blocking stream the graph is captured on and replayed
     hipEvent_t gev[2] = {nullptr, nullptr};
     hipGraphExec_t gexec = nullptr;
-    uint64_t gen = 0;                 // bumped whenever positions, the list or the batch change
+    uint64_t gen = 0;                 // bumped whenever anything changes that a captured training step bakes in
+    uint64_t geo_gen = 0;             // bumped whenever positions, the list or the batch change
     float* d_T = nullptr;             // moment form: per-atom moments T of the last G evaluation
-    uint64_t T_gen = ~0ull;           // gen at which d_T was written (~0: never)
+    uint64_t T_gen = ~0ull;           // geo_gen at which d_T was written (~0: never)
     bool ef_graph_on = false, ef_warm = false;   // E+F graph: enabled, one eager call done
     hipGraphExec_t ef_exec = nullptr;
     std::vector<uint64_t> ef_key;               // what the captured E+F kernels depend on

@@ -494,7 +494,7 @@ hipError_t network_rows(ann_ctx* ctx, int form, float* G) {
     if (ctx->npre > 0 && ctx->npre == ctx->nin_total) {
         float* T = (ctx->d_T && ctx->work_atoms >= ctx->natoms) ? ctx->d_T : nullptr;
         const hipError_t e = precise_inputs(ctx, G, nullptr, T);
-        ctx->T_gen = (e == hipSuccess && T && ctx->hm.moment_z > 0) ? ctx->gen : ~0ull;
+        ctx->T_gen = (e == hipSuccess && T && ctx->hm.moment_z > 0) ? ctx->geo_gen : ~0ull;
         return e;
     }
     const hipError_t e = symm_fwd(ctx, form, G);

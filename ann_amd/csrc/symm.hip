@@ -2104,7 +2104,7 @@ static hipError_t run(ann_ctx* ctx, int form, SymmArgs A) {
         // fits (a forward call on a grown batch before any fused call skips it)
         const bool tfits = ctx->d_T && ctx->work_atoms >= A.N;
         if (MODE == 0 && tfits) A.Tout = ctx->d_T;
-        if (MODE != 0 && tfits && ctx->T_gen == ctx->gen) A.Tin = ctx->d_T;
+        if (MODE != 0 && tfits && ctx->T_gen == ctx->geo_gen) A.Tin = ctx->d_T;
         const bool adjT = MODE == 1 && A.Tin, tanT = MODE == 2 && A.Tin;
         size_t sw = (moment_smem(A, MODE, M.moment_z, M.S, M.NP) + 15) / 16 * 16;
         if (adjT) {
@@ -2149,7 +2149,7 @@ static hipError_t run(ann_ctx* ctx, int form, SymmArgs A) {
             k_queue_reset<<<1, 64, 0, ctx->stream>>>(ctx->d_queue);
         }
         kern<<<grid, block, sm, ctx->stream>>>(A);
-        if (MODE == 0) ctx->T_gen = A.Tout ? ctx->gen : ~0ull;
+        if (MODE == 0) ctx->T_gen = A.Tout ? ctx->geo_gen : ~0ull;
         return hipGetLastError();
     }
     if (fast) {

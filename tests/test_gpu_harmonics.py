@@ -78,3 +78,32 @@ def test_every_degree_bound(oracle_mod, nspecies, z):
         eT = max(eT, float(np.linalg.norm(v[off[k]:off[k + 1], :n] - vr) / np.linalg.norm(vr)))
     print(f"  S {nspecies} z {z}: E {eE:.1e} F {eF:.1e} V {eV:.1e} G {eG:.1e} G64 {eG64:.1e} tangent {eT:.1e}", flush=True)
     assert eE <= 1e-6 and eF <= 1e-5 and eV <= 1e-5 and eG <= 2e-5 and eG64 <= 1e-10 and eT <= 1e-5
+
+
+def test_moments_kept_by_calls_that_move_nothing(oracle_mod):
+    """The loss, the structure weights and the tuning leave the stored moments in use
+    (the adjoint is then the same bits); new geometry does not."""
+    import torch
+    from ann_amd import configs
+    from ann_amd.gpu import FAST, Engine
+    model, batch = configs.model_lips(), configs.batch_lips(3, seed=43)
+    eng = Engine(model, "cuda:0")
+    eng.set_batch(batch)
+    eng.neighbors()
+    eng.energy_forces(FAST)
+    rng = np.random.default_rng(46)
+    dE = torch.from_numpy(rng.normal(size=(batch.ntotal, eng.ldg)).astype(np.float32)).cuda()
+    u = torch.from_numpy(rng.normal(size=(batch.ntotal, 3))).cuda()
+    P, v = eng.symm_bwd(dE).clone(), eng.tangent(u).clone()
+    w = torch.ones(batch.nstruc, dtype=torch.float64, device="cuda:0")
+    for call in (lambda: eng.set_loss("HUBER", 0.5), lambda: eng.set_struc_weights(w, w),
+                 lambda: eng.set_tuning([4, 4, 1, 0, 0])):
+        call()
+        assert torch.equal(eng.symm_bwd(dE), P) and torch.equal(eng.tangent(u), v)
+    eng.d_pos += 0.01 * u
+    eng.refresh_geometry()
+    P0, v0 = eng.symm_bwd(dE).clone(), eng.tangent(u).clone()   # sums the moments itself
+    assert float((P0 - P).norm()) > 1e-4 * float(P.norm())      # the old moments would give nearly the old values
+    eng.energy_forces(FAST)
+    for a, b in ((eng.symm_bwd(dE), P0), (eng.tangent(u), v0)):
+        assert float((a.double() - b.double()).norm()) <= 1e-5 * float(b.double().norm())
