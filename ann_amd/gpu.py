@@ -84,6 +84,30 @@ def _ptr(t: Optional[torch.Tensor]):
     return C.c_void_p(t.data_ptr()) if t is not None else C.c_void_p(0)
 
 
+def _flat_rows(neigh, nlocal: int):
+    """(row lengths, one flat int32 array, the address of every row in it) of nlocal
+    neighbour rows, any iterable of integer arrays or sequences."""
+    rows = list(neigh)
+    if len(rows) != nlocal:
+        raise ValueError("pair_compute: one neighbour row per local atom")
+    flat = None
+    if set(map(type, rows)) == {np.ndarray}:
+        try:
+            flat = np.concatenate(rows, dtype=np.int32, casting="unsafe")
+        except ValueError:                      # not all of one dimension
+            pass
+    if flat is not None and flat.ndim == 1:
+        num = size = np.fromiter(map(len, rows), np.int32, nlocal)
+    else:
+        # rows of other kinds one by one: integers out of range are an error
+        rows = [np.ascontiguousarray(r, dtype=np.int32) for r in rows]
+        num = np.fromiter(map(len, rows), np.int32, nlocal)
+        size = np.fromiter((r.size for r in rows), np.int64, nlocal)
+        flat = np.concatenate([r.reshape(-1) for r in rows]) if rows else np.zeros(0, np.int32)
+    first = np.concatenate([[0], np.cumsum(size[:-1], dtype=np.int64)])
+    return num, flat, (flat.ctypes.data + 4 * first).astype(np.uintp)
+
+
 class Engine:
     """One context of the GPU path for a potential ``model`` on ``device``."""
 
@@ -406,13 +430,7 @@ class Engine:
         nghost = len(x) - nlocal
         num = rows = ptrs = None
         if neigh is not None:
-            # one flat array and the address of every row in it
-            if len(neigh) != nlocal:
-                raise ValueError("pair_compute: one neighbour row per local atom")
-            num = np.fromiter(map(len, neigh), np.int32, nlocal)
-            rows = np.concatenate(neigh, dtype=np.int32, casting="unsafe") if nlocal else np.zeros(0, np.int32)
-            first = np.concatenate([[0], np.cumsum(num[:-1], dtype=np.int64)])
-            ptrs = (rows.ctypes.data + 4 * first).astype(np.uintp)
+            num, rows, ptrs = _flat_rows(neigh, nlocal)
         f = np.zeros((nlocal, 3))
         e = C.c_double(0.0)
         ea = np.zeros(nlocal) if per_atom else None
