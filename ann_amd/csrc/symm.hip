@@ -1027,6 +1027,7 @@ __device__ __forceinline__ void fused_net(const SymmArgs& A, const NetDesc& D, i
 // the waves of a workgroup are independent.
 template <int MODE, int Z>
 __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, float4* smem4) {
+    static_assert(MODE >= 1 && MODE <= 3, "adjoint, tangent, fused");
     constexpr int NM = nharm(Z);
     constexpr int ZP = Z + 1;
     constexpr int PWS = (NM * (MODE == 2 ? 2 : 1)) | 1;      // function values per neighbour, odd stride
@@ -1045,7 +1046,7 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
     sm.g = smem4;
     sm.ef = sm.g + maxn;
     sm.efd = sm.ef + maxn;
-    float4* tv = sm.efd + (MODE == 0 ? 0 : maxn);
+    float4* tv = sm.efd + maxn;
     sm.r = reinterpret_cast<float*>(tv + (MODE == 2 ? maxn : 0));
     int* const after_r = reinterpret_cast<int*>(sm.r + maxn);
     sm.canon = ADJ ? after_r : nullptr;                         // the adjoint's slot map
@@ -1071,7 +1072,7 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
     // adjoint's radial part runs after the moments, so they have their own rows)
     sm.fg = reinterpret_cast<float2*>(FUSED ? fgr : pw);
 
-    n = fast_load(A, Mo, i, a, o, n, sm, MODE != 0, ADJ, MODE == 2 ? tv : nullptr);
+    n = fast_load(A, Mo, i, a, o, n, sm, true, ADJ, MODE == 2 ? tv : nullptr);
     if (MODE == 1) {
         for (int m = lane; m < ldg; m += kWave) rowbuf[m] = A.dEdG[(size_t)i * ldg + m];
         for (int t = lane; t < 3 * n; t += kWave) sP[t] = 0.0f;
@@ -1084,7 +1085,7 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
     // function values of the unit vector (and, for the tangent, their derivatives
     // along the projected direction (t - r^ (r^.t)) / r) of neighbours c0 .. c1-1,
     // at most pw_chunk, into the chunk rows (the moment loop below walks each
-    // species segment in such chunks, so for G and the adjoint the rows take a
+    // species segment in such chunks, so for the adjoint the rows take a
     // fixed slice of LDS instead of one row per neighbour)
     auto function_rows = [&](int c0, int c1) {
         for (int J = c0 + lane; J < c1; J += kWave) {
@@ -1193,7 +1194,7 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
         }
     }
     wave_sync();
-    // block contractions (modes 0, 2, 3) or their adjoint seeds (mode 1; mode 3
+    // block contractions (modes 2, 3) or their adjoint seeds (mode 1; mode 3
     // after its network)
     auto adjoint_seeds = [&]() {
         // lanes over (pair, width, power) of every block at once; each lane loads
@@ -1272,7 +1273,7 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
         }
         wave_sync();
         if (!FUSED) {
-            float* out = (MODE == 0 ? A.G : A.v) + (size_t)i * ldg;
+            float* out = A.v + (size_t)i * ldg;
             for (int m = lane; m < ldg; m += kWave) out[m] = rowbuf[m];
             return;
         }
@@ -1920,16 +1921,13 @@ __global__ __launch_bounds__(256) void k_moment_queue(SymmArgs A) {
         int nk = 0;
         if (lane == 0) nk = atomicAdd(ctr, 1);
         const int2 it = A.items[beg + k];
-        if constexpr (MODE == kModeAdjT || MODE == 0 || MODE == kModeTanT) {
-            const int ib = __builtin_amdgcn_readfirstlane(it.x), ie = ib + __builtin_amdgcn_readfirstlane(it.y);
-            for (int a = ib; a < ie; a += A.atomsK) {
-                if constexpr (MODE == 0) g_atom<Z, SR, false>(A, a, smem4);
-                else if constexpr (MODE == kModeTanT) g_atom<Z, SR, true>(A, a, smem4);
-                else adjoint_wave<Z>(A, a, min(A.atomsK, ie - a), smem4);
-                wave_sync();                                    // the next atoms reuse the LDS slice
-            }
-        } else {
-            for (int a = it.x; a < it.x + it.y; ++a) moment_atom<MODE, Z>(A, a, smem4);
+        const int ib = __builtin_amdgcn_readfirstlane(it.x), ie = ib + __builtin_amdgcn_readfirstlane(it.y);
+        for (int a = ib; a < ie; a += A.atomsK) {
+            if constexpr (MODE == 0) g_atom<Z, SR, false>(A, a, smem4);
+            else if constexpr (MODE == kModeTanT) g_atom<Z, SR, true>(A, a, smem4);
+            else if constexpr (MODE == kModeAdjT) adjoint_wave<Z>(A, a, min(A.atomsK, ie - a), smem4);
+            else moment_atom<MODE, Z>(A, a, smem4);
+            wave_sync();                                        // the next atoms reuse the LDS slice
         }
         k = __shfl(nk, 0);
     }
@@ -1944,7 +1942,7 @@ static size_t moment_smem(const SymmArgs& A, int mode, int Z, int S, int NP) {
     const int NM = nharm(Z), ZP = Z + 1, U4 = kMaxUnionEta;
     const bool adj = mode == 1 || mode == 3;
     const int PWS = (NM * (mode == 2 ? 2 : 1)) | 1;
-    size_t b = 16 * (size_t)A.maxn * (2 + (mode == 0 ? 0 : 1) + (mode == 2 ? 1 : 0));
+    size_t b = 16 * (size_t)A.maxn * (3 + (mode == 2 ? 1 : 0));
     b += 4 * (adj ? 2 : 1) * (size_t)A.maxn + 4 * 16;                              // r, canon (adjoint), seg
     size_t f = (size_t)A.ldg + (mode == 1 ? 3 * (size_t)A.maxn : 0) + (mode == 3 ? 2 * (size_t)A.maxn : 0) +
                (size_t)pw_floats(mode, A.maxn, PWS);
@@ -2106,7 +2104,7 @@ static hipError_t run(ann_ctx* ctx, int form, SymmArgs A) {
         if (MODE == 0 && tfits) A.Tout = ctx->d_T;
         if (MODE != 0 && tfits && ctx->T_gen == ctx->geo_gen) A.Tin = ctx->d_T;
         const bool adjT = MODE == 1 && A.Tin, tanT = MODE == 2 && A.Tin;
-        size_t sw = (moment_smem(A, MODE, M.moment_z, M.S, M.NP) + 15) / 16 * 16;
+        size_t sw = 0;
         if (adjT) {
             A.atomsK = adj_atoms(ctx);
             if (adj_units(A.atomsK, M.moment_z, M.S, M.NP, A.nrs, A.ldg) > 1024) A.atomsK = 1;   // above 16 KiB
@@ -2121,6 +2119,8 @@ static hipError_t run(ann_ctx* ctx, int form, SymmArgs A) {
             A.grows = (MODE == 0 && M.moment_z <= 2) || fits ? kWave : (tanT && M.moment_z <= 2 ? 24 : kWave / 2);
             A.grows = std::min(A.grows, A.maxn);                // no more than the widest row has (a multiple of 4)
             sw = 16 * (size_t)units(A.grows);
+        } else {
+            sw = (moment_smem(A, MODE, M.moment_z, M.S, M.NP) + 15) / 16 * 16;
         }
         int apb = ctx->tune_apb[MODE];
         while (apb > 1 && sw * apb > 65536) apb /= 2;          // dynamic LDS of one workgroup
