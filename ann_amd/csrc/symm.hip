@@ -62,7 +62,7 @@ struct SymmArgs {
     const float* Tin;         // moment form, adjoint and tangent: moments of the same geometry (or null: recompute)
     int rad_gauss;            // every radial block is GAUSSIAN
     int nrad, nrs;            // widest radial block; its row stride in the adjoint's tables (odd)
-    int grows;                // function rows in LDS of the G kernel
+    int grows;                // function rows in LDS at a time (G, stored-moment tangent, recomputing adjoint)
     int atomsK;               // atoms per wavefront of G and of the stored-moment adjoint
     // fused E+F (mode 3): the network's parameter tables and inputs, the atom energies
     const float* wchunk;      // forward weight rows, biases, output neuron (net_dev.h layout)
@@ -893,19 +893,19 @@ __global__ __launch_bounds__(64) void k_fast(SymmArgs A) {
 // 216 us, 512 uneven water cells 4.18 -> 3.94 ms, five MD steps of 1 M atoms
 // 103.0 -> 97.2 ms, 64 water boxes and Li/P/S training unchanged.
 
-// moment_atom's chunk of function rows (adjoint: 64, fused: 32; tangent: every
-// neighbour at once while a row is short, up to degree 2, else 32), and the
+// moment_atom's chunk of function rows (adjoint: set by the host, 64 or 32; fused:
+// 32; tangent: every neighbour at once while a row is short, up to degree 2, else 32), and the
 // floats of the region that holds them (it also holds the cutoff pairs, two
 // floats per neighbour, before the rows are needed).  Mode 1 here is the adjoint
 // that recomputes the moments: it serves calls whose geometry no G call has seen.
 constexpr int kPwRows = 64;
 // adjoint: dE/dT entries per lane held in registers while they replace the moments
 constexpr int kUbRegs = 8;
-__host__ __device__ inline int pw_chunk(int mode, int maxn, int pws) {
-    return mode == 2 && pws <= 32 ? maxn : (mode == 1 ? kPwRows : kPwRows / 2);
+__host__ __device__ inline int pw_chunk(int mode, int maxn, int pws, int grows) {
+    return mode == 2 && pws <= 32 ? maxn : (mode == 1 ? grows : kPwRows / 2);
 }
-__host__ __device__ inline int pw_floats(int mode, int maxn, int pws) {
-    const int rows = pw_chunk(mode, maxn, pws);
+__host__ __device__ inline int pw_floats(int mode, int maxn, int pws, int grows) {
+    const int rows = pw_chunk(mode, maxn, pws, grows);
     if (mode == 3) {                                // fused: also the adjoint vectors and network vectors
         const int m = rows * pws > 3 * maxn ? rows * pws : 3 * maxn;
         return m > 3 * kVecMaxWidth ? m : 3 * kVecMaxWidth;
@@ -1059,7 +1059,7 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
     const int TS = S * U4 * NM;                                 // moments per atom
     float* fgr = rowbuf + ldg;                                  // fused: [maxn] cutoff pairs of their own
     float* pw = FUSED ? sP : sP + (MODE == 1 ? 3 * maxn : 0);  // [pw_chunk][PWS] (one chunk of neighbours)
-    float* T = pw + pw_floats(MODE, maxn, PWS);                // [S][U4][NM]
+    float* T = pw + pw_floats(MODE, maxn, PWS, A.grows);      // [S][U4][NM]
     float* dT = T + S * U4 * NM;                                // [S][U4][NM] (mode 2)
     float* D = dT + (MODE == 2 ? S * U4 * NM : 0);              // [S][U4]
     float* dD = D + S * U4;                                     // [S][U4] (mode 2: dD, mode 1: dE/dD)
@@ -1130,7 +1130,7 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
                     dacc[3] += f4.w * wm + e4.w * dy;
                 }
             };
-            const int chunk = pw_chunk(MODE, maxn, PWS);
+            const int chunk = pw_chunk(MODE, maxn, PWS, A.grows);
             for (int c0 = s0; c0 < s1; c0 += chunk) {
                 const int c1 = min(c0 + chunk, s1);
                 wave_sync();                                    // the previous chunk's rows are read
@@ -1945,7 +1945,7 @@ static size_t moment_smem(const SymmArgs& A, int mode, int Z, int S, int NP) {
     size_t b = 16 * (size_t)A.maxn * (3 + (mode == 2 ? 1 : 0));
     b += 4 * (adj ? 2 : 1) * (size_t)A.maxn + 4 * 16;                              // r, canon (adjoint), seg
     size_t f = (size_t)A.ldg + (mode == 1 ? 3 * (size_t)A.maxn : 0) + (mode == 3 ? 2 * (size_t)A.maxn : 0) +
-               (size_t)pw_floats(mode, A.maxn, PWS);
+               (size_t)pw_floats(mode, A.maxn, PWS, A.grows);
     f += (size_t)S * U4 * NM * (mode == 2 ? 2 : 1) + 2 * (size_t)S * U4 + (size_t)NP * U4 * ZP;
     f += (adj && S * NM * U4 > kUbRegs * kWave ? (size_t)S * NM * U4 : 0);         // dE/dT beside the moments
     return b + 4 * f;
@@ -2120,7 +2120,16 @@ static hipError_t run(ann_ctx* ctx, int form, SymmArgs A) {
             A.grows = std::min(A.grows, A.maxn);                // no more than the widest row has (a multiple of 4)
             sw = 16 * (size_t)units(A.grows);
         } else {
+            // the adjoint that sums the moments: 64 function rows at a time where the chip
+            // holds every wavefront's slice all the same or rows are short, else 32 (us, 64 /
+            // 32: 12,288 atoms of one species and degree 4 70 / 56, of two 80 / 65, of three 100
+            // / 78; 512 atoms 13.9 / 14.6; degree 5 98 / 98)
+            A.grows = kPwRows;
             sw = (moment_smem(A, MODE, M.moment_z, M.S, M.NP) + 15) / 16 * 16;
+            if (MODE == 1 && M.moment_z >= 4 && (int64_t)A.N > (int64_t)ctx->num_cu * (int64_t)((160 << 10) / sw)) {
+                A.grows = kPwRows / 2;
+                sw = (moment_smem(A, MODE, M.moment_z, M.S, M.NP) + 15) / 16 * 16;
+            }
         }
         int apb = ctx->tune_apb[MODE];
         while (apb > 1 && sw * apb > 65536) apb /= 2;          // dynamic LDS of one workgroup

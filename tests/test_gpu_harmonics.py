@@ -107,3 +107,18 @@ def test_moments_kept_by_calls_that_move_nothing(oracle_mod):
     eng.energy_forces(FAST)
     for a, b in ((eng.symm_bwd(dE), P0), (eng.tangent(u), v0)):
         assert float((a.double() - b.double()).norm()) <= 1e-5 * float(b.double().norm())
+
+
+@pytest.mark.parametrize("z", [3, 4, 5])
+def test_recomputing_adjoint_of_large_batches(z):
+    """More wavefronts than the chip's LDS holds at 64 function rows each (32 from degree 4 on)."""
+    import torch
+    from ann_amd import configs
+    from ann_amd.gpu import FAST, Engine
+    eng = Engine(_model(2, z), "cuda:0")
+    eng.set_batch(configs.batch_water(32, seed=47))
+    eng.neighbors()
+    dE = torch.from_numpy(np.random.default_rng(48).normal(size=(eng.N, eng.ldg)).astype(np.float32)).cuda()
+    P0 = eng.symm_bwd(dE).double()              # no moments of this list are stored yet
+    eng.energy_forces(FAST)
+    assert float((eng.symm_bwd(dE).double() - P0).norm()) <= 1e-5 * float(P0.norm())
