@@ -2,7 +2,7 @@
 //
 // Same mathematics as ANN::fpbp + DODZ::grad (src/ml/nn.cpp:1367-1389,
 // 1801-1830).  Atoms are grouped by species (a species-sorted permutation of
-// the batch) into tiles of 16 rows; four wavefronts share a tile and run every
+// the batch) into tiles of 16 rows; four or eight wavefronts share a tile and run every
 // layer as 16 x N x K products on the matrix cores (BF16 operands split into
 // three terms, FP32 accumulation; Operands below):
 //   forward:  Z_l = A_{l-1} W_l^T (+ b_l), activation on the accumulator;
@@ -11,6 +11,8 @@
 // Activations move between the accumulator layout and the operand layout
 // through LDS; the weights come as operand tables split once per parameter
 // update (k_wtables).
+#include <type_traits>
+
 #include "net_dev.h"
 
 namespace ann {
@@ -64,14 +66,13 @@ __device__ __forceinline__ bf16x8 as_bf16x8(uint4 u) {
 // and column tile ct, the three BF16 terms of lane l are the 16-byte entries
 // ((kk * nt + ct) * 3 + p) * 64 + l, p = 0, 1, 2.  The left operands are split
 // once, by the thread that writes them, into three BF16 planes of the tile.
-constexpr int kNetWaves = 4;                // wavefronts per tile; column tile ct belongs to wavefront ct % 4
 constexpr int kPlaneK = kMaxK + 8;          // row stride of a plane: 16-byte rows, all banks in a 16-row read
 typedef __bf16 PlaneRow[kPlaneK];
 
-// This wavefront's operands of a product with NH own column tiles and up to KB k
-// blocks.  Loaded a phase ahead, so that the loads' latency runs beside the phase
+// The operands of one of NW wavefronts (column tile ct belongs to wavefront ct % NW)
+// of a product with NH own column tiles and up to KB k blocks.  Loaded a phase ahead, so that the loads' latency runs beside the phase
 // before (they depend on nothing but the tile's species).
-template <int NH, int KB>
+template <int NH, int KB, int NW>
 struct Operands {
     uint4 w[NH][KB][3];
     __device__ __forceinline__ void load(const uint4* __restrict__ tab, int K, int ncol, int wv) {
@@ -80,7 +81,7 @@ struct Operands {
         for (int h = 0; h < NH; ++h)
 #pragma unroll
             for (int kk = 0; kk < KB; ++kk) {
-                const int ct = h * kNetWaves + wv;
+                const int ct = h * NW + wv;
                 if (ct < nt && kk < nkb) {
                     const uint4* e = tab + (size_t)((kk * nt + ct) * 3) * kWave + lane;
 #pragma unroll
@@ -102,7 +103,7 @@ struct Operands {
             const bf16x8 a2 = *reinterpret_cast<const bf16x8*>(&X2[row][32 * kk + kb]);
 #pragma unroll
             for (int h = 0; h < NH; ++h) {
-                if (h * kNetWaves + wv >= nt) break;
+                if (h * NW + wv >= nt) break;
                 const bf16x8 b0 = as_bf16x8(w[h][kk][0]), b1 = as_bf16x8(w[h][kk][1]), b2 = as_bf16x8(w[h][kk][2]);
                 f32x4 c = acc[h];
                 c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, b0, c, 0, 0, 0);
@@ -247,25 +248,29 @@ hipError_t split_weights(ann_ctx* ctx, int* tick) {
     return weight_tables(ctx, tick, true);
 }
 
-// Four wavefronts per 16-atom single-species tile, the column tiles of every
+// NW wavefronts per 16-atom single-species tile, the column tiles of every
 // product dealt round.  A batch of small structures has fewer tiles than the chip
 // has SIMDs and a tile is a chain of short products, so latency is what counts:
 // every product's weight operands are loaded a phase ahead, the inputs come
 // straight into the split planes, and the output neuron and the first gradient
 // share a phase.
 // NT: column tiles of 16 of the widest hidden layer (4 up to 64 neurons, 8 up
-// to 128), so narrow networks keep their registers and LDS.
+// to 128), so narrow networks keep their registers and LDS.  Four wavefronts for 4
+// column tiles, eight for 8: each then holds one tile's operands.  With two tiles'
+// on four wavefronts 316 registers left one wavefront per SIMD; 128-128-1, us, before
+// the loads ahead / four wavefronts / eight: 256 atoms 38 / 17 / 14.6, 6,144 atoms 41 /
+// 32 / 20, 102,400 atoms 286 / 362 / 186; 128-1: 150 / 232 / 113.
 // Against two wavefronts per tile that split the left operand at every product and
 // loaded each operand where it was used, us: 192 atoms 22.6 -> 12.1, 2,048 atoms 22
 // -> 12.4, 12,288 atoms 28.8 -> 17.3, 273,561 atoms 308 -> 248 (water 80-32-32-1),
 // 21,872 Li/P/S atoms (96-48-48-1) 35.4 -> 25.6.
-template <int NT>
-__global__ __launch_bounds__(kNetWaves * kWave) void k_net_mfma(MfmaArgs A) {
+template <int NT, int NW>
+__global__ __launch_bounds__(NW * kWave) void k_net_mfma(MfmaArgs A) {
     constexpr int W = 16 * NT;                  // widest hidden layer of this instance
-    constexpr int NH = NT / kNetWaves;          // own column tiles of a hidden layer
-    constexpr int NB = kMaxK / 16 / kNetWaves;  // own column tiles of the input side
+    constexpr int NH = NT / NW;          // own column tiles of a hidden layer
+    constexpr int NB = kMaxK / 16 / NW;  // own column tiles of the input side
     constexpr int KH = W / 32;                  // k blocks of a hidden layer
-    constexpr int kThreads = kNetWaves * kWave;
+    constexpr int kThreads = NW * kWave;
     __shared__ __align__(16) PlaneRow X0[kTile], X1[kTile], X2[kTile];   // left operand, split
     __shared__ float act[kTile][W + 1];         // activations of the last hidden layer
     __shared__ float sdz[kMaxLayers - 1][kTile][W + 1];
@@ -278,7 +283,7 @@ __global__ __launch_bounds__(kNetWaves * kWave) void k_net_mfma(MfmaArgs A) {
     const int L = D.nlayer, nin = D.nin;
     const float* iw = A.inpw + D.inoff;
     const float* ib = A.inpb + D.inoff;
-    Operands<NH, kMaxK / 32> wf;
+    Operands<NH, kMaxK / 32, NW> wf;
     if (L > 1) wf.load(A.wtab + D.wsf[0], nin, D.nodes[0], wv);
     // a value and its right neighbour, split, into the planes
     auto put2 = [&](int r, int k, float x, float y) {
@@ -296,40 +301,41 @@ __global__ __launch_bounds__(kNetWaves * kWave) void k_net_mfma(MfmaArgs A) {
         X1[r][k] = q;
         X2[r][k] = u;
     };
-    // scaled input s = inpw (G + inpb): a wavefront takes every fourth row, lanes two inputs each
+    // scaled input s = inpw (G + inpb): a wavefront takes every NW-th row, lanes two inputs each
     {
         const int k = 2 * lane;
         const bool in0 = k < nin, in1 = k + 1 < nin;
         const float w0 = in0 ? iw[k] : 0.0f, w1 = in1 ? iw[k + 1] : 0.0f;
         const float b0 = in0 ? ib[k] : 0.0f, b1 = in1 ? ib[k + 1] : 0.0f;
-        float g0[kTile / kNetWaves], g1[kTile / kNetWaves];
+        float g0[kTile / NW], g1[kTile / NW];
 #pragma unroll
-        for (int q = 0; q < kTile / kNetWaves; ++q) {
-            const int r = wv + q * kNetWaves;
+        for (int q = 0; q < kTile / NW; ++q) {
+            const int r = wv + q * NW;
             const float* G = A.G + (size_t)A.perm[tl.y + min(r, nrow - 1)] * A.ldg;
             g0[q] = in0 ? G[k] : 0.0f;
             g1[q] = in1 ? G[k + 1] : 0.0f;
         }
 #pragma unroll
-        for (int q = 0; q < kTile / kNetWaves; ++q) {
-            const int r = wv + q * kNetWaves;
+        for (int q = 0; q < kTile / NW; ++q) {
+            const int r = wv + q * NW;
             const float x = r < nrow ? w0 * (g0[q] + b0) : 0.0f, y = r < nrow ? w1 * (g1[q] + b1) : 0.0f;
             put2(r, k, x, y);                               // zero past the inputs, up to kMaxK
         }
     }
     const int col = lane % 16, rb = 4 * (lane / 16);
-    // thread (row, slot of 16) of the phases that run over a row's neurons
-    const int orow = tid / 16, osl = tid % 16;
+    // thread (row, slot) of the phases that run over a row's neurons
+    constexpr int SL = kThreads / kTile;
+    const int orow = tid / SL, osl = tid % SL;
     const float* WL = A.W + D.woff[L - 1];
     if (L == 1) {
         // no hidden layer: the output neuron reads the scaled inputs
         float z = 0.0f;
         if (orow < nrow) {
             const float* G = A.G + (size_t)A.perm[tl.y + orow] * A.ldg;
-            for (int m = osl; m < nin; m += 16) z += WL[m] * (iw[m] * (G[m] + ib[m]));
+            for (int m = osl; m < nin; m += SL) z += WL[m] * (iw[m] * (G[m] + ib[m]));
         }
 #pragma unroll
-        for (int o = 8; o > 0; o >>= 1) z += __shfl_xor(z, o);
+        for (int o = SL / 2; o > 0; o >>= 1) z += __shfl_xor(z, o);
         if (orow < nrow && osl == 0) A.Eatom[A.perm[tl.y + orow]] = D.outb + D.outw * (A.W[D.boff[0]] + z);
         if (!A.dEdG) return;
         for (int q = tid; q < kTile * A.ldg; q += kThreads) {
@@ -345,7 +351,7 @@ __global__ __launch_bounds__(kNetWaves * kWave) void k_net_mfma(MfmaArgs A) {
         float bias[NH];
 #pragma unroll
         for (int h = 0; h < NH; ++h) {
-            const int n = (h * kNetWaves + wv) * 16 + col;
+            const int n = (h * NW + wv) * 16 + col;
             bias[h] = n < no ? bl[n] : 0.0f;
         }
         __syncthreads();                                    // the planes are written
@@ -357,9 +363,9 @@ __global__ __launch_bounds__(kNetWaves * kWave) void k_net_mfma(MfmaArgs A) {
         __syncthreads();                                    // the planes are read
 #pragma unroll
         for (int h = 0; h < NH; ++h) {
-            const int n = (h * kNetWaves + wv) * 16 + col;
+            const int n = (h * NW + wv) * 16 + col;
             float av[4] = {0.f, 0.f, 0.f, 0.f}, dv[4] = {0.f, 0.f, 0.f, 0.f}, d2[4];
-            if ((h * kNetWaves + wv) * 16 < no) {
+            if ((h * NW + wv) * 16 < no) {
                 float z[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) z[i] = acc[h][i] + bias[h];
@@ -375,8 +381,15 @@ __global__ __launch_bounds__(kNetWaves * kWave) void k_net_mfma(MfmaArgs A) {
         }
         ni = no;
     }
-    Operands<NH, KH> wbh;                                   // backward through hidden layers
-    Operands<NB, KH> wb0;                                   // and through the input layer
+    using OpHidden = Operands<NH, KH, NW>;
+    using OpInput = Operands<NB, KH, NW>;
+    OpHidden wbh;                                           // backward through hidden layers
+    OpInput wbi;                                            // and through the input layer
+    // where the shapes agree they share registers: one is loaded when the other is used up
+    OpInput& wb0 = [&]() -> OpInput& {
+        if constexpr (std::is_same_v<OpHidden, OpInput>) return wbh;
+        else return wbi;
+    }();
     const bool grad = A.dEdG != nullptr;
     if (grad) {
         if (L > 2) wbh.load(A.wtab + D.wsb[L - 2], ni, D.nodes[L - 3], wv);
@@ -386,7 +399,7 @@ __global__ __launch_bounds__(kNetWaves * kWave) void k_net_mfma(MfmaArgs A) {
     // linear output neuron, and g_{L-1} = outw W_L . sigma'_{L-1} into the planes
     {
         if (grad)
-            for (int m = osl; m < W; m += 16) put1(orow, m, m < ni ? D.outw * WL[m] * sdz[L - 2][orow][m] : 0.0f);
+            for (int m = osl; m < W; m += SL) put1(orow, m, m < ni ? D.outw * WL[m] * sdz[L - 2][orow][m] : 0.0f);
         // one lane per atom, terms in order: atoms in like environments round alike, so
         // the order of this sum shows in a structure's energy
         if (tid < nrow) {
@@ -408,7 +421,7 @@ __global__ __launch_bounds__(kNetWaves * kWave) void k_net_mfma(MfmaArgs A) {
         __syncthreads();
 #pragma unroll
         for (int h = 0; h < NH; ++h) {
-            const int m = (h * kNetWaves + wv) * 16 + col;
+            const int m = (h * NW + wv) * 16 + col;
 #pragma unroll
             for (int i = 0; i < 4; ++i) put1(rb + i, m, m < nprev ? acc[h][i] * sdz[l - 1][rb + i][m] : 0.0f);
         }
@@ -417,7 +430,7 @@ __global__ __launch_bounds__(kNetWaves * kWave) void k_net_mfma(MfmaArgs A) {
         float iwm[NB];
 #pragma unroll
         for (int h = 0; h < NB; ++h) {
-            const int m = (h * kNetWaves + wv) * 16 + col;
+            const int m = (h * NW + wv) * 16 + col;
             iwm[h] = m < nin ? iw[m] : 0.0f;
         }
         __syncthreads();
@@ -432,7 +445,7 @@ __global__ __launch_bounds__(kNetWaves * kWave) void k_net_mfma(MfmaArgs A) {
             float* out = A.dEdG + (size_t)A.perm[tl.y + r] * A.ldg;
 #pragma unroll
             for (int h = 0; h < NB; ++h) {
-                const int m = (h * kNetWaves + wv) * 16 + col;
+                const int m = (h * NW + wv) * 16 + col;
                 if (m < A.ldg) out[m] = m < nin ? acc[h][i] * iwm[h] : 0.0f;
             }
         }
@@ -462,8 +475,8 @@ hipError_t net_fwd_mfma(ann_ctx* ctx, const float* G, float* Eatom, float* dEdG,
     for (int a = 0; a < ctx->hm.S; ++a)
         for (int l = 0; l < ctx->hm.net[a].nlayer - 1; ++l) wmax = std::max(wmax, ctx->hm.net[a].nodes[l]);
     Launch L(ctx, "net_mfma");
-    if (wmax <= 64) k_net_mfma<4><<<A.ntiles, kNetWaves * kWave, 0, ctx->stream>>>(A);
-    else k_net_mfma<8><<<A.ntiles, kNetWaves * kWave, 0, ctx->stream>>>(A);
+    if (wmax <= 64) k_net_mfma<4, 4><<<A.ntiles, 4 * kWave, 0, ctx->stream>>>(A);
+    else k_net_mfma<8, 8><<<A.ntiles, 8 * kWave, 0, ctx->stream>>>(A);
     return hipGetLastError();
 }
 

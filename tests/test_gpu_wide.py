@@ -116,3 +116,26 @@ def test_wide_train_step(oracle_mod, form):
     err = np.linalg.norm(g - gr) / np.linalg.norm(gr)
     print(f"  grad rel err {err:.2e}", flush=True)
     assert err <= 1e-5, err
+
+
+# widths around the column tiles of 16, 32 and 64, one to three hidden layers; the
+# widest layer's side of 64 picks four or eight wavefronts per tile
+@pytest.mark.parametrize("hidden", [[64], [65], [128], [1, 65], [65, 1, 128], [16, 127], [113, 96, 81], [128, 128, 128],
+                                    [64, 48, 33], []])
+def test_widths_of_the_matrix_core_network(oracle_mod, hidden):
+    """Energies and gradients on the same G, tiles of 16 atoms full and not."""
+    from ann_amd import configs
+    from ann_amd.model import init_network
+    m, batch = configs.model_lips(), configs.batch_lips(1, seed=66)
+    rng = np.random.default_rng(67)
+    m.nets = [init_network(96, hidden, n.neuron, rng) for n in m.nets]
+    eng = _engine(m, batch)
+    G = eng.symm(1)
+    E, dE = eng.net(G, 1)
+    E0, _ = eng.net(G, 1, grad=False)
+    orc = oracle_mod.Oracle(m)
+    Eo, dEo = orc.net(batch.species, G.cpu().numpy().astype(np.float64)[:, :orc.ld])
+    E, dE, E0 = E.cpu().numpy(), dE.cpu().numpy(), E0.cpu().numpy()
+    assert np.array_equal(E, E0)
+    assert np.max(np.abs(E - Eo)) <= 1e-6 * max(1.0, np.abs(Eo).max())
+    assert np.sqrt(((dE[:, :orc.ld] - dEo) ** 2).sum() / (dEo ** 2).sum()) <= 1e-5
