@@ -1,5 +1,7 @@
 """Arithmetic of the device headers that the host can run, compiled here with g++:
-packed image vectors, also of structures far from their cell."""
+packed image vectors, also of structures far from their cell, and the harmonics and
+Legendre coefficients of the moment kernels (the identity that
+test_moment_identity.py pins for monomials, in the functions that the kernels use)."""
 import os
 import subprocess
 
@@ -17,3 +19,7 @@ def _run(name, tmp_path):
 
 def test_packed_images(tmp_path):
     _run("test_images", tmp_path)
+
+
+def test_harmonics(tmp_path):
+    _run("test_harmonics", tmp_path)

@@ -102,3 +102,25 @@ def test_many_structures(oracle_mod, n, L):
         eng.set_batch(batch)
         eng.neighbors(6.0)
         _check(eng, batch, orc, 6.0)
+
+
+@pytest.mark.parametrize("n", [65, 2100])
+def test_nonfinite_between_good(oracle_mod, n):
+    """The same on a context whose list arrays are there, so that the fill beside the
+    wait also runs on the bad build; the next builds and the size report stand."""
+    import torch
+    from ann_amd.gpu import AnnError, Engine
+    model, batch = _model(), _gas(n, 9.0 if n < 100 else 28.0, 61)
+    eng, orc = Engine(model, "cuda:0"), oracle_mod.Oracle(model)
+    eng.set_batch(batch)
+    eng.neighbors(5.0)
+    _check(eng, batch, orc, 5.0)
+    for bad in (np.inf, np.nan, 1e300):
+        eng.d_pos[17, 2] = bad
+        with pytest.raises(AnnError):
+            eng.neighbors(5.0)
+        eng.d_pos.copy_(torch.from_numpy(batch.pos))
+        for _ in range(2):
+            eng.neighbors(5.0)
+            assert eng.nlist_size()[1] > 0
+        _check(eng, batch, orc, 5.0)
