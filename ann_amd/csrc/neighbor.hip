@@ -122,7 +122,9 @@ __global__ void k_fill_bins(int N, const int* __restrict__ bin_of, const int* __
 // 21.9 / 19.1; of four atoms 1,500 8.9 / 6.7, 20,000 62 / 17.
 constexpr int kSBinThreads = 512;
 constexpr int kSBinIt = 4;
-constexpr int kSBinAtoms = kSBinIt * kSBinThreads;   // largest structure (atoms, bins) of this path
+// largest structure (atoms, bins) of this path; at the limit, whole builds with three
+// launches / one: one structure of 2,000 atoms 39.3 / 38.3, 50 of them 276 / 268
+constexpr int kSBinAtoms = kSBinIt * kSBinThreads;
 constexpr int kSBinMany = 1536;
 
 template <int T>
@@ -304,10 +306,11 @@ __global__ __launch_bounds__(64) void k_search(
 // marked bin), bins that do not fit either are left to k_search.  Each block writes
 // the overflow mark (0 or 1) of each of its centre bins exactly once per build, so
 // the marks need no clearing between builds.
-// Bound by vector issue: about 25 instructions per 64 candidates and centre, and
-// the staging.  Against one sort per row, us: 1,048,576 atoms (rc 6.5, super-bins
-// now within the capacity) 5767 -> 1579, 273,561 atoms 621 -> 263, 87,912 Li/P/S
-// atoms 213 -> 148, 12,288 atoms 39.5 -> 26.3, 192 atoms 28.6 -> 11.7.
+// 470 vector instructions per atom on 64 water boxes (counters), issued 39 % of the
+// time: latency of the staging's phases, then issue.  Against one sort per row, us:
+// 1,048,576 atoms (rc 6.5, super-bins now within the capacity) 5767 -> 1540, 273,561
+// atoms 621 -> 256, 87,912 Li/P/S atoms 213 -> 146, 12,288 atoms 39.5 -> 25.2, 192
+// atoms 28.6 -> 11.4.
 constexpr int kStageCap = 1280;
 constexpr int kStageImages = 216;
 constexpr int kStageThreads = 512;

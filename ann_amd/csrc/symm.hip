@@ -887,8 +887,13 @@ __global__ __launch_bounds__(64) void k_fast(SymmArgs A) {
 // The kernels issue vector instructions most of the time, so the number of
 // functions is what counts: the harmonics are the (Z+1)^2 independent functions
 // among the (Z+1)(Z+2)(Z+3)/6 monomials of the unit vector's components (25
-// against 35 at zeta 4, 36 against 56 at zeta 5), and as an orthogonal basis
-// they have no alternating sum to amplify FP32 rounding.  Monomials against
+// against 35 at zeta 4, 36 against 56 at zeta 5).  Their recurrences round more
+// often than products of powers: in an FP32 emulation with exact widths one
+// angular input rounds 1.3 (zeta 2) to 2.0 times (zeta 5) as much as from
+// monomials.  With the exponentials of the widths the inputs' errors against
+// FP64, harmonics to monomials, are 1.09 (zeta 1) and 0.73 (zeta 4) on water, 0.98
+// and 0.91 (zeta 1, 2) on Li/P/S, 1.00, 1.01 and 0.91 (zeta 1, 2, 5) on argon.
+// Monomials against
 // harmonics, MI355X: E+F of 32 preconditioned water boxes (FP64 moments) 265 ->
 // 216 us, 512 uneven water cells 4.18 -> 3.94 ms, five MD steps of 1 M atoms
 // 103.0 -> 97.2 ms, 64 water boxes and Li/P/S training unchanged.
@@ -1362,11 +1367,11 @@ __device__ __forceinline__ void moment_atom(const SymmArgs& A, const int i, floa
 // entries take two passes, 170 take three); K comes from the batch
 // (adj_atoms).  LDS does not depend on the widest row, so the registers
 // alone set the number of resident wavefronts, also for lists with a skin.
-// Bound by vector issue: about 1,300 wave instructions per atom (water, two atoms
-// per wavefront) against 2,800 of the form with one LDS row per neighbour.
-// Measured against it: 1,048,576 atoms, list with a skin, 8.57 -> 3.15 ms;
-// 273,561 atoms 1285 -> 554 us; 12,288 atoms 54 -> 36 us; Li/P/S, 21,872 atoms,
-// 67 -> 36 us.
+// Bound by vector issue: 1,410 vector instructions per atom (water, two atoms per
+// wavefront, counters) of which the vector units are busy 74 % of the time, LDS
+// waits below 1 %.  Measured against the form with one LDS row per neighbour:
+// 1,048,576 atoms, list with a skin, 8.57 -> 3.03 ms; 273,561 atoms 1285 -> 555 us;
+// 12,288 atoms 54 -> 35 us; Li/P/S, 21,872 atoms, 67 -> 35 us.
 constexpr int kAdjAtoms = 2;
 
 // float4 entries of the wavefront's LDS slice (layout at the top of adjoint_wave)
@@ -1568,11 +1573,12 @@ __global__ __launch_bounds__(256) void k_adjoint(SymmArgs A) {
 // functions with lanes over (entry, function).  Every sum stays
 // in registers until the row ends, for three species or for all eight.  LDS holds
 // one pass, not one row per neighbour, so it does not grow with the widest row.
-// Bound by vector issue, about 1,650 wave instructions' worth of time per water
-// atom.  Against the form that regroups the whole row by species in LDS first
+// 1,356 vector instructions per water atom (counters), issued 59 % of the time with
+// 78 % of the lanes, LDS waits 6 %: bound by issue and by the chain of a pass's
+// phases.  Against the form that regroups the whole row by species in LDS first
 // (one row of 36 bytes per neighbour), us: 1,048,576 atoms with a skin 5119 ->
-// 4037, 273,561 atoms 820 -> 735, 12,288 atoms 47.4 -> 43.8, 87,912 Li/P/S atoms
-// 200 -> 152, 5.5 k 27.0 -> 18.1.  Two atoms per wavefront: 923 on the 273,561
+// 4037, 273,561 atoms 820 -> 737, 12,288 atoms 47.4 -> 43.5, 87,912 Li/P/S atoms
+// 200 -> 153, 5.5 k 27.0 -> 18.1.  Two atoms per wavefront: 923 on the 273,561
 // atoms, sums added up in LDS after every run: 829.  More species, 100,000 atoms, us,
 // whole row regrouped / sums in LDS / in registers: four (degree 4) 557 / 534 / 481,
 // five (degree 2) 402 / 440 / 387, eight (degree 2) 767 / 847 / 743; tangent with
@@ -1599,8 +1605,8 @@ __host__ inline int g_units(bool tan, int Z, int S, int NP, int nrad, int ldg, i
 // moments T that the G kernel stored: the runs then sum
 // dT_b[u][f] = sum (w de_u/dr Y_f + e_u dY_f), w = r^ . (u_i - u_j), and the
 // contraction is its product rule.  Against the form that regroups the row in LDS
-// and sums the moments again, Li/P/S: 21,872 atoms 89 -> 64 us (rows 24 / 32 / 48 /
-// 64 at a time: 64.5 / 67.3 / 70.2 / 85.5), 5.5 k 32 -> 25 us.
+// and sums the moments again, Li/P/S: 21,872 atoms 89 -> 62 us (rows 24 / 32 / 48 /
+// 64 at a time: 64.5 / 67.3 / 70.2 / 85.5), 5.5 k 32 -> 24 us.
 template <int Z, int SR, bool TAN>
 __device__ __forceinline__ void g_atom(const SymmArgs& A, const int i, float4* smem4) {
     constexpr int NM = GShape<Z>::NM, NX = GShape<Z>::NX, NW = GShape<Z>::NW, NG = GShape<Z>::NG;
@@ -2036,11 +2042,12 @@ static SymmArgs make_args(ann_ctx* ctx) {
 // Atoms per wavefront of the stored-moment adjoint.  A row of n entries takes
 // ceil(n / 64) passes, two rows together often one less; but two atoms' tables
 // are built one after the other, and half the wavefronts must still fill the
-// chip.  Measured (us, one / two / three atoms): 1,048,576 atoms 3559 / 3150 /
-// 3601, 273,561 atoms 673 / 576 / 649, 12,288 atoms 39.4 / 36.0 / 40.6, 5.5 k
-// 16.4 / 17.2 / 18.2, 2,048 atoms 17.0 / 25.1 / 30.6; argon, 4,096 atoms of 18
-// entries, 14.1 / 12.3 / 13.3 (both rows in one pass).  Three make more lanes
-// of an instruction read different LDS rows.
+// chip.  Measured (us, one / two atoms): 1,048,576 atoms 3349 / 3035, 273,561 atoms
+// 650 / 556, Li/P/S 21,872 atoms 40.5 / 35.3, 12,288 atoms 38.8 / 36.2, 5.5 k 14.8 /
+// 15.8, 2,048 atoms 16.4 / 23.9, 192 atoms 11.9 / 15.9; argon, 4,096 atoms of 18
+// entries, 13.3 / 11.7 (both rows in one pass).  Three (an earlier form, two / three
+// 576 / 649 on 273,561 atoms) make more lanes of an instruction read different LDS
+// rows.
 static int adj_atoms(const ann_ctx* ctx) {
     const int64_t N = ctx->natoms;
     const bool one_pass = 2 * ctx->nl.npairs <= (int64_t)kWave * 7 / 8 * N;

@@ -43,12 +43,12 @@ def work_model(model, batch, nl):
 
     triplet tiles and PLAIN form (the E+F convention P(30 + 12 nR) + T(60 + 12 nA)):
       symm_fwd = P(10 + 6 nR) + T(8 + 4 nA),  symm_bwd = P(20 + 6 nR) + T(52 + 8 nA)
-    moment form (M = (Z+1)(Z+2)(Z+3)/6 monomials, U widths of the centre species,
-    NP species pairs, nk (lambda, zeta) combinations, S species):
-      symm_fwd_mom = P(10 + 6 nR) + sum_i [n_i (M(2 + 2U) + 2U) + NP U 3M + sum_f 2(zeta_f + 1)]
-      symm_bwd_mom = P(20 + 6 nR) + sum_i [n_i (M(4U + 16) + 20) + NP U (Z+1) 2 nk + S M U 2S]
-                     (the moments themselves come from the G kernel)
-      symm_tan_mom = P(20 + 8 nR) + sum_i [n_i M (9 + 6U) + NP U 6M + sum_f 2(zeta_f + 1)]
+    moment form (M = (Z+1)^2 harmonics, U widths of the centre species, NP species
+    pairs, nk (lambda, zeta) combinations, S species):
+      symm_fwd_mom = P(10 + 6 nR) + sum_i [n_i (M(3 + 2U) + 2U) + NP U 2M + sum_f 2(zeta_f + 1)]
+      symm_bwd_mom = P(20 + 6 nR) + sum_i [n_i (M(4U + 8) + 20) + NP U (Z+1) 2 nk + S M U 2S]
+      symm_tan_mom = P(20 + 8 nR) + sum_i [n_i M (8 + 4U) + NP U 4M + sum_f 2(zeta_f + 1)]
+                     (adjoint and tangent read the moments that the G kernel stored)
       symm_tan (triplet tiles / PLAIN) = symm_fwd + symm_bwd
     networks: 4 MAC per atom and parameter-matrix entry (forward + input backward);
     second backward (net_bwd2) 8 MAC, parameter-gradient GEMMs (grad_reduce) 4 MAC;
@@ -80,17 +80,18 @@ def work_model(model, batch, nl):
                 T += t
         blocks = [model.angular[a][p] for p in range(NP)]
         Z = int(max(max(bl[2]) for bl in blocks if len(bl[2])))
-        M = (Z + 1) * (Z + 2) * (Z + 3) // 6
+        M = (Z + 1) ** 2
         U = len(set(np.concatenate([bl[1] for bl in blocks]).tolist()))
         nk = max(len(set(zip(bl[2].tolist(), bl[3].tolist()))) for bl in blocks)
         zsum = sum(float((bl[2] + 1).sum()) for bl in blocks)
-        fwd_m += n_i * 10 + 6 * pair + n_i * (M * (2 + 2 * U) + 2 * U) + NP * U * 3 * M + 2 * zsum
-        # the adjoint reads the moments the G kernel stored (no moment sums of its own)
-        bwd_m += n_i * 20 + 6 * pair + n_i * (M * (4 * U + 16) + 20) \
+        fwd_m += n_i * 10 + 6 * pair + n_i * (M * (3 + 2 * U) + 2 * U) + NP * U * 2 * M + 2 * zsum
+        # per function its value, U products each for the gradient's weight and the
+        # radial sums, and the sums over degrees
+        bwd_m += n_i * 20 + 6 * pair + n_i * (M * (4 * U + 8) + 20) \
             + NP * U * (Z + 1) * 2 * nk + S * M * U * 2 * S
-        # tangent (forward-mode G): per (neighbour, monomial) the monomial, its
-        # directional derivative and U value / derivative accumulations
-        tan_m += n_i * 20 + 8 * pair + n_i * M * (9 + 6 * U) + NP * U * 6 * M + 2 * zsum
+        # tangent (forward-mode G): per function its value, its directional derivative
+        # and the U sums of the moments' derivatives
+        tan_m += n_i * 20 + 8 * pair + n_i * M * (8 + 4 * U) + NP * U * 4 * M + 2 * zsum
     mac = 0
     for i in range(batch.ntotal):
         n = model.nets[batch.species[i]]

@@ -1,4 +1,4 @@
-"""The moment form at zeta 5 (56 monomials; the reference's Ar example basis,
+"""The moment form at zeta 5 (36 harmonics; the reference's Ar example basis,
 examples/Ar/basis_Ar, uses GAUSS zeta 5 with lambda -1) against the FP64
 oracle: E+F, G, the tangent and the training gradient, on one species (Ar, the
 example's cutoff) and two (water with zeta in {1, 5}); the moment kernels must
@@ -7,9 +7,8 @@ and the FP64-input path at zeta 5.
 
 Bars: energies <= 1e-6 eV/atom, forces and virial relative RMS <= 1e-5, G
 <= 2e-5 of the row maximum, tangent relative RMS <= 1e-5, gradient relative
-(L2) <= 1e-5.  The alternating binomial sum of the factorisation amplifies
-FP32 rounding by at most C(5,2) = 10 relative to the block's largest term; the
-printed errors show the margin.  Inputs scaled so that a small-valued one is
+(L2) <= 1e-5.  The sum over degrees of the factorisation carries FP32 rounding
+relative to the block's largest term; the printed errors show the margin.  Inputs scaled so that a small-valued one is
 amplified need the FP64 inputs (tested below).
 """
 import numpy as np
@@ -124,12 +123,12 @@ def test_zeta5_training_gradient_in_the_moment_form(oracle_mod):
 def test_zeta5_training_gradient_with_scaled_fp64_inputs(oracle_mod, name, form):
     """Inputs scaled by 1 / max |G| (the reference's MAX prescaling, no bias)
     and evaluated in FP64 (k_precise at zeta 5).  The FP32 moment form gives a
-    small-valued input (lambda -1, large zeta: an alternating binomial sum) an
-    absolute error set by its larger terms, in G and in the tangent, about 1e-4
-    of the input's own maximum at zeta 5 (6e-5 at zeta 4; 1.5e-6 in the triplet
+    small-valued input (lambda -1, large zeta: an alternating sum over degrees) an
+    absolute error set by its larger terms, in G and in the tangent, about 9e-5
+    of the input's own maximum at zeta 5 (4e-5 at zeta 4; 1.5e-6 in the triplet
     form), which this scaling amplifies: the Ar case keeps the moment-form
-    tangent (FAST), the water case, whose amplified inputs measured 5.3e-5 in
-    the moment form, takes the triplet form."""
+    tangent (FAST), the water case, whose gradient measured 1.4e-5 in the moment
+    form, takes the triplet form."""
     from ann_amd.gpu import FAST
     model, batch = _cases()[name]
     eng = _engine(model, batch)
