@@ -335,7 +335,7 @@ __global__ __launch_bounds__(kStageThreads) void k_search_bins(
     const CellInfo* __restrict__ ci, const double* __restrict__ cells, const int* __restrict__ bin_struc,
     const int* __restrict__ bin_start, const double4* __restrict__ rec, const double* __restrict__ pos, double rc2,
     uint64_t* __restrict__ keys_out, int* __restrict__ cnt_out, int* __restrict__ flag, int* __restrict__ bin_ovf,
-    const int* __restrict__ bin_atoms, const int* __restrict__ sof) {
+    const int* __restrict__ bin_atoms, const int* __restrict__ sof, const int* __restrict__ bin_of, int first) {
     __shared__ int im_first[kStageImages];
     __shared__ int im_m[kStageImages];
     __shared__ int im_pre[kStageImages + 1];
@@ -347,8 +347,13 @@ __global__ __launch_bounds__(kStageThreads) void k_search_bins(
     __shared__ int cen_bin[8], cen_pre[9], wsum[kStageWaves];
     __shared__ int s_total, s_max, s_xmax, s_jmin, s_jmax;
     uint64_t* sk = reinterpret_cast<uint64_t*>(cf);         // (j << 32 | image number) by bucket, until the ranks are known
-    const int g = xcd_block(blockIdx.x, gridDim.x), t = threadIdx.x;
-    const int lane = t % kWave, wave = t / kWave;
+    int g = first + xcd_block(blockIdx.x, gridDim.x);
+    const int t = threadIdx.x, lane = t % kWave, wave = t / kWave;
+    if (SPLIT && bin_of) {                                  // one block per atom in bin order: the first of each bin
+        const int slot = g;
+        g = bin_of[bin_atoms[slot]];
+        if (bin_start[g] != slot) return;
+    }
     if (SPLIT && (!bin_ovf[g] || bin_start[g] == bin_start[g + 1])) return;
     const int s = SPLIT ? sof[bin_atoms[bin_start[g]]] : bin_struc[g];   // structure of this bin or super-bin
     const CellInfo c = ci[s];
@@ -1123,7 +1128,7 @@ hipError_t neighbors_build(ann_ctx* ctx, double rc) {
         Launch L(ctx, "nb_search");
         k_search_bins<false><<<ctx->grid_nsb, kStageThreads, 0, st>>>(dci, ctx->d_cells, ctx->d_bin_struc, ctx->d_bin_start,
                                                       ctx->d_binrec, ctx->d_pos, rc * rc, ctx->d_keys, ctx->d_cnt,
-                                                      ctx->d_flag, ctx->d_bin_ovf, ctx->d_bin_atoms, ctx->d_struc_of);
+                                                      ctx->d_flag, ctx->d_bin_ovf, nullptr, nullptr, nullptr, 0);
     }
     // Super-bins are chosen on a structure's mean density; where its dense part (a
     // slab, a droplet) does not fit them, their bins are searched one by one.  A
@@ -1134,9 +1139,14 @@ hipError_t neighbors_build(ann_ctx* ctx, double rc) {
     // uniform atoms 1.57 -> 2.66 ms).
     auto search_split = [&]() {
         Launch L(ctx, "nb_search_split");
-        k_search_bins<true><<<nbins, kStageThreads, 0, st>>>(dci, ctx->d_cells, ctx->d_bin_struc, ctx->d_bin_start,
-                                                             ctx->d_binrec, ctx->d_pos, rc * rc, ctx->d_keys, ctx->d_cnt,
-                                                             ctx->d_flag, ctx->d_bin_ovf, ctx->d_bin_atoms, ctx->d_struc_of);
+        // a block per bin, or per atom where most bins are empty; a launch holds 2^32 threads
+        const bool atoms = N < nbins;
+        const int blocks = atoms ? N : nbins, most_blocks = 1 << 22;
+        for (int b = 0; b < blocks; b += most_blocks)
+            k_search_bins<true><<<std::min(blocks - b, most_blocks), kStageThreads, 0, st>>>(
+                dci, ctx->d_cells, ctx->d_bin_struc, ctx->d_bin_start, ctx->d_binrec, ctx->d_pos, rc * rc, ctx->d_keys,
+                ctx->d_cnt, ctx->d_flag, ctx->d_bin_ovf, ctx->d_bin_atoms, ctx->d_struc_of,
+                atoms ? ctx->d_bin_of : nullptr, b);
     };
     const bool ahead = ctx->nb_split;
     if (ahead) search_split();

@@ -63,6 +63,32 @@ def test_partly_overflowed_bins(oracle_mod, L, height, fill, spacing, rc, wide):
     print(f"  {batch.ntotal} atoms, rc {rc}: widest row {widest}", flush=True)
 
 
+@pytest.mark.parametrize("L,spacing,wide", [(80.0, 1.1, 1), (40.0, 1.1, 1), (40.0, 0.85, 4)])
+def test_droplet(oracle_mod, L, spacing, wide):
+    """A droplet in an otherwise empty cell, with more bins than atoms; its inner bins fit a
+    block one by one (rows of 200) or not (rows of 437)."""
+    import torch
+    from ann_amd import configs
+    from ann_amd.gpu import Engine
+    rng = np.random.default_rng(74)
+    g = np.arange(int(14.5 / spacing)) * spacing
+    # around the cell's first two bins per direction (2.05 or 2.1 wide), across its corner
+    pos = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3) - 0.5 * g[-1] + 2.05
+    pos = rng.permutation(pos + rng.normal(0.0, 0.05 * spacing, size=pos.shape))
+    batch = configs.single(pos, np.eye(3) * L, np.zeros(len(pos), np.int32))
+    assert len(pos) < (L // 2.0 - 1) ** 3
+    orc, eng = oracle_mod.Oracle(_model()), Engine(_model(), "cuda:0")
+    eng.set_batch(batch)
+    eng.profile(True)
+    for step in range(4):
+        eng.neighbors(4.0)
+        assert eng.nlist_size()[1] > 0
+        _check(eng, pos, batch, orc, 4.0)
+        pos = pos + rng.normal(0.0, 0.01, size=pos.shape)
+        eng.d_pos.copy_(torch.from_numpy(pos))
+    assert eng.profile_get("nb_search_wide")[1] == wide and eng.profile_get("nb_search_split")[1] == 4
+
+
 @pytest.mark.parametrize("n", [1900, 2600])
 def test_refused_then_good(oracle_mod, n):
     """A build refused for rows above the capacity leaves no fault behind for the next one."""
